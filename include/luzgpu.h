@@ -62,8 +62,9 @@ typedef struct luzgpu_settings
 	/* wavefront launch shape (0 = built-in default); no effect on the image */
 	uint32_t	traversal_grid;  /* persistent blocks per traversal launch, 1..2048 (default 1280)    */
 	int32_t		extend_refill;   /* idle lanes (1..64) at which a wave takes new closest-hit rays;    *
-	                              * 64 (default): whole-wave claims, each lane traverses to the end   */
-	int32_t		shadow_refill;   /* the same for shadow rays (default 64)                             */
+	                              * 64: whole-wave claims, each lane traverses to the end. Default    *
+	                              * 48 in triangle-only scenes, 16 with analytic primitives           */
+	int32_t		shadow_refill;   /* the same for shadow rays                                          */
 	uint32_t	fetch_chunk;     /* most rays a wave claims per queue atomic, 64..1024 (default 256;
 	                              * a claim is an eighth of a wave's even share of the queue,
 	                              * rounded up to 64, at most this)                             */

@@ -5,7 +5,8 @@
 //                   One cache-line fetch tests both children of a binary node; leaves
 //                   are folded into their parent's reference (count > 0).
 //   GpuTri    48 B  v0 | e1 | e2 in fp32 (e1, e2 formed in FP64, then rounded), with
-//                   the triangle's index in its mesh (after degenerate removal) in v0.w.
+//                   the triangle's index in its mesh (after degenerate removal) in v0.w; a
+//                   top-level triangle holds its hittable there.
 //   Hittable  8 B   kind:4 | index:28, material id — the reference's top-level list.
 #pragma once
 
@@ -25,20 +26,34 @@ namespace luzgpu
 	static_assert(sizeof(BvhNode) == 64, "BvhNode must be 64 bytes");
 
 	// 4-wide node in one 64-byte line. Child boxes are quantised to 8 bits per plane
-	// against the node's own box: plane = fma(q, 2^exp, origin), with q chosen on the host so
-	// that the decoded fp32 box contains the child's box (conservative by construction).
+	// against the node's own box: plane = fma(q, scale, origin), scale a power of two, with q
+	// chosen on the host so that the decoded fp32 box contains the child's box (conservative
+	// by construction). Child references are the traversal's stack entries, ready to push:
+	// an internal child is its node index; leaves have bit 31 set (see below). Used slots come
+	// first; the rest hold kEmptyChild.
 	struct alignas(64) Bvh4Node
 	{
 		float	origin[3];
-		std::int8_t	exp[3];
-		std::uint8_t	pad0;
+		float	scale[3];
 		std::uint8_t	qlo[3][4];	// [axis][child]
 		std::uint8_t	qhi[3][4];
-		std::int32_t	child[4];	// count == 0: node index; count 1..16: first primitive
-		std::uint8_t	count[4];	// 0 internal, 1..16 leaf, 255 empty
-		std::uint32_t	pad1;
+		std::uint32_t	child[4];
 	};
 	static_assert(sizeof(Bvh4Node) == 64, "Bvh4Node must be 64 bytes");
+
+	// Leaf references. Inside a mesh BVH: count - 1 in bits 27..30, first mesh triangle slot in
+	// bits 0..26. In the top level: a kind in bits 29..30, count - 1 in bits 27..28 and, in bits
+	// 0..26, the first top-level triangle slot (kTopTriangles), the instance (kTopInstance,
+	// count 1) or the first item of the leaf-item list (kTopItems: every other primitive).
+	constexpr std::uint32_t	kLeafBit = 0x80000000u;
+	constexpr std::uint32_t	kLeafStartMask = 0x07ffffffu;
+	constexpr std::uint32_t	kLeafCountShift = 27;
+	constexpr std::uint32_t	kTopKindShift = 29;
+	constexpr std::uint32_t	kTopItems = 0, kTopTriangles = 1, kTopInstance = 2;
+	constexpr std::uint32_t	kTopLeafMax = 4;
+	constexpr std::uint32_t	kEmptyChild = 0xffffffffu;
+	// Kernels address nodes with 32-bit byte offsets.
+	constexpr std::uint64_t	kMaxNodes = 1ull << 26;
 
 	struct alignas(16) GpuTri
 	{
@@ -131,10 +146,10 @@ namespace luzgpu
 	struct alignas(16) GpuInstance
 	{
 		float	worldToLocal[12];	// rows of a 3x4 affine map (inverse rotate, inverse scale)
-		std::int32_t	blasRoot;	// global Bvh4Node index of the mesh's root
+		std::int32_t	blasRoot;	// node index of the mesh's root
 		std::int32_t	triBase;	// first GpuTri of the mesh
 		std::int32_t	normalBase;	// first vertex-normal triple, -1 if the mesh has none
-		std::int32_t	pad0;
+		std::uint32_t	hittable;	// the instance's top-level hittable
 		float	normalToWorld[9];	// rotate(n / scale), renormalised after use
 		float	pad[3];
 	};

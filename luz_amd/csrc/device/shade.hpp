@@ -1115,7 +1115,8 @@ namespace luzgpu
 		}
 		const GpuTri& tri = s.topTris[L.index];
 		float u, v;
-		if (!triHit(tri, r, kTMinF, INFINITY, t, u, v) || L.area <= 0.0f) return 0.0f;
+		std::int32_t id;
+		if (!triHit(tri, r, kTMinF, INFINITY, t, u, v, id) || L.area <= 0.0f) return 0.0f;
 		const float c = fabsf(dot(vec, faceNormalOf(tri)) / sqrtf(vl2));
 		if (c <= 0.0f) return 0.0f;
 		return (t * t * vl2) / (c * L.area);

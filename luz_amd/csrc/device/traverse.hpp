@@ -24,8 +24,7 @@ namespace luzgpu
 
 	struct	SceneView
 	{
-		const Bvh4Node*	tlas;
-		const Bvh4Node*	blas;
+		const Bvh4Node*	nodes;	// top level, then the mesh BVHs
 		const GpuTri*	topTris;
 		const GpuTri*	meshTris;
 		const float*	meshNormals;
@@ -52,89 +51,29 @@ namespace luzgpu
 
 	struct	Ray
 	{
-		f3	o, d, inv;
+		f3	o, d;
 	};
 
-	__device__ __forceinline__ float	safeInv(float c)
-	{
-		// Ray::_inverseComponent: 0 for zero or non-finite components
-		if (c == 0.0f || !isfinite(c))
-		{
-			return 0.0f;
-		}
-		// hardware reciprocal (1 ulp): the inverse only feeds box tests, whose intervals are
-		// widened by far more than that
-		const float r = __builtin_amdgcn_rcpf(c);
-		return isfinite(r) ? r : 0.0f;
-	}
-
-	__device__ __forceinline__ Ray	makeRay(f3 o, f3 d)
-	{
-		return Ray{o, d, mk(safeInv(d.x), safeInv(d.y), safeInv(d.z))};
-	}
-
-	// Slab entry distance for one axis; zero inverse components test the origin against
-	// the slab instead (lo/hi of +/-inf keep or reject the interval).
-	__device__ __forceinline__ void	slab(float o, float inv, float bmin, float bmax, float& tn, float& tf)
-	{
-		if (inv == 0.0f)
-		{
-			const bool inside = !(o < bmin || o > bmax);
-			tn = inside ? -INFINITY : INFINITY;
-			tf = inside ? INFINITY : -INFINITY;
-			return;
-		}
-		float t0 = (bmin - o) * inv;
-		float t1 = (bmax - o) * inv;
-		tn = fminf(t0, t1);
-		tf = fmaxf(t0, t1);
-	}
-
-	__device__ __forceinline__ bool	boxHit(const Ray& r, const float* lo, const float* hi, float tMax, float& tNear)
-	{
-		float n0, f0, n1, f1, n2, f2;
-		slab(r.o.x, r.inv.x, lo[0], hi[0], n0, f0);
-		slab(r.o.y, r.inv.y, lo[1], hi[1], n1, f1);
-		slab(r.o.z, r.inv.z, lo[2], hi[2], n2, f2);
-		// widened by 2^-20 relative like the quantised-plane test (the inverse is 1 ulp)
-		const float tn = fmaxf(fmaxf(n0, n1) * (1.0f - 0x1p-20f), fmaxf(n2 * (1.0f - 0x1p-20f), kTMinF));
-		const float tf = fminf(fminf(f0, f1) * (1.0f + 0x1p-20f), fminf(f2 * (1.0f + 0x1p-20f), tMax));
-		tNear = tn;
-		return tf > tn;
-	}
+	__device__ __forceinline__ Ray	makeRay(f3 o, f3 d) { return Ray{o, d}; }
 
 	// The 48-byte triangle is fetched as three 16-byte loads issued together (one memory
-	// round trip), not field by field.
-	__device__ __forceinline__ bool	triHit(const GpuTri& tri, const Ray& r, float tMin, float tMax, float& t, float& u, float& v)
+	// round trip), not field by field, and tested without branches. `id`: GpuTri::prim.
+	__device__ __forceinline__ bool	triHit(const GpuTri& tri, const Ray& r, float tMin, float tMax, float& t, float& u, float& v,
+		std::int32_t& id)
 	{
 		const float4* tp = reinterpret_cast<const float4*>(&tri);
 		const float4 A = tp[0], B = tp[1], C = tp[2];
-		f3 v0 = mk(A.x, A.y, A.z);
-		const f3 e1 = mk(B.x, B.y, B.z), e2 = mk(C.x, C.y, C.z);
-		// v0 is needed only after the first exit: pin it here so its load is issued with
-		// the edges' instead of after the determinant test
-		asm volatile("" : "+v"(v0.x), "+v"(v0.y), "+v"(v0.z));
+		id = __float_as_int(A.w);
+		const f3 v0 = mk(A.x, A.y, A.z), e1 = mk(B.x, B.y, B.z), e2 = mk(C.x, C.y, C.z);
 		const f3 p = cross(r.d, e2);
 		const float det = dot(e1, p);
 		const f3 tv = r.o - v0;
-		if (fabsf(det) < 1e-12f)
-		{
-			return false;
-		}
 		const float inv = __builtin_amdgcn_rcpf(det);	// 1 ulp, against the FP64 reference's 1 / det
 		u = dot(tv, p) * inv;
-		if (u < 0.0f || u > 1.0f)
-		{
-			return false;
-		}
 		const f3 q = cross(tv, e1);
 		v = dot(r.d, q) * inv;
-		if (v < 0.0f || u + v > 1.0f)
-		{
-			return false;
-		}
 		t = dot(e2, q) * inv;
-		return !(t > tMax || t < tMin);
+		return !((fabsf(det) < 1e-12f) | (u < 0.0f) | (u > 1.0f) | (v < 0.0f) | (u + v > 1.0f) | (t > tMax) | (t < tMin));
 	}
 
 	__device__ __forceinline__ bool	rectHit(const GpuRect& rc, const Ray& r, float tMin, float tMax, float& t)
@@ -269,16 +208,6 @@ namespace luzgpu
 		return toLocal(mp[0], mp[1], mp[2], w);
 	}
 
-	// Stack entries: bit31 set = leaf (bits 27..30 = count-1, bits 0..26 = first prim);
-	// otherwise a node index; kExitInstance returns to the world-space ray.
-	constexpr std::uint32_t	kLeafBit = 0x80000000u;
-	constexpr std::uint32_t	kExitInstance = 0x7fffffffu;
-
-	__device__ __forceinline__ std::uint32_t	leafEntry(std::int32_t start, std::int32_t count)
-	{
-		return kLeafBit | (static_cast<std::uint32_t>(count - 1) << 27) | static_cast<std::uint32_t>(start);
-	}
-
 	struct	HitInfo
 	{
 		float	t;
@@ -310,8 +239,17 @@ namespace luzgpu
 		// The host refuses scenes whose BVH depth could exceed Depth; the clamp only keeps
 		// every LDS access inside this thread's column whatever happens.
 		__device__ __forceinline__ void	push(std::uint32_t v) { base[min(sp, Depth - 1) * Block] = v; sp++; }
+		// pushes a if wanted, then b, then c: a slot written in vain is the next push's
+		__device__ __forceinline__ void	push3(std::uint32_t a, bool wa, std::uint32_t b, bool wb, std::uint32_t c, bool wc)
+		{
+			base[min(sp, Depth - 1) * Block] = a;
+			sp += wa ? 1 : 0;
+			base[min(sp, Depth - 1) * Block] = b;
+			sp += wb ? 1 : 0;
+			base[min(sp, Depth - 1) * Block] = c;
+			sp += wc ? 1 : 0;
+		}
 		__device__ __forceinline__ std::uint32_t	pop() { sp--; return base[min(sp, Depth - 1) * Block]; }
-		__device__ __forceinline__ bool	empty() const { return sp == 0; }
 		__device__ __forceinline__ void	reset() { sp = 0; }
 	};
 
@@ -325,8 +263,13 @@ namespace luzgpu
 		int	sp;
 
 		__device__ __forceinline__ void	push(std::uint32_t x) { v[min(sp, kLocalStackDepth - 1)] = x; sp++; }
+		__device__ __forceinline__ void	push3(std::uint32_t a, bool wa, std::uint32_t b, bool wb, std::uint32_t c, bool wc)
+		{
+			if (wa) push(a);
+			if (wb) push(b);
+			if (wc) push(c);
+		}
 		__device__ __forceinline__ std::uint32_t	pop() { sp--; return v[min(sp, kLocalStackDepth - 1)]; }
-		__device__ __forceinline__ bool	empty() const { return sp == 0; }
 		__device__ __forceinline__ void	reset() { sp = 0; }
 	};
 
@@ -355,54 +298,107 @@ namespace luzgpu
 			else spill[static_cast<size_t>(min(sp, capacity - 1) - LdsDepth) * stride] = v;
 			sp++;
 		}
+		// As three pushes. While no lane of the wave is near the end of its LDS column (nearly
+		// always) the three slots are written without branches: one that was not wanted is the
+		// next push's slot.
+		__device__ __forceinline__ void	push3(std::uint32_t a, bool wa, std::uint32_t b, bool wb, std::uint32_t c, bool wc)
+		{
+			if (__ballot(sp > LdsDepth - 3) == 0ull)
+			{
+				base[sp * Block] = a;
+				sp += wa ? 1 : 0;
+				base[sp * Block] = b;
+				sp += wb ? 1 : 0;
+				base[sp * Block] = c;
+				sp += wc ? 1 : 0;
+				return;
+			}
+			if (wa) push(a);
+			if (wb) push(b);
+			if (wc) push(c);
+		}
 		__device__ __forceinline__ std::uint32_t	pop()
 		{
 			sp--;
-			if (sp < LdsDepth) return base[sp * Block];
+			if (__ballot(sp >= LdsDepth) == 0ull || sp < LdsDepth) return base[sp * Block];
 			return spill[static_cast<size_t>(min(sp, capacity - 1) - LdsDepth) * stride];
 		}
-		__device__ __forceinline__ bool	empty() const { return sp == 0; }
 		__device__ __forceinline__ void	reset() { sp = 0; }
 	};
 
-	// Resumable per-lane traversal state: one call of traceStep processes one stack entry
-	// (a node, a leaf or an instance exit), so a persistent kernel can hand a lane a new ray
-	// as soon as its traversal ends instead of waiting for the whole wave.
+	// Resumable per-lane traversal state. A persistent kernel advances it one entry at a time
+	// (nodeStep for an internal node, leafStep for a leaf, then popEntry when neither named the
+	// next entry), so it can hand a lane a new ray as soon as its traversal ends.
+	//
+	// Node tests run on the ray in slab form, set once per level: on each axis a plane at
+	// origin + q * scale is met at t = fma(q, scale * inv, fma(origin, inv, -o * inv)). The
+	// reciprocal is the hardware's (1 ulp); an axis the ray is parallel to takes a huge one, so
+	// its planes lie far behind or ahead, as AABB::hit's test of the origin against the slab
+	// has it (AABB.cpp:37-80). `nearC` / `farC` are -o * inv moved outward by 2^-21 of
+	// itself, which covers the rounding of that product and of the sums, and the far distance
+	// is compared with a relative margin of 2^-19: box tests are conservative (they only decide
+	// which primitives are tested), the primitive tests alone decide the hit.
 	struct	TraceState
 	{
-		Ray	world;		// world-space ray, restored when an instance is left
-		Ray	ray;		// ray of the current level
+		f3	world_o, world_d;	// world-space ray, restored when an instance is left
+		f3	o, d;				// ray of the current level
+		f3	inv, nearC, farC;	// its slab form
 		HitInfo	hit;	// hit.t is the current closest distance
-		const Bvh4Node*	nodes;	// node array of the current level
 		float	logU;	// log(max(u, 1e-12)) of the volume free-flight sample (scenes with volumes)
 		std::uint32_t	unbounded;	// this ray's scene: unbounded list base << 16 | count
 		std::uint32_t	entry;
 		std::uint32_t	instHittable;
 		RayOrigin	from;	// planar primitive the ray leaves from
-		bool	inInstance;
+		int	instBase;		// inside an instance: the stack height it was entered at; else -1
 		bool	found;
+
+		__device__ __forceinline__ Ray	ray() const { return Ray{o, d}; }
+		__device__ __forceinline__ Ray	world() const { return Ray{world_o, world_d}; }
+
+		__device__ __forceinline__ static void	slabAxis(float o, float d, float& inv, float& n, float& f)
+		{
+			float r = __builtin_amdgcn_rcpf(d);
+			// zero, denormal, infinite and NaN components: parallel
+			r = __builtin_amdgcn_classf(r, 0x198) ? r : 0x1p80f;	// +-normal, +-denormal
+			const float c = -o * r;
+			const float slack = fmaxf(fabsf(c) * 0x1p-21f, fabsf(r) * 0x1p-41f);
+			inv = r;
+			n = c - slack;
+			f = c + slack;
+		}
+
+		__device__ __forceinline__ void	setLevel(f3 origin, f3 dir)
+		{
+			o = origin;
+			d = dir;
+			slabAxis(o.x, d.x, inv.x, nearC.x, farC.x);
+			slabAxis(o.y, d.y, inv.y, nearC.y, farC.y);
+			slabAxis(o.z, d.z, inv.z, nearC.z, farC.z);
+		}
 	};
+
+	// Not a node: popped first when a scene has only unbounded hittables.
+	constexpr std::uint32_t	kNoEntry = kEmptyChild;
 
 	// Starts a traversal; returns false when there is nothing to traverse.
 	template <typename Stack>
-	__device__ __forceinline__ bool	traceBegin(TraceState& st, const SceneView& s, std::int32_t tlasRoot, std::uint32_t unbounded,
+	__device__ __forceinline__ bool	traceBegin(TraceState& st, std::int32_t tlasRoot, std::uint32_t unbounded,
 		const Ray& worldRay, float tMax, float logU, RayOrigin from, Stack& stack)
 	{
-		const Bvh4Node* tlas = s.tlas;
 		st.logU = logU;
 		st.from = from;
 		st.unbounded = unbounded;
-		st.world = worldRay;
-		st.ray = worldRay;
+		st.world_o = worldRay.o;
+		st.world_d = worldRay.d;
+		st.setLevel(worldRay.o, worldRay.d);
 		st.hit.t = tMax;
 		st.hit.hittable = 0xffffffffu;
 		st.hit.tri = -1;
 		// without bounded hittables only the unbounded ones are tested: start from the
-		// instance-exit entry, which leads straight to the end of the traversal
-		st.entry = tlasRoot >= 0 ? static_cast<std::uint32_t>(tlasRoot) : kExitInstance;
-		st.nodes = tlas;
+		// empty entry, which leads straight to the end of the traversal
+		st.entry = tlasRoot >= 0 ? static_cast<std::uint32_t>(tlasRoot) : kNoEntry;
 		st.instHittable = 0;
-		st.inInstance = false;
+		st.instBase = -1;
 		st.found = false;
 		// an any-hit query ends with entries still on the stack: every traversal starts
 		// from an empty stack
@@ -410,251 +406,221 @@ namespace luzgpu
 		return tlasRoot >= 0 || (unbounded & 0xffffu) != 0u;
 	}
 
-	// Processes the current entry; returns true when the traversal has ended (st.found and
-	// st.hit hold the result).
-	template <bool AnyHit, bool Count, int Feat, typename Stack>
-	__device__ __forceinline__ bool	traceStep(const SceneView& s, TraceState& st, float tMin, Stack& stack,
-		VisitCounter* counter)
+	// Opens the internal node st.entry: the nearest hit child becomes the entry, the others are
+	// pushed, farthest first. Returns false when no child is hit (the next entry is popped).
+	//
+	// Bound by VALU issue: the whole node is one straight line (about 130 instructions against
+	// the 330 of a form that branched per child, per push and for axis-parallel rays, and
+	// decoded exponents and leaf counts), so it keeps to four 16-byte loads issued together, a
+	// ready scale and ready stack entries in the node, one five-comparator sort, and stack
+	// writes that need no branch.
+	template <bool Count, typename Stack>
+	__device__ __forceinline__ bool	nodeStep(const SceneView& s, TraceState& st, Stack& stack, VisitCounter* counter)
+	{
+		//   n0 = origin xyz | scale x      n1 = scale yz | q_lo x, y
+		//   n2 = q_lo z | q_hi xyz         n3 = children
+		const uint4* np = reinterpret_cast<const uint4*>(reinterpret_cast<const char*>(s.nodes) + (st.entry << 6));
+		const uint4 n0 = np[0], n1 = np[1], n2 = np[2], n3 = np[3];
+		if (Count) counter->nodes++;
+		const float s0 = __uint_as_float(n0.w) * st.inv.x, s1 = __uint_as_float(n1.x) * st.inv.y, s2 = __uint_as_float(n1.y) * st.inv.z;
+		const float o0 = __uint_as_float(n0.x), o1 = __uint_as_float(n0.y), o2 = __uint_as_float(n0.z);
+		const float nb0 = fmaf(o0, st.inv.x, st.nearC.x), nb1 = fmaf(o1, st.inv.y, st.nearC.y), nb2 = fmaf(o2, st.inv.z, st.nearC.z);
+		const float fb0 = fmaf(o0, st.inv.x, st.farC.x), fb1 = fmaf(o1, st.inv.y, st.farC.y), fb2 = fmaf(o2, st.inv.z, st.farC.z);
+		// fma(q, s, b) is monotone in q (increasing for s >= 0), so on each axis the q_lo plane
+		// is the near one when the direction is positive and the q_hi plane otherwise: the words
+		// are chosen once per node
+		const bool p0 = st.inv.x > 0.0f, p1 = st.inv.y > 0.0f, p2 = st.inv.z > 0.0f;
+		const std::uint32_t near0 = p0 ? n1.z : n2.y, far0 = p0 ? n2.y : n1.z;
+		const std::uint32_t near1 = p1 ? n1.w : n2.z, far1 = p1 ? n2.z : n1.w;
+		const std::uint32_t near2 = p2 ? n2.x : n2.w, far2 = p2 ? n2.w : n2.x;
+		std::uint32_t e[4] = {n3.x, n3.y, n3.z, n3.w};
+		float key[4];	// entry distance; a miss sorts last
+		#pragma unroll
+		for (int k = 0; k < 4; k++)
+		{
+			const float l0 = fmaf(static_cast<float>((near0 >> (8 * k)) & 0xffu), s0, nb0);
+			const float h0 = fmaf(static_cast<float>((far0 >> (8 * k)) & 0xffu), s0, fb0);
+			const float l1 = fmaf(static_cast<float>((near1 >> (8 * k)) & 0xffu), s1, nb1);
+			const float h1 = fmaf(static_cast<float>((far1 >> (8 * k)) & 0xffu), s1, fb1);
+			const float l2 = fmaf(static_cast<float>((near2 >> (8 * k)) & 0xffu), s2, nb2);
+			const float h2 = fmaf(static_cast<float>((far2 >> (8 * k)) & 0xffu), s2, fb2);
+			const float near = fmaxf(fmaxf(fmaxf(l0, l1), l2), kTMinF);
+			const float far = fminf(fminf(fminf(h0, h1), h2), st.hit.t) * (1.0f + 0x1p-19f);
+			const bool in = (far >= near) & (k == 0 || e[k] != kEmptyChild);
+			key[k] = in ? near : INFINITY;
+		}
+		auto exchange = [&](int i, int j) {
+			const bool swap = key[j] < key[i];
+			const float ki = key[i];
+			const std::uint32_t ei = e[i];
+			key[i] = fminf(key[j], ki);
+			key[j] = fmaxf(key[j], ki);
+			e[i] = swap ? e[j] : ei;
+			e[j] = swap ? ei : e[j];
+		};
+		exchange(0, 1);
+		exchange(2, 3);
+		exchange(0, 2);
+		exchange(1, 3);
+		exchange(1, 2);
+		stack.push3(e[3], key[3] < INFINITY, e[2], key[2] < INFINITY, e[1], key[1] < INFINITY);
+		st.entry = e[0];
+		return key[0] < INFINITY;
+	}
+
+	// What a leaf step leaves: the next entry is on the stack, is st.entry already, or the
+	// any-hit query has ended.
+	enum : int { STEP_POP = 0, STEP_ENTRY = 1, STEP_END = 2 };
+
+	// Processes the leaf (or empty) st.entry: a run of triangles, a mesh instance (whose root
+	// becomes the entry), or a list of other primitives.
+	template <bool AnyHit, bool Count, int Feat>
+	__device__ __forceinline__ int	leafStep(const SceneView& s, TraceState& st, int stackHeight, float tMin, VisitCounter* counter)
 	{
 		const std::uint32_t entry = st.entry;
-		if (entry == kExitInstance)
+		const bool mesh = st.instBase >= 0;
+		if (entry == kNoEntry) return STEP_POP;
+		const std::uint32_t start = entry & kLeafStartMask;
+		const std::uint32_t kind = mesh ? kTopTriangles : (entry >> kTopKindShift) & 3u;
+		const std::uint32_t last = (entry >> kLeafCountShift) & (mesh ? 15u : 3u);	// count - 1
+		if (kind == kTopTriangles)
 		{
-			st.ray = st.world;
-			st.inInstance = false;
-			st.nodes = s.tlas;
-		}
-		else if ((entry & kLeafBit) == 0)
-		{
-			// the whole 64-byte node in four 16-byte loads issued together:
-			//   n0 = origin xyz | exp[3]      n1 = qlo[axis][child] x3 | qhi[0][child]
-			//   n2 = qhi[1], qhi[2] | child 0, 1      n3 = child 2, 3 | count[4] | pad
-			const uint4* np = reinterpret_cast<const uint4*>(st.nodes + entry);
-			const uint4 n0 = np[0], n1 = np[1], n2 = np[2], n3 = np[3];
-			if (Count) counter->nodes++;
-			// decode the four child boxes (plane = fma(q, 2^exp, origin)) and test them
-			const float org[3] = {__uint_as_float(n0.x), __uint_as_float(n0.y), __uint_as_float(n0.z)};
-			int ex[3];
-			for (int a = 0; a < 3; a++) ex[a] = static_cast<int>(static_cast<std::int8_t>((n0.w >> (8 * a)) & 0xffu));
-			const std::uint32_t qlo[3] = {n1.x, n1.y, n1.z};
-			const std::uint32_t qhi[3] = {n1.w, n2.x, n2.y};
-			const std::uint32_t child[4] = {n2.z, n2.w, n3.x, n3.y};
-			// per child: the entry distance as an ordering key (hit distances are >= T_MIN > 0,
-			// so their bit patterns order like the floats; a miss sorts last) and the stack entry
-			constexpr std::uint32_t kMissKey = 0xffffffffu;
-			std::uint32_t key[4], e[4];
-			const f3 inv = st.ray.inv;
-			if (inv.x != 0.0f && inv.y != 0.0f && inv.z != 0.0f)
-			{
-				// Slab distances straight from the quantised planes: with s = 2^exp / d and
-				// b = (origin - o) / d per axis, a plane at q is at t = fma(q, s, b). Rounding
-				// differs from decoding the plane first by a few ulps, so the interval is
-				// widened by 2^-20 relative (the quantised boxes already enclose the FP64 ones).
-				// 2^exp is a normal power of two (exp in [-100, 127]), so ldexp(1 / d, exp) is
-				// exactly 2^exp * (1 / d).
-				const float s0 = __builtin_amdgcn_ldexpf(inv.x, ex[0]), s1 = __builtin_amdgcn_ldexpf(inv.y, ex[1]),
-					s2 = __builtin_amdgcn_ldexpf(inv.z, ex[2]);
-				const float b0 = (org[0] - st.ray.o.x) * inv.x, b1 = (org[1] - st.ray.o.y) * inv.y, b2 = (org[2] - st.ray.o.z) * inv.z;
-				// fma(q, s, b) is monotone in q (increasing for s >= 0), so on each axis the
-				// q_lo plane is the near one when the direction is positive and the q_hi plane
-				// otherwise: choosing the words once per node gives the min / max of each pair
-				const std::uint32_t near0 = inv.x > 0.0f ? qlo[0] : qhi[0], far0 = inv.x > 0.0f ? qhi[0] : qlo[0];
-				const std::uint32_t near1 = inv.y > 0.0f ? qlo[1] : qhi[1], far1 = inv.y > 0.0f ? qhi[1] : qlo[1];
-				const std::uint32_t near2 = inv.z > 0.0f ? qlo[2] : qhi[2], far2 = inv.z > 0.0f ? qhi[2] : qlo[2];
-				#pragma unroll
-				for (int k = 0; k < 4; k++)
-				{
-					const std::uint32_t cnt = (n3.z >> (8 * k)) & 0xffu;
-					const float l0 = fmaf(static_cast<float>((near0 >> (8 * k)) & 0xffu), s0, b0);
-					const float h0 = fmaf(static_cast<float>((far0 >> (8 * k)) & 0xffu), s0, b0);
-					const float l1 = fmaf(static_cast<float>((near1 >> (8 * k)) & 0xffu), s1, b1);
-					const float h1 = fmaf(static_cast<float>((far1 >> (8 * k)) & 0xffu), s1, b1);
-					const float l2 = fmaf(static_cast<float>((near2 >> (8 * k)) & 0xffu), s2, b2);
-					const float h2 = fmaf(static_cast<float>((far2 >> (8 * k)) & 0xffu), s2, b2);
-					const float near = fmaxf(fmaxf(l0, l1), l2) * (1.0f - 0x1p-20f);
-					const float far = fminf(fminf(h0, h1), h2) * (1.0f + 0x1p-20f);
-					const float t = fmaxf(near, kTMinF);
-					key[k] = cnt != 255u && fminf(far, st.hit.t) > t ? __float_as_uint(t) : kMissKey;
-					e[k] = cnt > 0 ? leafEntry(static_cast<std::int32_t>(child[k]), static_cast<std::int32_t>(cnt)) : child[k];
-				}
-			}
-			else
-			{
-				// an axis-parallel ray: AABB::hit tests the origin against that slab (AABB.cpp:37-80)
-				float sc[3];
-				for (int a = 0; a < 3; a++) sc[a] = __int_as_float((ex[a] + 127) << 23);
-				#pragma unroll
-				for (int k = 0; k < 4; k++)
-				{
-					const std::uint32_t cnt = (n3.z >> (8 * k)) & 0xffu;
-					float lo[3], hi[3];
-					for (int a = 0; a < 3; a++)
-					{
-						lo[a] = fmaf(static_cast<float>((qlo[a] >> (8 * k)) & 0xffu), sc[a], org[a]);
-						hi[a] = fmaf(static_cast<float>((qhi[a] >> (8 * k)) & 0xffu), sc[a], org[a]);
-					}
-					float t;
-					key[k] = cnt != 255u && boxHit(st.ray, lo, hi, st.hit.t, t) ? __float_as_uint(t) : kMissKey;
-					e[k] = cnt > 0 ? leafEntry(static_cast<std::int32_t>(child[k]), static_cast<std::int32_t>(cnt)) : child[k];
-				}
-			}
-			// the hit children by entry distance, in child order among equal distances (a
-			// compare-exchange network of adjacent pairs is a stable sort), pushed far to near,
-			// the nearest taken next. An any-hit query ends at its first hit whatever the order
-			// (BVHNode::hitAny is unordered, BVHNode.cpp:326-380); near first finds occluders sooner.
-			auto exchange = [&](int i) {
-				const bool swap = key[i] > key[i + 1];
-				const std::uint32_t ki = key[i], ei = e[i];
-				key[i] = swap ? key[i + 1] : ki;
-				e[i] = swap ? e[i + 1] : ei;
-				key[i + 1] = swap ? ki : key[i + 1];
-				e[i + 1] = swap ? ei : e[i + 1];
-			};
-			exchange(0); exchange(1); exchange(0); exchange(2); exchange(1); exchange(0);
-			if (key[0] != kMissKey)
-			{
-				if (key[3] != kMissKey) stack.push(e[3]);
-				if (key[2] != kMissKey) stack.push(e[2]);
-				if (key[1] != kMissKey) stack.push(e[1]);
-				st.entry = e[0];
-				return false;
-			}
-		}
-		else
-		{
-			const std::int32_t start = static_cast<std::int32_t>(entry & 0x07ffffffu);
-			const std::int32_t count = static_cast<std::int32_t>((entry >> 27) & 0xfu) + 1;
-			for (std::int32_t i = 0; i < count; i++)
+			const GpuTri* tris = mesh ? s.meshTris : s.topTris;
+			// the triangle the ray leaves from: a mesh triangle by its slot, a top-level one by
+			// its hittable
+			const std::int32_t skip = mesh ? (st.instHittable == st.from.hittable ? st.from.tri : -1)
+				: static_cast<std::int32_t>(st.from.hittable);
+			for (std::uint32_t i = 0; i <= last; i++)
 			{
 				if (Count) counter->prims++;
-				if (st.inInstance)
-				{
-					if (start + i == st.from.tri && st.instHittable == st.from.hittable) continue;
-					const GpuTri& tri = s.meshTris[start + i];
-					float t, u, v;
-					if (triHit(tri, st.ray, tMin, st.hit.t, t, u, v))
-					{
-						st.found = true;
-						st.hit.t = t; st.hit.u = u; st.hit.v = v;
-						st.hit.hittable = st.instHittable;
-						st.hit.tri = start + i;
-						if (AnyHit) return true;
-					}
-					continue;
-				}
-				const uint2 item = s.tlasLeaf[start + i];
-				const std::uint32_t h = item.x;
-				const std::uint32_t kind = item.y >> kKindShift;
-				const std::uint32_t idx = item.y & kIndexMask;
-				if (kind == GPU_HIT_TRIANGLE)
-				{
-					float t, u, v;
-					if (h != st.from.hittable && triHit(s.topTris[idx], st.ray, tMin, st.hit.t, t, u, v))
-					{
-						st.found = true;
-						st.hit.t = t; st.hit.u = u; st.hit.v = v;
-						st.hit.hittable = h;
-						st.hit.tri = -1;
-						if (AnyHit) return true;
-					}
-				}
-				else if (kind == GPU_HIT_RECTANGLE)
-				{
-					float t;
-					if (h != st.from.hittable && rectHit(s.rects[idx], st.ray, tMin, st.hit.t, t))
-					{
-						st.found = true;
-						st.hit.t = t;
-						st.hit.hittable = h;
-						st.hit.tri = -1;
-						if (AnyHit) return true;
-					}
-				}
-				else if ((Feat & kFeatAnalytic) && kind == GPU_HIT_SPHERE)
-				{
-					float t;
-					if (sphereHit(s.spheres[idx], st.ray, tMin, st.hit.t, t))
-					{
-						st.found = true;
-						st.hit.t = t;
-						st.hit.hittable = h;
-						st.hit.tri = -1;
-						if (AnyHit) return true;
-					}
-				}
-				else if ((Feat & kFeatAnalytic) && kind == GPU_HIT_CUBE)
-				{
-					// Cube::hit (Cube.cpp:97-111): its six faces, closest first-found
-					for (int f = 0; f < 6; f++)
-					{
-						float t;
-						if ((h != st.from.hittable || f != st.from.tri) && rectHit(s.cubeFaces[6 * idx + f], st.ray, tMin, st.hit.t, t))
-						{
-							st.found = true;
-							st.hit.t = t;
-							st.hit.hittable = h;
-							st.hit.tri = f;
-							if (AnyHit) return true;
-						}
-					}
-				}
-				else if ((Feat & kFeatAnalytic) && kind == GPU_HIT_VOLUME)
-				{
-					float t;
-					if (volumeHit(s.volumes[idx], st.ray, tMin, st.hit.t, st.logU, t))
-					{
-						st.found = true;
-						st.hit.t = t;
-						st.hit.hittable = h;
-						st.hit.tri = -1;
-						if (AnyHit) return true;
-					}
-				}
-				else if ((Feat & kFeatAnalytic) && kind == GPU_HIT_HIDDEN_SPHERE)
-				{
-					// an invisible sphere (Sphere.cpp:227-233, 271-277): never hit
-				}
-				else
-				{
-					// 3x4 map and mesh links: one group of four 16-byte loads
-					const float4* ip = reinterpret_cast<const float4*>(s.instances + idx);
-					const float4 r0 = ip[0], r1 = ip[1], r2 = ip[2];
-					const int4 links = reinterpret_cast<const int4*>(ip)[3];
-					if (i + 1 < count)
-					{
-						stack.push(leafEntry(start + i + 1, count - i - 1));
-					}
-					stack.push(kExitInstance);
-					st.ray = toLocal(r0, r1, r2, st.world);
-					st.inInstance = true;
-					st.nodes = s.blas;
-					st.instHittable = h;
-					st.entry = static_cast<std::uint32_t>(links.x);
-					return false;
-				}
-			}
-		}
-		if (stack.empty())
-		{
-			// the unbounded hittables after the acceleration structure (HitHelper.cpp:5-32)
-			const std::uint32_t ubBase = st.unbounded >> 16, ubCount = (Feat & kFeatAnalytic) ? (st.unbounded & 0xffffu) : 0u;
-			for (std::uint32_t i = 0; i < ubCount; i++)
-			{
-				const std::uint32_t h = s.unbounded[ubBase + i];
-				const GpuPlane& pl = s.planes[s.hittables[h].kindIndex & kIndexMask];
-				float t;
-				if (h != st.from.hittable && planeHit(pl, st.world, tMin, st.hit.t, t))
+				const std::int32_t slot = static_cast<std::int32_t>(start + i);
+				float t, u, v;
+				std::int32_t id;
+				const bool hit = triHit(tris[slot], st.ray(), tMin, st.hit.t, t, u, v, id);
+				if (hit && (mesh ? slot : id) != skip)
 				{
 					st.found = true;
-					st.hit.t = t;
-					st.hit.hittable = h;
-					st.hit.tri = -1;
-					if (AnyHit) return true;
+					st.hit.t = t; st.hit.u = u; st.hit.v = v;
+					st.hit.hittable = mesh ? st.instHittable : static_cast<std::uint32_t>(id);
+					st.hit.tri = mesh ? slot : -1;
+					if (AnyHit) return STEP_END;
 				}
 			}
-			return true;
+			return STEP_POP;
 		}
-		st.entry = stack.pop();
-		return false;
+		if (kind == kTopInstance)
+		{
+			if (Count) counter->prims++;
+			// 3x4 map and mesh links: one group of four 16-byte loads
+			const float4* ip = reinterpret_cast<const float4*>(s.instances + start);
+			const float4 r0 = ip[0], r1 = ip[1], r2 = ip[2];
+			const int4 links = reinterpret_cast<const int4*>(ip)[3];
+			const Ray local = toLocal(r0, r1, r2, st.world());
+			st.setLevel(local.o, local.d);
+			st.instBase = stackHeight;
+			st.instHittable = static_cast<std::uint32_t>(links.w);
+			st.entry = static_cast<std::uint32_t>(links.x);
+			return STEP_ENTRY;
+		}
+		const Ray ray = st.ray();
+		for (std::uint32_t i = 0; i <= last; i++)
+		{
+			if (Count) counter->prims++;
+			const uint2 item = s.tlasLeaf[start + i];
+			const std::uint32_t h = item.x;
+			const std::uint32_t hk = item.y >> kKindShift;
+			const std::uint32_t idx = item.y & kIndexMask;
+			float t = 0.0f;
+			bool hit = false;
+			std::int32_t part = -1;
+			if (hk == GPU_HIT_RECTANGLE)
+			{
+				hit = h != st.from.hittable && rectHit(s.rects[idx], ray, tMin, st.hit.t, t);
+			}
+			else if ((Feat & kFeatAnalytic) && hk == GPU_HIT_SPHERE)
+			{
+				hit = sphereHit(s.spheres[idx], ray, tMin, st.hit.t, t);
+			}
+			else if ((Feat & kFeatAnalytic) && hk == GPU_HIT_CUBE)
+			{
+				// Cube::hit (Cube.cpp:97-111): its six faces, closest first-found
+				float closest = st.hit.t;
+				for (int f = 0; f < 6; f++)
+				{
+					float ft;
+					if ((h != st.from.hittable || f != st.from.tri) && rectHit(s.cubeFaces[6 * idx + f], ray, tMin, closest, ft))
+					{
+						hit = true;
+						t = closest = ft;
+						part = f;
+						if (AnyHit) break;
+					}
+				}
+			}
+			else if ((Feat & kFeatAnalytic) && hk == GPU_HIT_VOLUME)
+			{
+				hit = volumeHit(s.volumes[idx], ray, tMin, st.hit.t, st.logU, t);
+			}
+			// GPU_HIT_HIDDEN_SPHERE, an invisible sphere (Sphere.cpp:227-233, 271-277): never hit
+			if (hit)
+			{
+				st.found = true;
+				st.hit.t = t;
+				st.hit.hittable = h;
+				st.hit.tri = part;
+				if (AnyHit) return STEP_END;
+			}
+		}
+		return STEP_POP;
+	}
+
+	// Takes the next entry off the stack, leaving an instance whose entries are used up; returns
+	// true when the traversal has ended (st.found and st.hit hold the result).
+	template <bool AnyHit, int Feat, typename Stack>
+	__device__ __forceinline__ bool	popEntry(const SceneView& s, TraceState& st, float tMin, Stack& stack)
+	{
+		if (stack.sp == st.instBase)
+		{
+			st.setLevel(st.world_o, st.world_d);
+			st.instBase = -1;
+		}
+		if (stack.sp != 0)
+		{
+			st.entry = stack.pop();
+			return false;
+		}
+		// the unbounded hittables after the acceleration structure (HitHelper.cpp:5-32)
+		const std::uint32_t ubBase = st.unbounded >> 16, ubCount = (Feat & kFeatAnalytic) ? (st.unbounded & 0xffffu) : 0u;
+		for (std::uint32_t i = 0; i < ubCount; i++)
+		{
+			const std::uint32_t h = s.unbounded[ubBase + i];
+			const GpuPlane& pl = s.planes[s.hittables[h].kindIndex & kIndexMask];
+			float t;
+			if (h != st.from.hittable && planeHit(pl, st.world(), tMin, st.hit.t, t))
+			{
+				st.found = true;
+				st.hit.t = t;
+				st.hit.hittable = h;
+				st.hit.tri = -1;
+				if (AnyHit) return true;
+			}
+		}
+		return true;
+	}
+
+	// Runs a traversal to its end: a lane opens nodes until it holds a leaf.
+	template <bool AnyHit, bool Count, int Feat, typename Stack>
+	__device__ __forceinline__ void	traceToEnd(const SceneView& s, TraceState& st, float tMin, Stack& stack, VisitCounter* counter)
+	{
+		for (;;)
+		{
+			while ((st.entry & kLeafBit) == 0u)
+			{
+				if (!nodeStep<Count>(s, st, stack, counter) && popEntry<AnyHit, Feat>(s, st, tMin, stack)) return;
+			}
+			const int r = leafStep<AnyHit, Count, Feat>(s, st, stack.sp, tMin, counter);
+			if (r == STEP_END || (r == STEP_POP && popEntry<AnyHit, Feat>(s, st, tMin, stack))) return;
+		}
 	}
 
 	__device__ __forceinline__ std::uint32_t	unboundedOf(const GpuParams& p)
@@ -669,25 +635,14 @@ namespace luzgpu
 		float tMax, HitInfo& hit)
 	{
 		const GpuInstance& in = s.instances[instance];
-		TraceState st;
-		st.world = world;
-		st.ray = toLocal(in, world);
-		st.hit.t = tMax;
-		st.hit.hittable = 0xffffffffu;
-		st.hit.tri = -1;
-		st.nodes = s.blas;
-		st.logU = 0.0f;
-		st.unbounded = 0u;
-		st.entry = static_cast<std::uint32_t>(in.blasRoot);
-		st.instHittable = hittable;
-		st.from = kNoOrigin;
-		st.inInstance = true;
-		st.found = false;
+		const Ray local = toLocal(in, world);
 		LocalStack stack;
-		stack.reset();
-		while (!traceStep<false, false, 0>(s, st, kTMinF, stack, nullptr))
-		{
-		}
+		TraceState st;
+		// entered at the bottom of the stack: popEntry ends the traversal there
+		traceBegin(st, in.blasRoot, 0u, local, tMax, 0.0f, kNoOrigin, stack);
+		st.instBase = 0;
+		st.instHittable = hittable;
+		traceToEnd<false, false, 0>(s, st, kTMinF, stack, nullptr);
 		hit = st.hit;
 		return st.found;
 	}
@@ -706,11 +661,9 @@ namespace luzgpu
 		HitInfo& hit, Stack& stack, VisitCounter* counter = nullptr, float logU = 0.0f, RayOrigin from = kNoOrigin)
 	{
 		TraceState st;
-		if (traceBegin(st, s, p.tlasRoot, unboundedOf(p), worldRay, tMax, logU, from, stack))
+		if (traceBegin(st, p.tlasRoot, unboundedOf(p), worldRay, tMax, logU, from, stack))
 		{
-			while (!traceStep<AnyHit, Count, Feat>(s, st, tMin, stack, counter))
-			{
-			}
+			traceToEnd<AnyHit, Count, Feat>(s, st, tMin, stack, counter);
 		}
 		hit = st.hit;
 		return st.found;

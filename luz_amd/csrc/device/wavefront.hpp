@@ -135,9 +135,14 @@ namespace luzgpu
 	constexpr unsigned	kWaveGrid = 2048;	// 256 CUs x 8 waves per SIMD x 4 SIMDs / 4 waves per block
 	// default traversal launch shape: as many persistent waves as the traversal kernels'
 	// registers let every SIMD hold (256 CUs x 4 SIMDs x 5 waves / 4 waves per block; 2 %
-	// faster than 1024 blocks on the sphere frame), whole-wave claims of 64 rays
+	// faster than 1024 blocks on the sphere frame)
 	constexpr unsigned	kDefaultGrid = 1280;
-	constexpr int	kDefaultRefill = 64;
+	// Idle lanes at which a wave takes new rays when the caller names no number: 48 in
+	// triangle-only scenes (1080p spheres: extend + shadow 22.4 ms, against 24.5 at 64 and
+	// 24.1 at 16), 16 in scenes with analytic primitives or volumes, whose rays differ more in
+	// length (720p hazy terrain: 52.3 ms, against 62.2 at 48 and 84.0 at 64).
+	constexpr int	kRefillTriangles = 48;
+	constexpr int	kRefillAnalytic = 16;
 	// Lanes whose next entry is a leaf (primitive tests, an instance entry) wait while other
 	// lanes of the wave still have internal nodes to open, until this many are waiting or no
 	// lane has a node left; then every live lane takes one step. Each lane's entries are
@@ -306,7 +311,10 @@ namespace luzgpu
 	// Persistent traversal over one ray queue with lane refill: a lane whose traversal has
 	// ended takes the next ray of the queue once at least `refillAt` lanes of its wave are
 	// idle (refillAt = 64: the wave claims 64 rays at a time and every lane traverses its
-	// ray to the end before the next claim).
+	// ray to the end before the next claim). Each turn of the loop runs the leaf code, if its
+	// turn has come, then the node code, then the pop they share, each once per wave.
+	// VALU-bound before the node test became a straight line (nodeStep): 1080p spheres extend
+	// 27.7 -> 18.9 ms, shadow 5.8 -> 3.5; 720p hazy terrain 50.9 -> 25.6 and 53.7 -> 26.7.
 	// Source supplies the queue: count(), load(slot, ray, tMax) and store(slot, state).
 	template <bool AnyHit, bool Count, int Feat, int LdsDepth, typename Source>
 	__device__ __forceinline__ void	traceQueue(const SceneView& s, const PassJob* jobs, Source& src, std::uint32_t* fetch,
@@ -339,57 +347,6 @@ namespace luzgpu
 		// the last job's root and unbounded list: a single-scene pass loads them once per lane
 		std::uint32_t lastJob = 0xffffffffu, lastUnbounded = 0u;
 		std::int32_t lastRoot = -1;
-		if (refillAt >= 64)
-		{
-			// whole-wave cadence: the wave claims 64 rays, each lane runs its traversal to the
-			// end in a tight loop, then the wave claims the next 64
-			for (;;)
-			{
-				const std::uint32_t k = feed.hand(~0ull, n, fetch, chunk);
-				if (__ballot(k != 0xffffffffu) == 0ull)
-				{
-					break;
-				}
-				bool done = true;
-				if (k != 0xffffffffu)
-				{
-					Ray r;
-					float tMax, logU;
-					RayOrigin from;
-					const std::uint32_t job = src.load(k, r, tMax, logU, from);
-					if (job != lastJob)
-					{
-						const GpuParams& jp = jobs[job].params;
-						lastJob = job;
-						lastRoot = jp.tlasRoot;
-						lastUnbounded = unboundedOf(jp);
-					}
-					done = !traceBegin(st, s, lastRoot, lastUnbounded, r, tMax, logU, from, stack);
-				}
-				for (;;)
-				{
-					const bool wantNode = !done && (st.entry & kLeafBit) == 0u;
-					const unsigned long long live = __ballot(!done);
-					if (live == 0ull)
-					{
-						break;
-					}
-					const unsigned long long nodes = __ballot(wantNode);
-					const bool leafTurn = nodes == 0ull || __popcll(live & ~nodes) >= kLeafBatch<Feat, AnyHit>;
-					if (leafTurn ? !done : wantNode)
-					{
-						done = traceStep<AnyHit, Count, Feat>(s, st, kTMinF, stack, &visits);
-					}
-				}
-				if (k != 0xffffffffu)
-				{
-					src.store(k, st);
-					rays++;
-				}
-			}
-			flushCounters(counters, counterSlot, rays, visits, Count);
-			return;
-		}
 		while (true)
 		{
 			const unsigned long long idle = __ballot(!active);
@@ -410,7 +367,7 @@ namespace luzgpu
 						lastRoot = jp.tlasRoot;
 						lastUnbounded = unboundedOf(jp);
 					}
-					active = traceBegin(st, s, lastRoot, lastUnbounded, r, tMax, logU, from, stack);
+					active = traceBegin(st, lastRoot, lastUnbounded, r, tMax, logU, from, stack);
 					if (!active)
 					{
 						src.store(slot, st);
@@ -425,7 +382,22 @@ namespace luzgpu
 			const bool wantNode = active && (st.entry & kLeafBit) == 0u;
 			const unsigned long long nodes = __ballot(wantNode);
 			const bool leafTurn = nodes == 0ull || __popcll(__ballot(active) & ~nodes) >= kLeafBatch<Feat, AnyHit>;
-			if ((leafTurn ? active : wantNode) && traceStep<AnyHit, Count, Feat>(s, st, kTMinF, stack, &visits))
+			bool pop = false, ended = false;
+			if (leafTurn && active && !wantNode)
+			{
+				const int step = leafStep<AnyHit, Count, Feat>(s, st, stack.sp, kTMinF, &visits);
+				pop = step == STEP_POP;
+				ended = step == STEP_END;
+			}
+			if (wantNode)
+			{
+				pop = !nodeStep<Count>(s, st, stack, &visits);
+			}
+			if (pop)
+			{
+				ended = popEntry<AnyHit, Feat>(s, st, kTMinF, stack);
+			}
+			if (ended)
 			{
 				src.store(slot, st);
 				rays++;
@@ -916,12 +888,14 @@ namespace luzgpu
 		unsigned	chunk = 0;			// most rays a wave claims per queue atomic
 		int	ldsStack = 0;			// LDS stack entries per lane (the rest spill to HBM)
 
-		WaveTuning	resolved() const
+		// `features`: the scene's kFeat* classes
+		WaveTuning	resolved(int features) const
 		{
 			WaveTuning t = *this;
 			if (t.grid == 0) t.grid = kDefaultGrid;
-			if (t.extendRefill == 0) t.extendRefill = kDefaultRefill;
-			if (t.shadowRefill == 0) t.shadowRefill = kDefaultRefill;
+			const int refill = (features & kFeatAnalytic) ? kRefillAnalytic : kRefillTriangles;
+			if (t.extendRefill == 0) t.extendRefill = refill;
+			if (t.shadowRefill == 0) t.shadowRefill = refill;
 			if (t.chunk == 0) t.chunk = kFetchChunk;
 			if (t.ldsStack == 0) t.ldsStack = kWaveLdsStack;
 			if (t.grid > kWaveGrid || t.extendRefill < 1 || t.extendRefill > 64 || t.shadowRefill < 1 || t.shadowRefill > 64
@@ -1165,7 +1139,7 @@ namespace luzgpu
 	inline void	renderWavefront(WavefrontState& st, const SceneView& s, int features, const std::vector<BatchJob>& jobs,
 		unsigned long long* counters, hipStream_t stream, bool count, StageTimes* times, WaveTuning tune)
 	{
-		tune = tune.resolved();
+		tune = tune.resolved(features);
 		if (jobs.empty() || jobs.size() > kMaxBatchScenes)
 		{
 			throw std::invalid_argument("wavefront: 1.." + std::to_string(kMaxBatchScenes) + " scenes per launch");

@@ -558,13 +558,16 @@ namespace luzgpu
 			Ref	group(std::vector<std::uint32_t> items)
 			{
 				AABBd box = boxes[items[0]];
-				bool instances = false;
+				std::size_t instances = 0, triangles = 0;
+				auto isTriangle = [&](std::uint32_t h) { return (hittables[h].kindIndex >> kKindShift) == GPU_HIT_TRIANGLE; };
 				for (std::uint32_t h : items)
 				{
 					box = merge(box, boxes[h]);
-					instances = instances || (hittables[h].kindIndex >> kKindShift) == GPU_HIT_INSTANCE;
+					instances += (hittables[h].kindIndex >> kKindShift) == GPU_HIT_INSTANCE ? 1u : 0u;
+					triangles += isTriangle(h) ? 1u : 0u;
 				}
-				if (items.size() == 1 || (!instances && items.size() <= 4))
+				const bool mixed = triangles != 0 && triangles != items.size();
+				if (items.size() == 1 || (instances == 0 && !mixed && items.size() <= kTopLeafMax))
 				{
 					const std::int32_t start = static_cast<std::int32_t>(prims.size());
 					prims.insert(prims.end(), items.begin(), items.end());
@@ -578,12 +581,21 @@ namespace luzgpu
 					cb = i == 0 ? cc : merge(cb, cc);
 				}
 				const int axis = largestAxis(cb);
-				const std::size_t mid = items.size() / 2;
-				std::nth_element(items.begin(), items.begin() + static_cast<std::ptrdiff_t>(mid), items.end(),
-					[&](std::uint32_t a, std::uint32_t b) {
-						const double ca = boxes[a].lo[axis] + boxes[a].hi[axis], cbv = boxes[b].lo[axis] + boxes[b].hi[axis];
-						return ca < cbv || (ca == cbv && a < b);
-					});
+				std::size_t mid = items.size() / 2;
+				if (instances == 0 && mixed && items.size() <= kTopLeafMax)
+				{
+					// a leaf's triangles are a run of their own array: the other primitives apart
+					std::stable_partition(items.begin(), items.end(), isTriangle);
+					mid = triangles;
+				}
+				else
+				{
+					std::nth_element(items.begin(), items.begin() + static_cast<std::ptrdiff_t>(mid), items.end(),
+						[&](std::uint32_t a, std::uint32_t b) {
+							const double ca = boxes[a].lo[axis] + boxes[a].hi[axis], cbv = boxes[b].lo[axis] + boxes[b].hi[axis];
+							return ca < cbv || (ca == cbv && a < b);
+						});
+				}
 				const std::size_t idx = nodes.size();
 				nodes.push_back(BvhNode{});
 				const Ref l = group(std::vector<std::uint32_t>(items.begin(), items.begin() + static_cast<std::ptrdiff_t>(mid)));
@@ -628,7 +640,9 @@ namespace luzgpu
 			return x * y + x * z + y * z;
 		}
 
-		void	encodeWide(Bvh4Node& n, const std::vector<WideSlot>& slots)
+		// `leaf(start, count)` gives a leaf's reference.
+		template <typename Leaf>
+		void	encodeWide(Bvh4Node& n, const std::vector<WideSlot>& slots, const Leaf& leaf)
 		{
 			float lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
 			for (const WideSlot& s : slots)
@@ -663,7 +677,7 @@ namespace luzgpu
 					}
 					if (ok)
 					{
-						n.exp[a] = static_cast<std::int8_t>(e);
+						n.scale[a] = scale;
 						break;
 					}
 				}
@@ -672,13 +686,11 @@ namespace luzgpu
 			{
 				if (k < slots.size())
 				{
-					n.child[k] = slots[k].child;
-					n.count[k] = static_cast<std::uint8_t>(slots[k].count);
+					n.child[k] = slots[k].count == 0 ? static_cast<std::uint32_t>(slots[k].child) : leaf(slots[k].child, slots[k].count);
 				}
 				else
 				{
-					n.child[k] = 0;
-					n.count[k] = 255;
+					n.child[k] = kEmptyChild;
 					for (int a = 0; a < 3; a++) { n.qlo[a][k] = 255; n.qhi[a][k] = 0; }
 				}
 			}
@@ -686,7 +698,8 @@ namespace luzgpu
 
 		// Collapses the binary device tree below `node` into 4-wide nodes (largest-area
 		// internal child opened first). Returns the wide index of the new node.
-		std::int32_t	widen(const std::vector<BvhNode>& bin, std::int32_t node, std::vector<Bvh4Node>& out)
+		template <typename Leaf>
+		std::int32_t	widen(const std::vector<BvhNode>& bin, std::int32_t node, std::vector<Bvh4Node>& out, const Leaf& leaf)
 		{
 			std::vector<WideSlot> slots;
 			auto addChildren = [&](std::int32_t b) {
@@ -728,9 +741,9 @@ namespace luzgpu
 			out.push_back(Bvh4Node{});
 			for (WideSlot& w : slots)
 			{
-				if (w.count == 0) w.child = widen(bin, w.child, out);
+				if (w.count == 0) w.child = widen(bin, w.child, out, leaf);
 			}
-			encodeWide(out[idx], slots);
+			encodeWide(out[idx], slots, leaf);
 			return static_cast<std::int32_t>(idx);
 		}
 
@@ -742,9 +755,9 @@ namespace luzgpu
 			int valid = 0, below = 0;
 			for (int k = 0; k < 4; k++)
 			{
-				if (n.count[k] == 255) continue;
+				if (n.child[k] == kEmptyChild) continue;
 				valid++;
-				if (n.count[k] == 0) below = std::max(below, wideStackBound(nodes, n.child[k]));
+				if (!(n.child[k] & kLeafBit)) below = std::max(below, wideStackBound(nodes, static_cast<std::int32_t>(n.child[k])));
 			}
 			return std::max(0, valid - 1) + below;
 		}
@@ -755,9 +768,21 @@ namespace luzgpu
 			int d = 0;
 			for (int k = 0; k < 4; k++)
 			{
-				if (n.count[k] == 0) d = std::max(d, wideDepth(nodes, n.child[k]));
+				if (!(n.child[k] & kLeafBit)) d = std::max(d, wideDepth(nodes, static_cast<std::int32_t>(n.child[k])));
 			}
 			return 1 + d;
+		}
+
+		// Adds `by` to every internal child reference.
+		void	shiftNodes(std::vector<Bvh4Node>& nodes, std::uint32_t by)
+		{
+			for (Bvh4Node& n : nodes)
+			{
+				for (std::uint32_t& c : n.child)
+				{
+					if (!(c & kLeafBit)) c += by;
+				}
+			}
 		}
 
 		GpuTri	packTriangle(const Triangle& t, std::int32_t prim)
@@ -1071,7 +1096,13 @@ namespace luzgpu
 				}
 			}
 			const std::int32_t binaryRoot = packBlas(blas, triBase, p.blasNodes);
-			meshRoot[m] = widen(p.blasNodes, binaryRoot, p.blasWide);
+			meshRoot[m] = widen(p.blasNodes, binaryRoot, p.blasWide, [](std::int32_t start, std::int32_t count) {
+				if (static_cast<std::uint32_t>(start) > kLeafStartMask || count > 16)
+				{
+					throw std::runtime_error("Unsupported for the device path: mesh triangle slots beyond 27 bits");
+				}
+				return kLeafBit | (static_cast<std::uint32_t>(count - 1) << kLeafCountShift) | static_cast<std::uint32_t>(start);
+			});
 			p.blasDeviceDepth = std::max(p.blasDeviceDepth, wideDepth(p.blasWide, meshRoot[m]));
 			p.blasStackBound = std::max(p.blasStackBound, wideStackBound(p.blasWide, meshRoot[m]));
 			p.triangleCount += mesh.triangles.size();
@@ -1210,6 +1241,7 @@ namespace luzgpu
 					g.blasRoot = meshRoot[inst.mesh];
 					g.triBase = meshTriBase[inst.mesh];
 					g.normalBase = meshNormalBase[inst.mesh];
+					g.hittable = static_cast<std::uint32_t>(i);
 					gh.kindIndex = (GPU_HIT_INSTANCE << kKindShift) | static_cast<std::uint32_t>(p.instances.size());
 					p.instances.push_back(g);
 					break;
@@ -1275,10 +1307,46 @@ namespace luzgpu
 			{
 				p.params.tlasRoot = root.child;
 			}
-			p.params.tlasRoot = widen(p.tlasNodes, p.params.tlasRoot, p.tlasWide);
+			// top-level triangles in leaf order, so a leaf's triangles are one run
+			std::vector<GpuTri> ordered;
+			ordered.reserve(p.topTris.size());
+			std::vector<std::uint32_t> slotOf(p.topTris.size(), 0xffffffffu);
+			auto take = [&](std::uint32_t old) {
+				if (slotOf[old] != 0xffffffffu) return;
+				slotOf[old] = static_cast<std::uint32_t>(ordered.size());
+				ordered.push_back(p.topTris[old]);
+			};
+			for (const std::uint32_t h : p.tlasPrims)
+			{
+				if ((p.hittables[h].kindIndex >> kKindShift) == GPU_HIT_TRIANGLE) take(p.hittables[h].kindIndex & kIndexMask);
+			}
+			for (std::uint32_t k = 0; k < p.topTris.size(); k++) take(k);	// degenerate ones, never in a leaf
+			p.topTris.swap(ordered);
+			for (GpuHittable& h : p.hittables)
+			{
+				if ((h.kindIndex >> kKindShift) == GPU_HIT_TRIANGLE) h.kindIndex = (GPU_HIT_TRIANGLE << kKindShift) | slotOf[h.kindIndex & kIndexMask];
+			}
+			p.params.tlasRoot = widen(p.tlasNodes, p.params.tlasRoot, p.tlasWide, [&](std::int32_t start, std::int32_t count) {
+				const std::uint32_t kindIndex = p.hittables[p.tlasPrims[static_cast<std::size_t>(start)]].kindIndex;
+				const std::uint32_t kind = kindIndex >> kKindShift;
+				const std::uint32_t top = kind == GPU_HIT_TRIANGLE ? kTopTriangles : kind == GPU_HIT_INSTANCE ? kTopInstance : kTopItems;
+				const std::uint32_t first = top == kTopItems ? static_cast<std::uint32_t>(start) : kindIndex & kIndexMask;
+				if (first > kLeafStartMask)
+				{
+					throw std::runtime_error("Unsupported for the device path: top-level primitives beyond 27 bits");
+				}
+				return kLeafBit | (top << kTopKindShift) | (static_cast<std::uint32_t>(count - 1) << kLeafCountShift) | first;
+			});
 			p.tlasDeviceDepth = wideDepth(p.tlasWide, p.params.tlasRoot);
 			p.tlasStackBound = wideStackBound(p.tlasWide, p.params.tlasRoot);
 		}
+		// one node array on the device: the mesh BVHs follow the top level
+		if (p.tlasWide.size() + p.blasWide.size() > kMaxNodes)
+		{
+			throw std::runtime_error("Unsupported for the device path: more than 2^26 BVH nodes");
+		}
+		shiftNodes(p.blasWide, static_cast<std::uint32_t>(p.tlasWide.size()));
+		for (GpuInstance& in : p.instances) in.blasRoot += static_cast<std::int32_t>(p.tlasWide.size());
 		p.tlasLeaf.reserve(2 * p.tlasPrims.size());
 		for (const std::uint32_t h : p.tlasPrims)
 		{
@@ -1606,21 +1674,34 @@ namespace luzgpu
 				if (idx > kIndexMask) throw std::runtime_error("Unsupported: batch too large for 28-bit primitive indices");
 				return (kind << kKindShift) | idx;
 			};
+			// a part's references count its own nodes, top level first; merged, every part's top
+			// level comes before every mesh BVH (whose share is added once the parts are known)
+			auto leafRef = [](std::uint32_t c, std::uint32_t by) {
+				const std::uint64_t start = static_cast<std::uint64_t>(c & kLeafStartMask) + by;
+				if (start > kLeafStartMask) throw std::runtime_error("Unsupported: batch too large for 27-bit leaf references");
+				return (c & ~kLeafStartMask) | static_cast<std::uint32_t>(start);
+			};
+			const std::uint32_t partTlas = static_cast<std::uint32_t>(p.tlasWide.size());
 			for (Bvh4Node n : p.tlasWide)
 			{
-				for (int k = 0; k < 4; k++)
+				for (std::uint32_t& c : n.child)
 				{
-					if (n.count[k] == 0) n.child[k] += static_cast<std::int32_t>(tlasBase);
-					else if (n.count[k] != 255) n.child[k] += static_cast<std::int32_t>(leafBase);
+					if (c == kEmptyChild) continue;
+					if (!(c & kLeafBit)) c += tlasBase;
+					else
+					{
+						const std::uint32_t top = (c >> kTopKindShift) & 3u;
+						c = leafRef(c, top == kTopTriangles ? base[GPU_HIT_TRIANGLE] : top == kTopInstance ? base[GPU_HIT_INSTANCE] : leafBase);
+					}
 				}
 				m.tlasWide.push_back(n);
 			}
 			for (Bvh4Node n : p.blasWide)
 			{
-				for (int k = 0; k < 4; k++)
+				for (std::uint32_t& c : n.child)
 				{
-					if (n.count[k] == 0) n.child[k] += static_cast<std::int32_t>(blasBase);
-					else if (n.count[k] != 255) n.child[k] += static_cast<std::int32_t>(meshTriBase);
+					if (c == kEmptyChild) continue;
+					c = (c & kLeafBit) ? leafRef(c, meshTriBase) : c - partTlas + blasBase;
 				}
 				m.blasWide.push_back(n);
 			}
@@ -1645,7 +1726,8 @@ namespace luzgpu
 			m.rects.insert(m.rects.end(), p.rects.begin(), p.rects.end());
 			for (GpuInstance in : p.instances)
 			{
-				in.blasRoot += static_cast<std::int32_t>(blasBase);
+				in.blasRoot += static_cast<std::int32_t>(blasBase) - static_cast<std::int32_t>(partTlas);
+				in.hittable += hittableBase;
 				in.triBase += static_cast<std::int32_t>(meshTriBase);
 				if (in.normalBase >= 0) in.normalBase += static_cast<std::int32_t>(normalSlotBase);
 				m.instances.push_back(in);
@@ -1695,6 +1777,9 @@ namespace luzgpu
 			m.blasStackBound = std::max(m.blasStackBound, p.blasStackBound);
 			m.triangleCount += p.triangleCount;
 		}
+		if (m.tlasWide.size() + m.blasWide.size() > kMaxNodes) throw std::runtime_error("Unsupported: more than 2^26 BVH nodes in a batch");
+		shiftNodes(m.blasWide, static_cast<std::uint32_t>(m.tlasWide.size()));
+		for (GpuInstance& in : m.instances) in.blasRoot += static_cast<std::int32_t>(m.tlasWide.size());
 		return (m);
 	}
 }

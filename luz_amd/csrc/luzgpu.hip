@@ -91,6 +91,20 @@ namespace luzgpu
 				check(hipMemcpyAsync(ptr, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice, stream), "hipMemcpyAsync");
 			}
 
+			// two vectors, one after the other
+			template <typename T>
+			void	upload(const std::vector<T>& a, const std::vector<T>& b, hipStream_t stream)
+			{
+				if (a.empty() && b.empty()) return;
+				reserve((a.size() + b.size()) * sizeof(T));
+				if (!a.empty()) check(hipMemcpyAsync(ptr, a.data(), a.size() * sizeof(T), hipMemcpyHostToDevice, stream), "hipMemcpyAsync");
+				if (!b.empty())
+				{
+					check(hipMemcpyAsync(static_cast<T*>(ptr) + a.size(), b.data(), b.size() * sizeof(T), hipMemcpyHostToDevice, stream),
+						"hipMemcpyAsync");
+				}
+			}
+
 			template <typename T> T*	as() const { return static_cast<T*>(ptr); }
 		};
 
@@ -633,14 +647,14 @@ namespace luzgpu
 	struct	GpuScene
 	{
 		PackedScene	host;
-		DeviceBuffer	tlas, blas, topTris, meshTris, meshNormals, tlasPrims, hittables, rects, instances, materials,
+		DeviceBuffer	nodes, topTris, meshTris, meshNormals, tlasPrims, hittables, rects, instances, materials,
 			lights, lightCdf, lightTriCdf, lightTriSlot, envPixels, envPdf, envCdf, envGuide, iesData, unbounded, spheres, cubeFaces, volumes, planes;
 		SceneView	view{};
 		luzgpu_scene_info	info{};
 
 		void	releaseDevice()
 		{
-			for (DeviceBuffer* b : {&tlas, &blas, &topTris, &meshTris, &meshNormals, &tlasPrims, &hittables, &rects, &instances,
+			for (DeviceBuffer* b : {&nodes, &topTris, &meshTris, &meshNormals, &tlasPrims, &hittables, &rects, &instances,
 				&materials, &lights, &lightCdf, &lightTriCdf, &lightTriSlot, &envPixels, &envPdf, &envCdf, &envGuide, &iesData, &unbounded, &spheres,
 				&cubeFaces, &volumes, &planes})
 			{
@@ -732,8 +746,7 @@ namespace luzgpu
 		{
 			PackedScene& h = g.host;
 			hipStream_t st = ctx->stream;
-			g.tlas.upload(h.tlasWide, st);
-			g.blas.upload(h.blasWide, st);
+			g.nodes.upload(h.tlasWide, h.blasWide, st);
 			g.topTris.upload(h.topTris, st);
 			g.meshTris.upload(h.meshTris, st);
 			g.meshNormals.upload(h.meshNormals, st);
@@ -758,8 +771,7 @@ namespace luzgpu
 			g.planes.upload(h.planes, st);
 			check(hipStreamSynchronize(st), "scene upload");
 			SceneView& v = g.view;
-			v.tlas = g.tlas.as<Bvh4Node>();
-			v.blas = g.blas.as<Bvh4Node>();
+			v.nodes = g.nodes.as<Bvh4Node>();
 			v.topTris = g.topTris.as<GpuTri>();
 			v.meshTris = g.meshTris.as<GpuTri>();
 			v.meshNormals = g.meshNormals.as<float>();
@@ -853,7 +865,7 @@ namespace luzgpu
 			t.shadowRefill = r.shadow_refill;
 			t.chunk = r.fetch_chunk;
 			t.ldsStack = static_cast<int>(r.lds_stack);
-			return t.resolved();
+			return t;
 		}
 
 		std::vector<std::uint64_t>	tuneKey(const std::vector<std::uint64_t>& serials, const std::vector<BatchJob>& jobs)
@@ -908,7 +920,7 @@ namespace luzgpu
 				trials++;
 				return static_cast<double>(ms);
 			};
-			WaveTuning best = WaveTuning{}.resolved();
+			WaveTuning best = WaveTuning{}.resolved(features);
 			const double defaultMs = timeOf(best);
 			double bestMs = defaultMs;
 			for (int sweep = 0; sweep < 2; sweep++)
@@ -919,7 +931,7 @@ namespace luzgpu
 						WaveTuning t = best;
 						set(t, v);
 						if (t == best) continue;
-						const double ms = timeOf(t.resolved());
+						const double ms = timeOf(t.resolved(features));
 						if (ms < bestMs)
 						{
 							bestMs = ms;
@@ -1543,7 +1555,7 @@ int	luzgpu_render(luzgpu_ctx* ctx, luzgpu_scene* scene, const luzgpu_settings* s
 		}
 		const std::uint32_t integrator = resolveIntegrator(settings ? settings->integrator : LUZGPU_INTEGRATOR_WAVEFRONT,
 			static_cast<std::uint64_t>(p.width) * p.height * p.sampleCount, "luzgpu_render");
-		WaveTuning tune = tuningOf(settings).resolved();
+		WaveTuning tune = tuningOf(settings).resolved(scene->gpu.host.features);
 		double tuneMs = 0.0;
 		if (settings && settings->autotune && integrator == LUZGPU_INTEGRATOR_WAVEFRONT)
 		{
@@ -1818,7 +1830,7 @@ int	luzgpu_render_denoised(luzgpu_ctx* ctx, luzgpu_scene* scene, const luzgpu_se
 		e0.record(st);
 		const std::uint32_t integrator = resolveIntegrator(settings ? settings->integrator : LUZGPU_INTEGRATOR_WAVEFRONT,
 			static_cast<std::uint64_t>(p.width) * p.height * p.sampleCount, "luzgpu_render_denoised");
-		const WaveTuning tune = tuningOf(settings).resolved();
+		const WaveTuning tune = tuningOf(settings).resolved(scene->gpu.host.features);
 		// samples [begin, begin + count) of `active` pixels (`list`, or all) into the statistics
 		auto renderRange = [&](std::uint32_t begin, std::uint32_t count, const std::uint32_t* list, std::uint32_t active, double* moments) {
 			if (integrator == LUZGPU_INTEGRATOR_WAVEFRONT)
@@ -2104,7 +2116,7 @@ int	luzgpu_render_batch(luzgpu_ctx* ctx, uint32_t n, luzgpu_scene* const* scenes
 		zero_doubles<<<blocks(sumTotal, 256), 256, 0, st>>>(ctx->batchSums.as<double>(), sumTotal);
 		zero_u64<<<1, 64, 0, st>>>(ctx->counters.as<unsigned long long>(), 8);
 		for (uint32_t i = 0; i < n; i++) jobs[i].sums = ctx->batchSums.as<double>() + sumOffset[i];
-		WaveTuning tune = tuningOf(settings).resolved();
+		WaveTuning tune = tuningOf(settings).resolved(ctx->batch->host.features);
 		double tuneMs = 0.0;
 		if (settings && settings[0].autotune && settings[0].integrator == LUZGPU_INTEGRATOR_WAVEFRONT)
 		{
