@@ -12,10 +12,9 @@
 //   MSE estimation, its and the bandwidth selection's cross-bilateral filtering (:834-936);
 //   per-pixel blend, then a final regression of the blend (:1074-1101).
 //
-// The regression solves a 12 x 12 weighted least-squares system per pixel. Two lanes own a
-// pixel, each half of its system in registers: they walk the window in the reference's
-// raster order, so every entry is summed in the reference's order (with a fused
-// multiply-add per term), and a second kernel solves each system by the reference's
+// The regression solves a 12 x 12 weighted least-squares system per pixel. The systems are
+// accumulated on the FP64 matrix unit, four window samples (in the reference's raster
+// order) to an instruction, and a second kernel solves each by the reference's
 // Gauss-Jordan elimination with partial pivoting.
 #pragma once
 
@@ -274,19 +273,15 @@ namespace luzgpu
 		for (int j = 0; j < 3; j++) out[j] = total <= 2.220446049250313e-16 ? image[3 * c + j] : acc[j] / total;
 	}
 
-	constexpr int	kNforTile = 16;						// pixels per tile side
-	constexpr int	kNforTilePixels = kNforTile * kNforTile;
+	constexpr int	kNforTileX = 16, kNforTileY = 8;	// pixels of a regression tile
+	constexpr int	kNforTilePixels = kNforTileX * kNforTileY;
+	constexpr int	kNforBlock = 512;					// 8 waves, one per tile row
 	constexpr int	kNforMaxPatchRadius = 8;
-	constexpr int	kNforChunk = 4;						// window displacements per pair of barriers
-	constexpr int	kNforHalfSlots = kNforSystem / 2;	// 57 system entries per half
-
-	// The two halves of a pixel's system, by rows of the upper triangle (each row's entries
-	// and its three right-hand sides): 39 matrix + 18 right-hand-side entries each.
-	__host__ __device__ constexpr int	nforHalfRow(int half, int i)
-	{
-		constexpr int rows[2][6] = {{0, 3, 4, 7, 8, 11}, {1, 2, 5, 6, 9, 10}};
-		return rows[half][i];
-	}
+	constexpr int	kNforDepth = 4;						// window samples (k) of one matrix instruction
+	constexpr int	kNforChunk = 8;						// window displacements per step, two per lane
+	constexpr int	kNforQuads = kNforTileX / 4;		// a wave's row in groups of 4 pixels
+	constexpr int	kNforWeightStride = kNforTilePixels + 4;	// doubles between a step's displacements: disjoint LDS banks
+	static_assert(kNforBlock == 64 * kNforTileY && 2 * kNforBlock == kNforTilePixels * kNforChunk, "a wave per row, two weights per lane");
 
 	// index of upper-triangle entry (row, col >= row) in the row-major packing
 	__host__ __device__ constexpr int	nforUpperIndex(int row, int col)
@@ -297,331 +292,446 @@ namespace luzgpu
 	// Dynamic LDS of nfor_accumulate, in doubles. Staged: the colours (three planes) and
 	// variances of the tile grown by the window and patch radii, and the 11 feature planes of
 	// the tile grown by the window radius, each slot holding the pixel of its clamped
-	// coordinate. Both forms: the patch terms and the weights of kNforChunk displacements.
+	// coordinate. Both forms: the patch terms and the weights of two steps each. Strides keep
+	// the doubles that lanes read together on disjoint banks: an operand reads four planes at
+	// once, up to 7 neighbours of each (planes 8 doubles apart modulo the LDS's 32), and half a
+	// wave reads the patch terms of two rows four apart (rows 4 doubles apart modulo 8).
 	struct	NforLdsLayout
 	{
-		int	colorWidth, featureWidth, apron;
+		int	colorWidth, colorHeight, featureWidth, featureHeight, apronX, apronY, apronStride;
+		std::uint32_t	colorStride, featureStride;	// doubles between planes
 		std::uint32_t	colors, variances, features, pairs, weights, doubles;
 	};
 
 	__host__ __device__ inline NforLdsLayout	nforLdsLayout(std::uint32_t regressionRadius, std::uint32_t patchRadius, bool staged)
 	{
 		NforLdsLayout L;
-		L.colorWidth = staged ? kNforTile + 2 * static_cast<int>(regressionRadius + patchRadius) : 0;
-		L.featureWidth = staged ? kNforTile + 2 * static_cast<int>(regressionRadius) : 0;
-		L.apron = kNforTile + 2 * static_cast<int>(patchRadius);
-		const std::uint32_t cc = static_cast<std::uint32_t>(L.colorWidth * L.colorWidth);
-		const std::uint32_t ff = static_cast<std::uint32_t>(L.featureWidth * L.featureWidth);
+		const int cr = 2 * static_cast<int>(regressionRadius + patchRadius), fr = 2 * static_cast<int>(regressionRadius);
+		L.colorWidth = staged ? kNforTileX + cr : 0;
+		L.colorHeight = staged ? kNforTileY + cr : 0;
+		L.featureWidth = staged ? kNforTileX + fr : 0;
+		L.featureHeight = staged ? kNforTileY + fr : 0;
+		L.apronX = kNforTileX + 2 * static_cast<int>(patchRadius);
+		L.apronY = kNforTileY + 2 * static_cast<int>(patchRadius);
+		L.apronStride = L.apronX + (12 - L.apronX % 8) % 8;
+		const std::uint32_t cc = static_cast<std::uint32_t>(L.colorWidth * L.colorHeight);
+		const std::uint32_t ff = static_cast<std::uint32_t>(L.featureWidth * L.featureHeight);
+		L.colorStride = staged ? cc + (40u - cc % 32u) % 32u : 0u;
+		L.featureStride = staged ? ff + (40u - ff % 32u) % 32u : 0u;
 		L.colors = 0;
-		L.variances = 3 * cc;
+		L.variances = 3 * L.colorStride;
 		L.features = L.variances + cc;
-		L.pairs = L.features + kNforFeatures * ff;
-		L.weights = L.pairs + kNforChunk * static_cast<std::uint32_t>(L.apron * L.apron);
-		L.doubles = L.weights + kNforChunk * kNforTilePixels;
+		L.pairs = L.features + kNforFeatures * L.featureStride;
+		L.weights = L.pairs + 2 * kNforChunk * static_cast<std::uint32_t>(L.apronStride * L.apronY);
+		L.doubles = L.weights + 2 * kNforChunk * kNforWeightStride;
 		return L;
 	}
 
-	// a half of a fresh system: the ridge 1e-4 on the diagonal, zero elsewhere
-	template <int Half>
-	__device__ __forceinline__ void	nforClearHalf(double (&acc)[kNforHalfSlots])
+	// exp(-x) for x >= 0 (NaN stays NaN): 2^k e^r with k the nearest integer to -x log2 e, r the
+	// rest (ln 2 in two parts), e^r its Taylor sum to r^13 (|r| <= ln 2 / 2: the first term left
+	// out is 4e-18 of it). Within 1 ulp.
+	__device__ __forceinline__ double	nforExpNegative(double x)
 	{
-		int e = 0;
-		#pragma unroll
-		for (int i = 0; i < 6; i++)
-		{
-			const int row = nforHalfRow(Half, i);
-			#pragma unroll
-			for (int col = row; col < kNforBasis; col++) acc[e++] = col == row ? 1e-4 : 0.0;
-			acc[e++] = 0.0;
-			acc[e++] = 0.0;
-			acc[e++] = 0.0;
-		}
+		x = x > 1000.0 ? 1000.0 : x;	// 2^-1443: zero already
+		const double k = rint(x * -1.4426950408889634);
+		double r = fma(k, -0.69314718055994529, -x);
+		r = fma(k, -2.3190468138462996e-17, r);
+		// two half sums of the even and odd powers: two chains in flight
+		const double r2 = r * r;
+		double even = fma(r2, 2.0876756987868099e-09, 2.7557319223985893e-07);		// 1/12!, 1/10!
+		double odd = fma(r2, 1.6059043836821613e-10, 2.5052108385441720e-08);		// 1/13!, 1/11!
+		even = fma(r2, even, 2.4801587301587302e-05);
+		odd = fma(r2, odd, 2.7557319223985893e-06);
+		even = fma(r2, even, 1.3888888888888889e-03);
+		odd = fma(r2, odd, 1.9841269841269841e-04);
+		even = fma(r2, even, 4.1666666666666664e-02);
+		odd = fma(r2, odd, 8.3333333333333332e-03);
+		even = fma(r2, even, 0.5);
+		odd = fma(r2, odd, 1.6666666666666666e-01);
+		// 1 + (r + r^2 (even + r odd))
+		const double tail = fma(r2, fma(r, odd, even), r);
+		return ldexp(1.0 + tail, static_cast<int>(k));
 	}
 
-	// addRegressionSample (NFOR.cpp:582-600) for one half of the system. Each entry adds
-	// (w * basis[row]) * basis[col] with one fused multiply-add: one rounding per sample where
-	// the reference rounds the product and the sum separately, so the systems differ from
-	// the reference's by FP64 rounding only (the same entries, summed in the same order).
-	template <int Half>
-	__device__ __forceinline__ void	nforAddSample(double (&acc)[kNforHalfSlots], const double (&basis)[kNforBasis], double w, double cr,
-		double cg, double cb)
-	{
-		#pragma clang fp contract(off)
-		int e = 0;
-		#pragma unroll
-		for (int i = 0; i < 6; i++)
-		{
-			const int row = nforHalfRow(Half, i);
-			const double wb = w * basis[row];
-			#pragma unroll
-			for (int col = row; col < kNforBasis; col++)
-			{
-				acc[e] = fma(wb, basis[col], acc[e]);
-				e++;
-			}
-			acc[e] = fma(wb, cr, acc[e]);
-			acc[e + 1] = fma(wb, cg, acc[e + 1]);
-			acc[e + 2] = fma(wb, cb, acc[e + 2]);
-			e += 3;
-		}
-	}
-
-	// The half's entries into the pixel's system (slot-major: entry k of pixel p at k * n + p;
-	// entries 0..77 the upper triangle, 78 + 3 * row + channel the right-hand sides).
-	template <int Half>
-	__device__ __forceinline__ void	nforStoreHalf(const double (&acc)[kNforHalfSlots], double* __restrict__ system, size_t n, size_t pixel)
-	{
-		int e = 0;
-		#pragma unroll
-		for (int i = 0; i < 6; i++)
-		{
-			const int row = nforHalfRow(Half, i);
-			#pragma unroll
-			for (int col = row; col < kNforBasis; col++) system[static_cast<size_t>(nforUpperIndex(row, col)) * n + pixel] = acc[e++];
-			#pragma unroll
-			for (int j = 0; j < 3; j++) system[static_cast<size_t>(kNforUpper + 3 * row + j) * n + pixel] = acc[e++];
-		}
-	}
-
-	// regressionPass (NFOR.cpp:679-737), accumulation: a 16 x 16 tile per block of 512 lanes,
-	// two per pixel, each owning half of the pixel's 12 x 12 system and its right-hand sides
-	// (nforHalfRow). The halves are whole waves (lanes 0-255 and 256-511), so every branch on
-	// the half is wave-uniform and every register index static; both halves form the pixel's
-	// weights. The window is visited in the reference's raster order, so every entry is summed
-	// in the reference's order; nfor_solve then solves the systems.
+	// regressionPass (NFOR.cpp:679-737), accumulation: each pixel's 12 x 12 weighted normal
+	// matrix and its three right-hand sides, over the samples of its window, at one bandwidth
+	// or at two (the systems then differ by the weights only). nfor_solve solves the systems.
 	//
-	// Patch distances: for a window displacement d, the term of patch offset o between pixel
-	// p and its sample p + d is D(p + o, p + o + d) (patchDistance, NFOR.cpp:240-311), which
-	// depends on p + o only. For kNforChunk displacements at a time the block evaluates
-	// D(q, q + d) once for every q of its tile and apron into LDS, the two halves form the
-	// chunk's weights between them (two displacements each) into LDS, and both then add the
-	// chunk's samples; three barriers fence the steps. Lanes whose patch or sample would be
-	// clamped at the image border take the direct, clamped form.
+	// The sums are a contraction over the window: basis^T (w * [basis | colour]). It runs on
+	// the FP64 matrix instruction of four independent 4 x 4 x 4 products: a block is one
+	// pixel, k four window samples, and the 12 x 15 system is nine 4 x 4 products (the upper
+	// triangle's six and the colours' three), accumulated in two VGPRs each. Lane l holds row
+	// or column l % 4 of block (l / 4) % 4 for sample l / 16, so an operand is one feature
+	// difference per lane, and a wave's row of 16 pixels at two bandwidths takes 144
+	// accumulator VGPRs.
+	//
+	// A 16 x 8 tile per block of 8 waves. Patch distances: for a window displacement d, the
+	// term of patch offset o between pixel p and its sample p + d is D(p + o, p + o + d)
+	// (patchDistance, NFOR.cpp:240-311), which depends on p + o only, so a step's terms are
+	// evaluated once for every pixel of the tile and its apron into LDS. The stages of a step
+	// of 8 displacements (terms, then weights, then products) run on three consecutive steps
+	// at once, with one barrier a step; the two waves of a SIMD take them in opposite order.
+	// Lanes whose sample would lie off the image take the border sample's own terms. `Two`: bandwidth 1 and half of it; the second weight is the first's fourth
+	// power (the host takes two passes where the variance floor breaks that ratio).
 	//
 	// Staged: the block first copies every colour, variance and feature its window reads into
-	// LDS, so the per-step reads are LDS reads (radius 9, patch radius 1: 158 KiB); the
-	// unstaged form reads them from global memory, for windows too wide for LDS.
-	template <bool Staged>
-	__global__ __launch_bounds__(2 * kNforTilePixels) void	nfor_accumulate(const double* __restrict__ image,
+	// LDS (radius 9, patch radius 1: 152 KiB); the unstaged form reads them from global
+	// memory, for windows too wide for LDS.
+	//
+	// Bound by FP64 issue, which matrix and vector instructions share: at 1280 x 720, radius 9,
+	// 5.5 ms for one bandwidth and 7.7 for two, of which the products take 2.4 and 3.8 (1.2 and
+	// 2.4 at the matrix unit's rate), the weights 1.6, the terms 1.5, staging and stores 0.6 and
+	// 0.9. With each lane owning half a pixel's system in vector FMAs, 14 LDS reads a sample and
+	// three barriers per 4 displacements, one bandwidth took 8.8 ms. Border lanes that read
+	// their patches from global memory cost 1.8 ms of the weights; 16 waves of half the pixels
+	// each were slower (spills).
+	template <bool Staged, bool Two>
+	__global__ __launch_bounds__(kNforBlock, 2) void	nfor_accumulate(const double* __restrict__ image,
 		const double* __restrict__ features, const double* __restrict__ variance, double* __restrict__ system, NforParams P,
-		double bandwidth)
+		double bandwidth, std::uint32_t firstRow, std::uint32_t rows)
 	{
 		#pragma clang fp contract(off)
 		extern __shared__ double lds[];
+		constexpr int Bandwidths = Two ? 2 : 1;
 		const NforLdsLayout L = nforLdsLayout(P.regressionRadius, P.patchRadius, Staged);
 		double* const colors = lds + L.colors;
 		double* const vars = lds + L.variances;
 		double* const feats = lds + L.features;
 		double* const pairs = lds + L.pairs;
 		double* const weights = lds + L.weights;
-		const int cw = L.colorWidth, fw = L.featureWidth, apron = L.apron;
-		const int cc = cw * cw, ff = fw * fw, aa = apron * apron;
-		const int lane = static_cast<int>(threadIdx.x) % kNforTilePixels;
-		const int half = static_cast<int>(threadIdx.x) / kNforTilePixels;	// wave-uniform
-		// each 32-lane half of a wave takes tile rows h and h + 8: 8 rows of the staged feature
-		// (34 wide) and patch-term (18 wide) planes apart, their 16 doubles fall on disjoint
-		// LDS banks
-		const int tx = lane % kNforTile, ty = lane / 32 + ((lane % 32) >= kNforTile ? 8 : 0);
-		const std::uint32_t tilesX = (P.width + kNforTile - 1) / kNforTile;
-		const long long x0 = static_cast<long long>(blockIdx.x % tilesX) * kNforTile;
-		const long long y0 = static_cast<long long>(blockIdx.x / tilesX) * kNforTile;
-		const std::uint32_t x = static_cast<std::uint32_t>(x0) + tx, y = static_cast<std::uint32_t>(y0) + ty;
-		const bool active = x < P.width && y < P.height;
-		const std::uint32_t c = active ? y * P.width + x : 0u;
-		const long long r = P.regressionRadius, pr = P.patchRadius;
-		const long long cx0 = x0 - r - pr, cy0 = y0 - r - pr;	// staged colour region origin
-		const long long fx0 = x0 - r, fy0 = y0 - r;				// staged feature region origin
+		const int cw = L.colorWidth, fw = L.featureWidth, ax = L.apronX, as = L.apronStride;
+		const int cells = cw * L.colorHeight, ff = fw * L.featureHeight, aa = ax * L.apronY, termsSize = as * L.apronY;
+		const int cc = static_cast<int>(L.colorStride), fs = static_cast<int>(L.featureStride);
+		const int iw = static_cast<int>(P.width), ih = static_cast<int>(P.height);
+		const int ir = static_cast<int>(P.regressionRadius), ipr = static_cast<int>(P.patchRadius);
+		const int tilesX = (iw + kNforTileX - 1) / kNforTileX;
+		const int x0 = static_cast<int>(blockIdx.x % static_cast<unsigned>(tilesX)) * kNforTileX;
+		const int y0 = static_cast<int>(firstRow) + static_cast<int>(blockIdx.x / static_cast<unsigned>(tilesX)) * kNforTileY;
+		const int thread = static_cast<int>(threadIdx.x);
+		auto pixelAt = [&](int x, int y) { return static_cast<size_t>(nforClampInt(y, ih)) * P.width + static_cast<size_t>(nforClampInt(x, iw)); };
 		if constexpr (Staged)
 		{
-			for (int i = static_cast<int>(threadIdx.x); i < cc; i += 2 * kNforTilePixels)
+			for (int i = thread; i < cells; i += kNforBlock)
 			{
-				const std::uint32_t g = nforClamp(cy0 + i / cw, P.height) * P.width + nforClamp(cx0 + i % cw, P.width);
-				colors[i] = image[3 * static_cast<size_t>(g)];
-				colors[cc + i] = image[3 * static_cast<size_t>(g) + 1];
-				colors[2 * cc + i] = image[3 * static_cast<size_t>(g) + 2];
+				const size_t g = pixelAt(x0 - ir - ipr + i % cw, y0 - ir - ipr + i / cw);
+				colors[i] = image[3 * g];
+				colors[cc + i] = image[3 * g + 1];
+				colors[2 * cc + i] = image[3 * g + 2];
 				vars[i] = variance[g];
 			}
-			for (int i = static_cast<int>(threadIdx.x); i < ff; i += 2 * kNforTilePixels)
+			for (int i = thread; i < ff; i += kNforBlock)
 			{
-				const std::uint32_t g = nforClamp(fy0 + i / fw, P.height) * P.width + nforClamp(fx0 + i % fw, P.width);
+				const size_t g = pixelAt(x0 - ir + i % fw, y0 - ir + i / fw);
 				#pragma unroll
-				for (int j = 0; j < kNforFeatures; j++) feats[j * ff + i] = features[kNforFeatures * static_cast<size_t>(g) + j];
+				for (int j = 0; j < kNforFeatures; j++) feats[j * fs + i] = features[kNforFeatures * g + j];
 			}
 			__syncthreads();
 		}
-		const double patchTerms = static_cast<double>((2 * pr + 1) * (2 * pr + 1));
-		const bool patchInside = active && static_cast<long long>(x) >= pr && static_cast<long long>(y) >= pr
-			&& static_cast<long long>(x) + pr < static_cast<long long>(P.width) && static_cast<long long>(y) + pr < static_cast<long long>(P.height);
-		double acc[kNforHalfSlots];
-		if (half == 0) nforClearHalf<0>(acc);
-		else nforClearHalf<1>(acc);
-		// 32-bit index arithmetic from here on (the image and window sizes are far below 2^31)
-		const int ix = static_cast<int>(x), iy = static_cast<int>(y);
-		const int iw = static_cast<int>(P.width), ih = static_cast<int>(P.height);
-		const int ir = static_cast<int>(r), ipr = static_cast<int>(pr);
-		const int fBase = (ty + ir) * fw + (tx + ir);				// the pixel's staged feature slot
-		const int cBase = (ty + ir + ipr) * cw + (tx + ir + ipr);	// the pixel's staged colour slot
-		const double bw2 = fmax(P.minVariance, bandwidth * bandwidth);
 		const int side = 2 * ir + 1;
-		const int steps = side * side;
-		// the chunk's displacements, raster order: (stepY[k], stepX[k]) = (oy, ox)
-		int stepY[kNforChunk], stepX[kNforChunk];
-		// one window sample: its weight w, its basis (1, features - the pixel's) and colour
-		auto sampleAt = [&]<int Half>(int k, double w) {
-			const int oy = stepY[k], ox = stepX[k];
-			double basis[kNforBasis];
-			double cr, cg, cb;
-			basis[0] = 1.0;
+		const int samples = side * side;
+		const int steps = (samples + kNforChunk - 1) / kNforChunk;
+		// a window sample's displacement, walked in raster order; past the last sample it is the
+		// pixel itself (with weight 0)
+		struct	Walk
+		{
+			int	s, x, y;
+		};
+		auto walkFrom = [&](int s0) { return Walk{s0, s0 % side - ir, s0 / side - ir}; };
+		auto advance = [&](Walk& w) {
+			w.s += kNforDepth;
+			w.x += kNforDepth % side;
+			w.y += kNforDepth / side;
+			const bool wrap = w.x > ir;
+			w.x -= wrap ? side : 0;
+			w.y += wrap ? 1 : 0;
+		};
+
+		// Stages that form terms and weights: two waves have displacements kk and kk + 4 of the
+		// step, one pixel per lane
+		const int kk = __builtin_amdgcn_readfirstlane(thread / kNforTilePixels);
+		const int kLane = thread % kNforTilePixels;
+		// a patch term of two pixels: slots of the staged colours, or pixels
+		auto term = [&](auto a, auto b) {
+			double dr, dg, db, lv;
 			if constexpr (Staged)
 			{
-				const int fi = fBase + oy * fw + ox;
-				const int ci = cBase + oy * cw + ox;
-				#pragma unroll
-				for (int j = 0; j < kNforFeatures; j++) basis[j + 1] = feats[j * ff + fi] - feats[j * ff + fBase];
-				cr = colors[ci];
-				cg = colors[cc + ci];
-				cb = colors[2 * cc + ci];
+				dr = colors[a] - colors[b];
+				dg = colors[cc + a] - colors[cc + b];
+				db = colors[2 * cc + a] - colors[2 * cc + b];
+				lv = vars[a] + vars[b] + P.minVariance;
 			}
 			else
 			{
-				const size_t sp = static_cast<size_t>(nforClampInt(iy + oy, ih)) * P.width + nforClampInt(ix + ox, iw);
-				#pragma unroll
-				for (int j = 0; j < kNforFeatures; j++)
-				{
-					basis[j + 1] = features[kNforFeatures * sp + j] - features[kNforFeatures * static_cast<size_t>(c) + j];
-				}
-				cr = image[3 * sp];
-				cg = image[3 * sp + 1];
-				cb = image[3 * sp + 2];
+				dr = image[3 * a] - image[3 * b];
+				dg = image[3 * a + 1] - image[3 * b + 1];
+				db = image[3 * a + 2] - image[3 * b + 2];
+				lv = variance[a] + variance[b] + P.minVariance;
 			}
-			nforAddSample<Half>(acc, basis, w, cr, cg, cb);
+			return ((dr * dr) + (dg * dg) + (db * db)) / (3.0 * lv);
 		};
-		// colorWeightFromDistance (NFOR.cpp:313-318) of one window displacement
-		auto weightAt = [&](int k) {
-			const int ux = ix + stepX[k], uy = iy + stepY[k];
+		// patch terms D(q, q + d) of a step over the tile and its apron, coordinates clamped
+		auto pairTerm = [&](int j, const Walk& w, int slot) {
+			const int ox = w.s < samples ? w.x : 0, oy = w.s < samples ? w.y : 0;
+			const int jy = j / ax, jx = j - jy * ax;
+			if constexpr (Staged)
+			{
+				const int a = (jy + ir) * cw + (jx + ir);	// q = tile origin - patch radius + (jx, jy)
+				pairs[slot + jy * as + jx] = term(a, a + oy * cw + ox);
+			}
+			else pairs[slot + jy * as + jx] = term(pixelAt(x0 - ipr + jx, y0 - ipr + jy), pixelAt(x0 - ipr + jx + ox, y0 - ipr + jy + oy));
+		};
+		auto formPairs = [&](int t, const Walk& w0, const Walk& w1) {
+			const int slot = ((t & 1) * kNforChunk + kk) * termsSize;
+			for (int j = kLane; j < aa; j += kNforTilePixels)
+			{
+				pairTerm(j, w0, slot);
+				pairTerm(j, w1, slot + kNforDepth * termsSize);
+			}
+		};
+
+		// weights of a step (colorWeightFromDistance, NFOR.cpp:313-318), at bandwidth 1
+		const int wtx = kLane % kNforTileX, wty = (kLane / kNforTileX % 2) * 4 + kLane / (2 * kNforTileX);
+		const int wPixel = wty * kNforTileX + wtx;
+		const int wx = x0 + wtx, wy = y0 + wty;
+		const bool wActive = wx < iw && wy < ih;
+		const double patchTerms = static_cast<double>((2 * ipr + 1) * (2 * ipr + 1));
+		const double scale = patchTerms * fmax(P.minVariance, bandwidth * bandwidth);
+		const double inverseScale = 1.0 / scale, farthest = 1000.0 * scale;
+		auto patchSum = [&](int t, int k, const Walk& at) {
+			const int ux = at.s < samples ? wx + at.x : wx, uy = at.s < samples ? wy + at.y : wy;
 			const int sx = nforClampInt(ux, iw), sy = nforClampInt(uy, ih);
 			double distance = 0.0;
-			if (sx == ix && sy == iy)
+			if (!wActive || (sx == wx && sy == wy))
 			{
 				distance = 0.0;
 			}
-			else if (patchInside && ux == sx && uy == sy && ux >= ipr && uy >= ipr && ux + ipr < iw && uy + ipr < ih)
+			else if (ux == sx && uy == sy)
 			{
-				const double* terms = pairs + k * aa;
-				if (pr == 1)
+				// patches may overhang the image: a term's two pixels are clamped one by one, as here
+				const double* terms = pairs + ((t & 1) * kNforChunk + k) * termsSize;
+				if (ipr == 1)
 				{
 					// the common 3 x 3 patch: the nine reads issued together, then summed in order
-					double t[9];
+					double v[9];
 					#pragma unroll
-					for (int i = 0; i < 9; i++) t[i] = terms[(ty + i / 3) * apron + (tx + i % 3)];
+					for (int i = 0; i < 9; i++) v[i] = terms[(wty + i / 3) * as + (wtx + i % 3)];
 					#pragma unroll
-					for (int i = 0; i < 9; i++) distance += t[i];
+					for (int i = 0; i < 9; i++) distance += v[i];
 				}
 				else
 				{
-					for (long long py = -pr; py <= pr; py++)
+					for (int py = 0; py <= 2 * ipr; py++)
 					{
-						for (long long px = -pr; px <= pr; px++)
-						{
-							distance += terms[(ty + pr + py) * apron + (tx + pr + px)];
-						}
+						for (int px = 0; px <= 2 * ipr; px++) distance += terms[(wty + py) * as + (wtx + px)];
 					}
 				}
-				distance = distance / patchTerms;
 			}
 			else
 			{
-				distance = nforPatchDistance(image, variance, P, x, y, static_cast<std::uint32_t>(sx), static_cast<std::uint32_t>(sy),
-					P.patchRadius);
-			}
-			return exp(-distance / bw2);
-		};
-		int nextY = -ir, nextX = -ir;
-		for (int base = 0; base < steps; base += kNforChunk)
-		{
-			const int count = min(kNforChunk, steps - base);
-			#pragma unroll
-			for (int k = 0; k < kNforChunk; k++)
-			{
-				stepY[k] = nextY;
-				stepX[k] = nextX;
-				if (k < count && ++nextX > ir)
+				// the window overhangs: the sample is a pixel of the border, with its own patch
+				for (int py = -ipr; py <= ipr; py++)
 				{
-					nextX = -ir;
-					nextY++;
+					for (int px = -ipr; px <= ipr; px++)
+					{
+						if constexpr (Staged)
+						{
+							const int left = x0 - ir - ipr, top = y0 - ir - ipr;
+							distance += term((nforClampInt(wy + py, ih) - top) * cw + nforClampInt(wx + px, iw) - left,
+								(nforClampInt(sy + py, ih) - top) * cw + nforClampInt(sx + px, iw) - left);
+						}
+						else distance += term(pixelAt(wx + px, wy + py), pixelAt(sx + px, sy + py));
+					}
 				}
 			}
-			// D(q, q + d) over the tile and its apron for the chunk's displacements (entries off
-			// the image are clamped reads whose values no lane uses)
-			for (int i = static_cast<int>(threadIdx.x); i < count * aa; i += 2 * kNforTilePixels)
+			return distance;
+		};
+		// exp(-distance / scale); the quotient by the reciprocal and one correction (the nearest
+		// double, as a division gives it)
+		auto weightOf = [&](double distance) {
+			distance = distance > farthest ? farthest : distance;
+			const double q = distance * inverseScale;
+			return nforExpNegative(fma(fma(-q, scale, distance), inverseScale, q));
+		};
+		auto formWeights = [&](int t, const Walk& at0, const Walk& at1) {
+			const double d0 = patchSum(t, kk, at0), d1 = patchSum(t, kk + kNforDepth, at1);
+			const double e0 = weightOf(d0), e1 = weightOf(d1);
+			double* out = weights + ((t & 1) * kNforChunk + kk) * kNforWeightStride + wPixel;
+			out[0] = wActive && at0.s < samples ? e0 : 0.0;
+			out[kNforDepth * kNforWeightStride] = wActive && at1.s < samples ? e1 : 0.0;
+		};
+
+		// products of step t
+		const int wave = __builtin_amdgcn_readfirstlane(thread / 64);
+		const int lane = thread % 64;
+		const int li = lane % 4, lb = (lane / 4) % 4, lk = lane / 16;
+		// basis entry 4 m + li is 1 for entry 0, else feature 4 m + li - 1 less the pixel's own
+		const int plane0 = li > 0 ? li - 1 : 0, plane1 = 3 + li, colorPlane = li < 3 ? li : 2;
+		const int fBase = (wave + ir) * fw + (lb + ir);
+		const int cBase = (wave + ir + ipr) * cw + (lb + ir + ipr);
+		double own[kNforQuads][3];
+		#pragma unroll
+		for (int q = 0; q < kNforQuads; q++)
+		{
+			if constexpr (Staged)
 			{
-				const int k = i / aa, j = i % aa;
-				const int oy = stepY[k], ox = stepX[k];
-				const int jx = j % apron, jy = j / apron;
+				own[q][0] = feats[plane0 * fs + fBase + 4 * q];
+				own[q][1] = feats[plane1 * fs + fBase + 4 * q];
+				own[q][2] = feats[(plane1 + 4) * fs + fBase + 4 * q];
+			}
+			else
+			{
+				const double* f = features + kNforFeatures * pixelAt(x0 + 4 * q + lb, y0 + wave);
+				own[q][0] = f[plane0];
+				own[q][1] = f[plane1];
+				own[q][2] = f[plane1 + 4];
+			}
+		}
+		// [bandwidth][quad]: products 00 01 02 11 12 22 of basis quarters, then 0 1 2 by colour;
+		// a fresh system has the ridge 1e-4 on its diagonal
+		double acc[Bandwidths][kNforQuads][9];
+		#pragma unroll
+		for (int b = 0; b < Bandwidths; b++)
+		{
+			#pragma unroll
+			for (int q = 0; q < kNforQuads; q++)
+			{
+				#pragma unroll
+				for (int e = 0; e < 9; e++) acc[b][q][e] = (e == 0 || e == 3 || e == 5) && lk == li ? 1e-4 : 0.0;
+			}
+		}
+		auto multiply = [&](int t, int g, const Walk& at) {
+			const int ox = at.s < samples ? at.x : 0, oy = at.s < samples ? at.y : 0;
+			const int fOff = oy * fw + ox, cOff = oy * cw + ox;
+			const double* f0 = feats + plane0 * fs + fBase + fOff;
+			const double* f1 = feats + plane1 * fs + fBase + fOff;
+			const double* col = colors + colorPlane * cc + cBase + cOff;
+			const double* w = weights + ((t & 1) * kNforChunk + g * kNforDepth + lk) * kNforWeightStride + wave * kNforTileX + lb;
+			#pragma unroll
+			for (int q = 0; q < kNforQuads; q++)
+			{
+				double v0, v1, v2, c;
 				if constexpr (Staged)
 				{
-					const int a = (jy + ir) * cw + (jx + ir);	// q = tile origin - pr + (jx, jy)
-					const int b = a + oy * cw + ox;
-					const double dr = colors[a] - colors[b], dg = colors[cc + a] - colors[cc + b], db = colors[2 * cc + a] - colors[2 * cc + b];
-					pairs[i] = (((dr * dr) + (dg * dg) + (db * db)) / 3.0) / (vars[a] + vars[b] + P.minVariance);
+					v0 = f0[4 * q];
+					v1 = f1[4 * q];
+					v2 = f1[4 * fs + 4 * q];
+					c = col[4 * q];
 				}
 				else
 				{
-					const long long qx = x0 - pr + jx, qy = y0 - pr + jy;
-					const std::uint32_t qa = nforClamp(qy, P.height) * P.width + nforClamp(qx, P.width);
-					const std::uint32_t qb = nforClamp(qy + oy, P.height) * P.width + nforClamp(qx + ox, P.width);
-					pairs[i] = nforDist2(image + 3 * static_cast<size_t>(qa), image + 3 * static_cast<size_t>(qb))
-						/ (variance[qa] + variance[qb] + P.minVariance);
+					const size_t at0 = pixelAt(x0 + 4 * q + lb + ox, y0 + wave + oy);
+					const double* f = features + kNforFeatures * at0;
+					v0 = f[plane0];
+					v1 = f[plane1];
+					v2 = f[plane1 + 4];
+					c = image[3 * at0 + colorPlane];
+				}
+				const double d0 = v0 - own[q][0], b1 = v1 - own[q][1], b2 = v2 - own[q][2];
+				const double b0 = li == 0 ? 1.0 : d0;
+				double wk = w[4 * q];
+				#pragma unroll
+				for (int k = 0; k < Bandwidths; k++)
+				{
+					if (k == 1)
+					{
+						wk = wk * wk;
+						wk = wk * wk;
+					}
+					const double a0 = wk * b0, a1 = wk * b1, a2 = wk * b2;
+					double (&d)[9] = acc[k][q];
+					d[0] = __builtin_amdgcn_mfma_f64_4x4x4f64(a0, b0, d[0], 0, 0, 0);
+					d[1] = __builtin_amdgcn_mfma_f64_4x4x4f64(a0, b1, d[1], 0, 0, 0);
+					d[2] = __builtin_amdgcn_mfma_f64_4x4x4f64(a0, b2, d[2], 0, 0, 0);
+					d[3] = __builtin_amdgcn_mfma_f64_4x4x4f64(a1, b1, d[3], 0, 0, 0);
+					d[4] = __builtin_amdgcn_mfma_f64_4x4x4f64(a1, b2, d[4], 0, 0, 0);
+					d[5] = __builtin_amdgcn_mfma_f64_4x4x4f64(a2, b2, d[5], 0, 0, 0);
+					d[6] = __builtin_amdgcn_mfma_f64_4x4x4f64(a0, c, d[6], 0, 0, 0);
+					d[7] = __builtin_amdgcn_mfma_f64_4x4x4f64(a1, c, d[7], 0, 0, 0);
+					d[8] = __builtin_amdgcn_mfma_f64_4x4x4f64(a2, c, d[8], 0, 0, 0);
 				}
 			}
-			__syncthreads();
-			// the halves split the chunk's weights (steps k = half, half + 2), then both add
-			// every sample of the chunk
-			if (active)
+		};
+
+		Walk walk0 = walkFrom(kk), walk1 = walkFrom(kk + kNforDepth), productWalk = walkFrom(lk);
+		auto nextStep = [&]() {
+			advance(walk0);
+			advance(walk0);
+			advance(walk1);
+			advance(walk1);
+		};
+		auto products = [&](int t) {
+			#pragma unroll
+			for (int g = 0; g < kNforChunk / kNforDepth; g++)
 			{
-				if (count == kNforChunk)
-				{
-					// two independent exp chains in flight
-					const double w0 = weightAt(half), w1 = weightAt(half + 2);
-					weights[half * kNforTilePixels + lane] = w0;
-					weights[(half + 2) * kNforTilePixels + lane] = w1;
-				}
-				else
-				{
-					for (int k = half; k < count; k += 2) weights[k * kNforTilePixels + lane] = weightAt(k);
-				}
+				multiply(t, g, productWalk);
+				advance(productWalk);
 			}
-			__syncthreads();
-			if (active)
-			{
-				if (half == 0)
-				{
-					for (int k = 0; k < count; k++) sampleAt.template operator()<0>(k, weights[k * kNforTilePixels + lane]);
-				}
-				else
-				{
-					for (int k = 0; k < count; k++) sampleAt.template operator()<1>(k, weights[k * kNforTilePixels + lane]);
-				}
-			}
+		};
+		formPairs(0, walk0, walk1);
+		__syncthreads();
+		formWeights(0, walk0, walk1);
+		nextStep();
+		if (steps > 1) formPairs(1, walk0, walk1);
+		__syncthreads();
+		const bool first = wave < 4;
+		for (int t = 0; t < steps; t++)
+		{
+			if (first) products(t);
+			if (t + 1 < steps) formWeights(t + 1, walk0, walk1);
+			nextStep();
+			if (t + 2 < steps) formPairs(t + 2, walk0, walk1);
+			if (!first) products(t);
 			__syncthreads();
 		}
-		if (!active) return;
-		const size_t n = static_cast<size_t>(P.width) * P.height;
-		if (half == 0) nforStoreHalf<0>(acc, system, n, c);
-		else nforStoreHalf<1>(acc, system, n, c);
+
+		// the systems, slot-major: entry k of pixel p of the band at k * n + p; entries 0..77 the
+		// upper triangle, 78 + 3 * row + channel the right-hand sides. A product's row is held
+		// by lane / 16, its column by lane % 4.
+		const int y = y0 + wave;
+		if (y >= ih || y >= static_cast<int>(firstRow + rows)) return;
+		const size_t n = static_cast<size_t>(P.width) * rows;
+		#pragma unroll
+		for (int b = 0; b < Bandwidths; b++)
+		{
+			#pragma unroll
+			for (int q = 0; q < kNforQuads; q++)
+			{
+				const int x = x0 + 4 * q + lb;
+				if (x >= iw) continue;
+				double* out = system + static_cast<size_t>(b) * kNforSystem * n + static_cast<size_t>(y - static_cast<int>(firstRow)) * P.width + x;
+				int e = 0;
+				#pragma unroll
+				for (int m = 0; m < 3; m++)
+				{
+					#pragma unroll
+					for (int c = m; c < 3; c++)
+					{
+						const int row = 4 * m + lk, col = 4 * c + li;
+						if (row <= col) out[static_cast<size_t>(nforUpperIndex(row, col)) * n] = acc[b][q][e];
+						e++;
+					}
+				}
+				#pragma unroll
+				for (int m = 0; m < 3; m++)
+				{
+					if (li < 3) out[static_cast<size_t>(kNforUpper + 3 * (4 * m + lk) + li) * n] = acc[b][q][6 + m];
+				}
+			}
+		}
 	}
 
 	// completeRegressionMatrix (NFOR.cpp:628-637), then solveLinearSystemRGB (:466-516): the
-	// reference's Gauss-Jordan elimination with partial pivoting on each pixel's system from
-	// nfor_accumulate; a singular system takes weightedAverageFallback.
+	// reference's Gauss-Jordan elimination with partial pivoting on each system from
+	// nfor_accumulate (the pixels of `rows` image rows from firstRow); a singular system takes
+	// weightedAverageFallback.
 	__global__ __launch_bounds__(256) void	nfor_solve(const double* __restrict__ system, const double* __restrict__ image,
-		const double* __restrict__ variance, double* __restrict__ out, NforParams P)
+		const double* __restrict__ variance, double* __restrict__ out, NforParams P, std::uint32_t firstRow, std::uint32_t rows)
 	{
 		#pragma clang fp contract(off)
-		const size_t n = static_cast<size_t>(P.width) * P.height;
+		const size_t n = static_cast<size_t>(P.width) * rows;
 		const size_t c = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
 		if (c >= n) return;
-		const std::uint32_t x = static_cast<std::uint32_t>(c % P.width), y = static_cast<std::uint32_t>(c / P.width);
+		const std::uint32_t x = static_cast<std::uint32_t>(c % P.width), y = firstRow + static_cast<std::uint32_t>(c / P.width);
 		double upper[kNforUpper];
 		double rhs[kNforBasis][3];
 		#pragma unroll
@@ -706,7 +816,7 @@ namespace luzgpu
 				for (int j = 0; j < 3; j++) rhs[row][j] -= factor * rhs[pivot][j];
 			}
 		}
-		double* o = out + 3 * c;
+		double* o = out + 3 * (static_cast<size_t>(y) * P.width + x);
 		if (solved)
 		{
 			o[0] = rhs[0][0];

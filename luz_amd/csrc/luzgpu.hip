@@ -1037,41 +1037,62 @@ namespace luzgpu
 			nfor_variances<<<g, 256, 0, st>>>(colorVariance, featVariance, regVar, featVarAvg, static_cast<std::uint32_t>(n));
 			nfor_prefilter<<<g, 256, 0, st>>>(featA, featB, featVarAvg, ffA, P);
 			nfor_prefilter<<<g, 256, 0, st>>>(featB, featA, featVarAvg, ffB, P);
-			const unsigned tiles = blocks(P.width, kNforTile) * blocks(P.height, kNforTile);
-			constexpr unsigned tb = 2 * kNforTilePixels;
-			// each regression's per-pixel systems (nfor_accumulate -> nfor_solve)
-			ctx->nforSystems.reserve(static_cast<size_t>(kNforSystem) * n * sizeof(double));
+			// each regression's per-pixel systems (nfor_accumulate -> nfor_solve), for a band of
+			// image rows at a time: at most 4 GiB of systems, at least one row of tiles
+			const size_t rowBytes = static_cast<size_t>(kNforSystem) * P.width * sizeof(double) * 2;
+			const std::uint32_t bandTiles = static_cast<std::uint32_t>(std::max<size_t>(1, (size_t(4) << 30) / (rowBytes * kNforTileY)));
+			const std::uint32_t band = static_cast<std::uint32_t>(std::min<std::uint64_t>(P.height, static_cast<std::uint64_t>(bandTiles) * kNforTileY));
+			ctx->nforSystems.reserve(rowBytes * band);
 			double* systems = ctx->nforSystems.as<double>();
-			// the LDS-staged accumulation when its window fits the device's LDS per block
-			// (radius 9, patch radius 1: 158 KiB of the MI355X's 160 KiB), else the unstaged form
-			const size_t stagedBytes = static_cast<size_t>(nforLdsLayout(P.regressionRadius, P.patchRadius, true).doubles) * sizeof(double);
-			const size_t plainBytes = static_cast<size_t>(nforLdsLayout(P.regressionRadius, P.patchRadius, false).doubles) * sizeof(double);
 			int device = 0, ldsLimit = 0;
 			check(hipGetDevice(&device), "hipGetDevice");
 			check(hipDeviceGetAttribute(&ldsLimit, hipDeviceAttributeMaxSharedMemoryPerBlock, device), "LDS per block");
-			const bool staged = stagedBytes <= static_cast<size_t>(ldsLimit)
-				&& hipFuncSetAttribute(reinterpret_cast<const void*>(&nfor_accumulate<true>), hipFuncAttributeMaxDynamicSharedMemorySize,
-					static_cast<int>(stagedBytes)) == hipSuccess;
-			if (!staged && (plainBytes > static_cast<size_t>(ldsLimit)
-				|| hipFuncSetAttribute(reinterpret_cast<const void*>(&nfor_accumulate<false>), hipFuncAttributeMaxDynamicSharedMemorySize,
-					static_cast<int>(plainBytes)) != hipSuccess))
-			{
-				throw Error{LUZGPU_E_UNSUPPORTED, "NFOR patch radius too large for the device's LDS"};
-			}
-			auto regress = [&](const double* img, const double* feat, const double* var, double* dst, double bandwidth) {
-				if (staged) nfor_accumulate<true><<<tiles, tb, stagedBytes, st>>>(img, feat, var, systems, P, bandwidth);
-				else nfor_accumulate<false><<<tiles, tb, plainBytes, st>>>(img, feat, var, systems, P, bandwidth);
-				nfor_solve<<<g, 256, 0, st>>>(systems, img, var, dst, P);
+			// the LDS-staged accumulation when its window fits the device's LDS per block
+			// (radius 9, patch radius 1: 152 KiB of the MI355X's 160 KiB), else the unstaged form
+			const size_t stagedBytes = nforLdsLayout(P.regressionRadius, P.patchRadius, true).doubles * sizeof(double);
+			const size_t plainBytes = nforLdsLayout(P.regressionRadius, P.patchRadius, false).doubles * sizeof(double);
+			// one regression at bandwidth k into dst0, or (Two) one at 1 into dst0 and one at 1/2
+			// into dst1
+			auto regress = [&]<bool Two>(const double* img, const double* feat, const double* var, double* dst0, double* dst1, double k) {
+				auto fits = [&](const void* kernel, size_t bytes) {
+					return bytes <= static_cast<size_t>(ldsLimit)
+						&& hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(bytes)) == hipSuccess;
+				};
+				const bool staged = fits(reinterpret_cast<const void*>(&nfor_accumulate<true, Two>), stagedBytes);
+				if (!staged && !fits(reinterpret_cast<const void*>(&nfor_accumulate<false, Two>), plainBytes))
+				{
+					throw Error{LUZGPU_E_UNSUPPORTED, "NFOR patch radius too large for the device's LDS"};
+				}
+				for (std::uint32_t y = 0; y < P.height; y += band)
+				{
+					const std::uint32_t rows = std::min(band, P.height - y);
+					const unsigned tiles = blocks(P.width, kNforTileX) * blocks(rows, kNforTileY);
+					if (staged) nfor_accumulate<true, Two><<<tiles, kNforBlock, stagedBytes, st>>>(img, feat, var, systems, P, k, y, rows);
+					else nfor_accumulate<false, Two><<<tiles, kNforBlock, plainBytes, st>>>(img, feat, var, systems, P, k, y, rows);
+					const size_t n1 = static_cast<size_t>(P.width) * rows;
+					nfor_solve<<<blocks(n1, 256), 256, 0, st>>>(systems, img, var, dst0, P, y, rows);
+					if (Two) nfor_solve<<<blocks(n1, 256), 256, 0, st>>>(systems + kNforSystem * n1, img, var, dst1, P, y, rows);
+				}
 			};
-			regress(supA, ffB, regVar, a0, 0.5);
-			regress(supA, ffB, regVar, a1, 1.0);
-			regress(supB, ffA, regVar, b0, 0.5);
-			regress(supB, ffA, regVar, b1, 1.0);
+			// bandwidths 1/2 and 1: one pass while the second weight is the first's fourth power
+			// (the variance floor leaves their squares 4 apart), else two
+			if (P.minVariance <= 0.25)
+			{
+				regress.template operator()<true>(supA, ffB, regVar, a1, a0, 1.0);
+				regress.template operator()<true>(supB, ffA, regVar, b1, b0, 1.0);
+			}
+			else
+			{
+				regress.template operator()<false>(supA, ffB, regVar, a0, nullptr, 0.5);
+				regress.template operator()<false>(supA, ffB, regVar, a1, nullptr, 1.0);
+				regress.template operator()<false>(supB, ffA, regVar, b0, nullptr, 0.5);
+				regress.template operator()<false>(supB, ffA, regVar, b1, nullptr, 1.0);
+			}
 			nfor_mse<<<g, 256, 0, st>>>(supA, supB, a0, b0, a1, b1, regVar, m0, m1, static_cast<std::uint32_t>(n));
 			nfor_filter_pair<<<g, 256, 0, st>>>(m0, m1, color, colorVariance, f0, f1, P, 0);
 			nfor_filter_pair<<<g, 256, 0, st>>>(f0, f1, color, colorVariance, s0, s1, P, 1);
 			nfor_combine<<<g, 256, 0, st>>>(s0, s1, f0, f1, a0, a1, b0, b1, ffA, ffB, combined, finalFeat, finalVar, P);
-			regress(combined, finalFeat, finalVar, out, 1.0);
+			regress.template operator()<false>(combined, finalFeat, finalVar, out, nullptr, 1.0);
 			check(hipGetLastError(), "NFOR launch");
 		}
 
