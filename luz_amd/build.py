@@ -13,6 +13,7 @@ import os
 import shutil
 import subprocess
 import sys
+from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
@@ -20,7 +21,9 @@ LIB = os.path.join(HERE, "libluzgpu.so")
 BUILD = os.path.join(HERE, "_build")
 
 HOST_SOURCES = ["host/scene_file.cpp", "host/accel.cpp", "host/scene_desc.cpp"]
-DEVICE_SOURCES = ["luzgpu.hip"]
+# (source, object, defines): the kernels of each scene feature class compile on their own
+DEVICE_SOURCES = [("luzgpu.hip", "luzgpu.hip.o", [])] + [
+    ("features.hip", f"features{f}.hip.o", [f"-DLUZ_FEATURES={f}"]) for f in (0, 1, 2, 3, 7, 9)]
 ARCH = "gfx950"
 
 
@@ -44,16 +47,19 @@ def build(verbose: bool = False) -> str:
     os.makedirs(BUILD, exist_ok=True)
     objs = []
     common = ["-std=c++20", "-O3", "-fPIC", "-Wall", "-Wno-unused-parameter"]
+    jobs = []
+    for src, name, defines in DEVICE_SOURCES:
+        obj = os.path.join(BUILD, name)
+        jobs.append([hipcc, *common, f"--offload-arch={ARCH}", "-x", "hip", *defines,
+                     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+                     "-munsafe-fp-atomics", "-c", os.path.join(CSRC, src), "-o", obj])
+        objs.append(obj)
     for src in HOST_SOURCES:
         obj = os.path.join(BUILD, os.path.basename(src) + ".o")
-        _run(["g++", *common, "-ffp-contract=off", "-fno-fast-math", "-c", os.path.join(CSRC, src), "-o", obj])
+        jobs.append(["g++", *common, "-ffp-contract=off", "-fno-fast-math", "-c", os.path.join(CSRC, src), "-o", obj])
         objs.append(obj)
-    for src in DEVICE_SOURCES:
-        obj = os.path.join(BUILD, os.path.basename(src) + ".o")
-        _run([hipcc, *common, f"--offload-arch={ARCH}", "-x", "hip",
-              "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
-              "-munsafe-fp-atomics", "-c", os.path.join(CSRC, src), "-o", obj])
-        objs.append(obj)
+    with ThreadPoolExecutor(max_workers=8) as pool:
+        list(pool.map(_run, jobs))
     tmp = LIB + ".tmp"
     _run([hipcc, "-shared", "-fPIC", f"--offload-arch={ARCH}", *objs, "-o", tmp])
     os.replace(tmp, LIB)

@@ -309,11 +309,25 @@ namespace luzgpu
 
 	// Scene content classes the kernels are specialised on (a scene without them runs
 	// kernels that do not carry their code or registers).
-	constexpr int	kFeatAnalytic = 1;	// spheres, cubes, volumes, planes, directional and mesh-instance lights
-	constexpr int	kFeatRich = 2;		// glossy, diffuse-glossy, principled, isotropic, Henyey-Greenstein; the atmosphere sky
+	constexpr int	kFeatAnalytic = 1;	// spheres, cubes, volumes, planes, directional and sphere lights
+	constexpr int	kFeatRich = 2;		// glossy, diffuse-glossy, principled, isotropic, Henyey-Greenstein; the atmosphere
+										// sky; mesh-instance lights (with kFeatAnalytic)
 	constexpr int	kFeatAll = 3;
 	constexpr int	kFeatSubsurface = 4;	// Burley subsurface exits (a closest-hit probe ray while shading)
 	constexpr int	kFeatEvery = 7;
+	// isotropic and Henyey-Greenstein media alone, a class of its own with kFeatAnalytic: the
+	// rich class's shading needs twice the registers (720p hazy terrain: shade 35.8 -> 21.4 ms, with the staged appends of wf_shade)
+	constexpr int	kFeatPhase = 8;
+	constexpr int	kFeatMedia = kFeatAnalytic | kFeatPhase;
+
+	// The class whose kernels a scene of these features runs: 0, kFeatAnalytic, kFeatMedia,
+	// kFeatRich, kFeatAll or kFeatEvery.
+	constexpr int	featureClass(int features)
+	{
+		if (features & kFeatSubsurface) return kFeatEvery;
+		if (features & kFeatRich) return features & kFeatAll;
+		return (features & kFeatPhase) ? kFeatMedia : features & kFeatAnalytic;
+	}
 
 	// Per-scene traversal entry of a multi-scene launch: TLAS root and the unbounded
 	// (plane) list as base << 16 | count.

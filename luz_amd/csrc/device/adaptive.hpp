@@ -103,10 +103,11 @@ namespace luzgpu
 			&& channelConverged(m[kAdaptiveColorSum + 2] / n, bCI, r.threshold);
 	}
 
+#ifndef LUZ_FEATURES
 	// After a round that brought every listed pixel to `used` samples: records `used` for
 	// each, and appends the pixels the rule keeps active to `next` (order unspecified; one
 	// atomic per wave). `list` == nullptr lists every pixel 0..count-1.
-	__global__ void	adaptive_check(AdaptiveRule rule, const std::uint32_t* __restrict__ list, std::uint32_t count, std::uint32_t used,
+	static __global__ void	adaptive_check(AdaptiveRule rule, const std::uint32_t* __restrict__ list, std::uint32_t count, std::uint32_t used,
 		const double* __restrict__ moments, std::uint32_t* __restrict__ usedOut, std::uint32_t* __restrict__ next,
 		std::uint32_t* __restrict__ nextCount)
 	{
@@ -127,4 +128,5 @@ namespace luzgpu
 		base = __shfl(base, leader < 0 ? 0 : leader);
 		if (active) next[base + static_cast<std::uint32_t>(__popcll(mask & ((1ull << lane) - 1ull)))] = pixel;
 	}
+#endif
 }

@@ -222,8 +222,8 @@ namespace luzgpu
 	__device__ __forceinline__ f3	scatterDirection(const Surface& sf, const Scatter& sc, const PixelSampler& ps)
 	{
 		if (sc.pdfType == PDF_COSINE) return cosineDirection(sf, ps);
-		if ((Feat & kFeatRich) && sc.pdfType == PDF_SPHERE) return sphereDirection(ps);
-		if ((Feat & kFeatRich) && sc.pdfType == PDF_HG) return hgDirection(sc, ps);
+		if (kHasPhase<Feat> && sc.pdfType == PDF_SPHERE) return sphereDirection(ps);
+		if (kHasPhase<Feat> && sc.pdfType == PDF_HG) return hgDirection(sc, ps);
 		return sc.direction;
 	}
 

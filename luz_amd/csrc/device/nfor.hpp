@@ -59,6 +59,7 @@ namespace luzgpu
 		}
 	}
 
+#ifndef LUZ_FEATURES	// the denoiser's kernels are compiled once, in luzgpu.hip
 	struct	NforParams
 	{
 		std::uint32_t	width, height;
@@ -121,7 +122,7 @@ namespace luzgpu
 	// neighbours in its 5 x 5 window that stands 2.5x and 0.18 above the window's median
 	// luminance takes the luminance-median of its darker neighbours. `average` != 0: the
 	// input is the mean of a and b (averageColorBuffers) instead of a.
-	__global__ void	nfor_fireflies(const double* __restrict__ a, const double* __restrict__ b, double* __restrict__ out,
+	static __global__ void	nfor_fireflies(const double* __restrict__ a, const double* __restrict__ b, double* __restrict__ out,
 		NforParams P, int average)
 	{
 		const std::uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -204,7 +205,7 @@ namespace luzgpu
 	}
 
 	// doubledVariance and averageFeatureVarianceMap (NFOR.cpp:331-353)
-	__global__ void	nfor_variances(const double* __restrict__ colorVariance, const double* __restrict__ featureVariance,
+	static __global__ void	nfor_variances(const double* __restrict__ colorVariance, const double* __restrict__ featureVariance,
 		double* __restrict__ regressionVariance, double* __restrict__ featureVarianceAverage, std::uint32_t n)
 	{
 		const std::uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -217,7 +218,7 @@ namespace luzgpu
 
 	// prefilterFeatures (NFOR.cpp:403-464): `image`'s features averaged with weights from
 	// `guide`'s feature distances and a spatial Gaussian.
-	__global__ void	nfor_prefilter(const double* __restrict__ image, const double* __restrict__ guide,
+	static __global__ void	nfor_prefilter(const double* __restrict__ image, const double* __restrict__ guide,
 		const double* __restrict__ varianceAverage, double* __restrict__ out, NforParams P)
 	{
 		const std::uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -386,7 +387,7 @@ namespace luzgpu
 	// their patches from global memory cost 1.8 ms of the weights; 16 waves of half the pixels
 	// each were slower (spills).
 	template <bool Staged, bool Two>
-	__global__ __launch_bounds__(kNforBlock, 2) void	nfor_accumulate(const double* __restrict__ image,
+	static __global__ __launch_bounds__(kNforBlock, 2) void	nfor_accumulate(const double* __restrict__ image,
 		const double* __restrict__ features, const double* __restrict__ variance, double* __restrict__ system, NforParams P,
 		double bandwidth, std::uint32_t firstRow, std::uint32_t rows)
 	{
@@ -724,7 +725,7 @@ namespace luzgpu
 	// reference's Gauss-Jordan elimination with partial pivoting on each system from
 	// nfor_accumulate (the pixels of `rows` image rows from firstRow); a singular system takes
 	// weightedAverageFallback.
-	__global__ __launch_bounds__(256) void	nfor_solve(const double* __restrict__ system, const double* __restrict__ image,
+	static __global__ __launch_bounds__(256) void	nfor_solve(const double* __restrict__ system, const double* __restrict__ image,
 		const double* __restrict__ variance, double* __restrict__ out, NforParams P, std::uint32_t firstRow, std::uint32_t rows)
 	{
 		#pragma clang fp contract(off)
@@ -830,7 +831,7 @@ namespace luzgpu
 	}
 
 	// estimateMSE (NFOR.cpp:875-893) of the first and the second bandwidth
-	__global__ void	nfor_mse(const double* __restrict__ colorA, const double* __restrict__ colorB, const double* __restrict__ a0,
+	static __global__ void	nfor_mse(const double* __restrict__ colorA, const double* __restrict__ colorB, const double* __restrict__ a0,
 		const double* __restrict__ b0, const double* __restrict__ a1, const double* __restrict__ b1,
 		const double* __restrict__ variance, double* __restrict__ mse0, double* __restrict__ mse1, std::uint32_t n)
 	{
@@ -849,7 +850,7 @@ namespace luzgpu
 	// filterScalarMapPair (NFOR.cpp:834-873): radius-3 cross-bilateral filter of two maps,
 	// weights from 3 x 3 colour patches of `guide` (bandwidth 1). `select` != 0: the maps are
 	// first turned into bandwidthSelectionMap(first, second) and (second, first) (:907-919).
-	__global__ void	nfor_filter_pair(const double* __restrict__ first, const double* __restrict__ second,
+	static __global__ void	nfor_filter_pair(const double* __restrict__ first, const double* __restrict__ second,
 		const double* __restrict__ guide, const double* __restrict__ guideVariance, double* __restrict__ out0,
 		double* __restrict__ out1, NforParams P, int select)
 	{
@@ -897,7 +898,7 @@ namespace luzgpu
 
 	// The per-pixel blend of applyNFOR (NFOR.cpp:1072-1087) and combinedResultVariance
 	// (:895-905): combined colour, blended features and the final regression's variance.
-	__global__ void	nfor_combine(const double* __restrict__ sel0, const double* __restrict__ sel1, const double* __restrict__ mse0,
+	static __global__ void	nfor_combine(const double* __restrict__ sel0, const double* __restrict__ sel1, const double* __restrict__ mse0,
 		const double* __restrict__ mse1, const double* __restrict__ a0, const double* __restrict__ a1, const double* __restrict__ b0,
 		const double* __restrict__ b1, const double* __restrict__ featA, const double* __restrict__ featB,
 		double* __restrict__ combined, double* __restrict__ features, double* __restrict__ variance, NforParams P)
@@ -918,4 +919,5 @@ namespace luzgpu
 		}
 		variance[i] = nforDist2(a1 + 3 * i, b1 + 3 * i) * 0.25;
 	}
+#endif
 }

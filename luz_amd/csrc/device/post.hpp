@@ -163,7 +163,7 @@ namespace luzgpu
 	}
 
 	// applyExposure (Image.cpp:467-484)
-	__global__ void	post_exposure(const double* __restrict__ in, double* __restrict__ out, PostParams P)
+	static __global__ void	post_exposure(const double* __restrict__ in, double* __restrict__ out, PostParams P)
 	{
 		#pragma clang fp contract(off)
 		const size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -172,7 +172,7 @@ namespace luzgpu
 	}
 
 	// extractBloom (Image.cpp:599-640) with suppressIsolatedBloomFirefly (Image.cpp:42-103)
-	__global__ void	post_bloom_extract(const double* __restrict__ img, double* __restrict__ bright, PostParams P)
+	static __global__ void	post_bloom_extract(const double* __restrict__ img, double* __restrict__ bright, PostParams P)
 	{
 		#pragma clang fp contract(off)
 		const size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -214,7 +214,7 @@ namespace luzgpu
 	}
 
 	// Gaussian::blur (Gaussian.cpp:80-150): the horizontal pass, clamped at the borders
-	__global__ void	post_blur_h(const double* __restrict__ in, double* __restrict__ out, PostParams P)
+	static __global__ void	post_blur_h(const double* __restrict__ in, double* __restrict__ out, PostParams P)
 	{
 		#pragma clang fp contract(off)
 		const size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -233,7 +233,7 @@ namespace luzgpu
 	}
 
 	// the vertical pass, and the bloom added back (applyBloom, Threads.cpp:55-75)
-	__global__ void	post_blur_v_add(const double* __restrict__ in, double* __restrict__ img, PostParams P)
+	static __global__ void	post_blur_v_add(const double* __restrict__ in, double* __restrict__ img, PostParams P)
 	{
 		#pragma clang fp contract(off)
 		const size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -255,7 +255,7 @@ namespace luzgpu
 	// The view transform to display-encoded sRGB: applyViewTransformAndEncodeSRGB
 	// (Image.cpp:571-597) at the default contrast, else applyViewTransform, applyContrast and
 	// gammaCorrect (Image.cpp:486-569). Not launched for the raw view.
-	__global__ void	post_view(const double* __restrict__ in, double* __restrict__ out, PostParams P)
+	static __global__ void	post_view(const double* __restrict__ in, double* __restrict__ out, PostParams P)
 	{
 		#pragma clang fp contract(off)
 		const size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -310,7 +310,7 @@ namespace luzgpu
 
 	// suppressIsolatedFireflies (Image.cpp:506-526) with suppressDisplayFirefly
 	// (Image.cpp:154-268), over the display-encoded image.
-	__global__ void	post_fireflies(const double* __restrict__ src, double* __restrict__ dst, PostParams P)
+	static __global__ void	post_fireflies(const double* __restrict__ src, double* __restrict__ dst, PostParams P)
 	{
 		#pragma clang fp contract(off)
 		const size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -395,7 +395,7 @@ namespace luzgpu
 		postStore(dst, i, postMedianColor(candidates, nCandidates));
 	}
 
-	__global__ void	post_to_float(const double* __restrict__ in, float* __restrict__ out, size_t n)
+	static __global__ void	post_to_float(const double* __restrict__ in, float* __restrict__ out, size_t n)
 	{
 		const size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
 		if (i < n) out[i] = static_cast<float>(in[i]);

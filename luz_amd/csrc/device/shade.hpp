@@ -22,6 +22,10 @@ namespace luzgpu
 {
 	constexpr float	kPiF = 3.14159265358979323846f;
 
+	// The kernels carry the phase functions.
+	template <int Feat>
+	constexpr bool	kHasPhase = (Feat & (kFeatRich | kFeatPhase)) != 0;
+
 	struct	Surface
 	{
 		f3	position;
@@ -504,8 +508,8 @@ namespace luzgpu
 			const float c = dot(dir, sc.cosineW);
 			return c <= 0.0f ? 0.0f : c / kPiF;
 		}
-		if ((Feat & kFeatRich) && sc.pdfType == PDF_SPHERE) return 1.0f / (4.0f * kPiF);
-		if ((Feat & kFeatRich) && sc.pdfType == PDF_HG) return hgPdf(sc.cosineW, sc.g, dir);
+		if (kHasPhase<Feat> && sc.pdfType == PDF_SPHERE) return 1.0f / (4.0f * kPiF);
+		if (kHasPhase<Feat> && sc.pdfType == PDF_HG) return hgPdf(sc.cosineW, sc.g, dir);
 		if (sc.pdfType == PDF_BSDF) return bsdfPdf<Feat>(m, sf, sc, dir);
 		return 0.0f;
 	}
@@ -583,7 +587,7 @@ namespace luzgpu
 			sc.cosineW = normalize(sf.normal);
 			return true;
 		}
-		if constexpr ((Feat & kFeatRich) != 0)
+		if constexpr (kHasPhase<Feat>)
 		{
 		if (m.kind == GPU_MAT_ISOTROPIC)
 		{
@@ -591,6 +595,17 @@ namespace luzgpu
 			sc.pdfType = PDF_SPHERE;
 			return true;
 		}
+		if (m.kind == GPU_MAT_HG)
+		{
+			sc.attenuation = ld3(m.color);
+			sc.pdfType = PDF_HG;
+			sc.cosineW = len2(inDir) <= 0.0f ? mk(0.0f, 0.0f, 1.0f) : normalize(inDir);
+			sc.g = m.anisotropy;
+			return true;
+		}
+		}
+		if constexpr ((Feat & kFeatRich) != 0)
+		{
 		if (m.kind == GPU_MAT_GLOSSY)
 		{
 			return acceptBsdfSample(m, sf, sampleGGXReflection(inDir, sf.normal, m.alpha, ps), sc);
@@ -666,14 +681,6 @@ namespace luzgpu
 				dir = sampleGGXReflection(inDir, sf.normal, comp == 6 ? m.clearcoatAlpha : m.alpha, ps);
 			}
 			return acceptBsdfSample(m, sf, dir, sc);
-		}
-		if (m.kind == GPU_MAT_HG)
-		{
-			sc.attenuation = ld3(m.color);
-			sc.pdfType = PDF_HG;
-			sc.cosineW = len2(inDir) <= 0.0f ? mk(0.0f, 0.0f, 1.0f) : normalize(inDir);
-			sc.g = m.anisotropy;
-			return true;
 		}
 		}
 		if (m.kind == GPU_MAT_METAL)
@@ -996,7 +1003,7 @@ namespace luzgpu
 			return sl;
 		}
 		f3 point, normal;
-		if ((Feat & kFeatAnalytic) && L.kind == GPU_HIT_INSTANCE)
+		if ((Feat & kFeatRich) && L.kind == GPU_HIT_INSTANCE)
 		{
 			// MeshInstance::sampleLight / _sampleSurface (MeshInstance.cpp:409-466,510-546): a
 			// triangle by area (std::lower_bound over the FP64 prefix sums), a point on it
@@ -1088,7 +1095,7 @@ namespace luzgpu
 			const double cosMax = sqrt(1.0 - rr / (cx * cx + cy * cy + cz * cz));
 			return static_cast<float>(1.0 / (2.0 * 3.14159265358979323846 * (1.0 - cosMax)));
 		}
-		if ((Feat & kFeatAnalytic) && L.kind == GPU_HIT_INSTANCE)
+		if ((Feat & kFeatRich) && L.kind == GPU_HIT_INSTANCE)
 		{
 			// MeshInstance::pdfValue (MeshInstance.cpp:468-497): this instance alone
 			if (!(L.area > 0.0f) || !(vl2 > 0.0f)) return 0.0f;

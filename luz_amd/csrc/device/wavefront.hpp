@@ -13,14 +13,15 @@
 //   raygen            camera rays (FP64, bit-exact sampler) -> queue 0, path state init
 //   for b = 0..maxBounces:
 //     extend          closest hit for every ray of queue b (persistent, lane refill)
-//     shade           miss / emission / scatter / NEE and environment connections, one
-//                     scene per wave iteration (waterfall over the wave's scene ids); the
-//                     next ray and up to two shadow rays are appended with one atomic per
-//                     wave (ballot + popcount prefix)
+//     shade           first adds the visible connections of the path's previous vertex in the
+//                     reference's order (light, then environment); then miss / emission /
+//                     scatter / NEE and environment connections, in batches one scene per
+//                     wave iteration (waterfall over the wave's scene ids); the next ray and
+//                     up to two shadow rays are appended with one atomic per block and queue;
+//                     a path that ended writes its colour
 //     shadow          any-hit test of the appended shadow rays -> visibility bytes
-//     resolve         adds visible connection terms in the reference's order (light, then
-//                     environment) and writes the colour of every path that ended
-//   accumulate        adds the pass's sample colours into each scene's FP64 pixel sums
+//   accumulate        adds the pass's sample colours into each scene's FP64 pixel sums; a path
+//                     that ended with connections to test gets them added here
 // Queue lengths and the pass's job table live in device memory and every stage is a
 // grid-stride or work-claiming loop over them, so a pass is a fixed launch sequence that
 // the host captures once as a hipGraph and replays for every pass.
@@ -43,10 +44,8 @@ namespace luzgpu
 	// path flags
 	constexpr std::uint32_t	PF_PREV_SPECULAR = 1u;
 	constexpr std::uint32_t	PF_PREV_INFINITE = 2u;
-	constexpr std::uint32_t	PF_DONE = 4u;		// the path ended in this bounce
 	constexpr std::uint32_t	PF_CONN_LIGHT = 8u;	// a light connection is pending
 	constexpr std::uint32_t	PF_CONN_ENV = 16u;	// an environment connection is pending
-	constexpr std::uint32_t	PF_CONN_FREE_LIGHT = 32u;	// light connection needs no shadow test
 
 	struct	WaveBuffers
 	{
@@ -115,11 +114,68 @@ namespace luzgpu
 		std::uint32_t	pathBase;	// first global path id of the slice
 		std::uint32_t	pixels;		// pixels rendered: the image, or the entries of pixelList
 		double*	sums;			// the scene's FP64 pixel sums
+		std::uint32_t	pixelsInverse;	// floor(2^32 / pixels) and floor(2^32 / width) for divide()
+		std::uint32_t	widthInverse;
 		const std::uint32_t*	pixelList;	// adaptive rounds: the active pixels (nullptr: every pixel)
 		double*	moments;		// adaptive rounds: per-pixel AdaptiveAccumulator (or nullptr)
 		float*	features;		// denoising: primary features per global path id (or nullptr)
 		double*	denoise;		// denoising: per-pixel statistics (kDenoiseStats) instead of sums
 	};
+
+	// n / d and n % d for inverse = floor(2^32 / d) (0xffffffff for d = 1): the estimate is at
+	// most one short.
+	__host__ __device__ __forceinline__ std::uint32_t	divide(std::uint32_t n, std::uint32_t d, std::uint32_t inverse, std::uint32_t& rest)
+	{
+		std::uint32_t q = static_cast<std::uint32_t>((static_cast<std::uint64_t>(n) * inverse) >> 32);
+		rest = n - q * d;
+		const bool more = rest >= d;
+		q += more ? 1u : 0u;
+		rest -= more ? d : 0u;
+		return q;
+	}
+
+	inline std::uint32_t	inverseOf(std::uint32_t d)
+	{
+		return d <= 1u ? 0xffffffffu : static_cast<std::uint32_t>((1ull << 32) / d);
+	}
+
+	// A colour that no sample has (cleanColor leaves finite values only): the path ended with
+	// connections that had yet to be tested, and accumulation adds them (pathColor).
+	constexpr std::uint32_t	kPendingColor = 0x7fc0beefu;
+
+	// Adds the visible ones of a path's connections to its radiance (light, then environment).
+	__device__ __forceinline__ f3	addConnections(const WaveBuffers& w, std::uint32_t path, std::uint32_t flags, f3 acc)
+	{
+		if ((flags & PF_CONN_LIGHT) && w.visible[2 * path])
+		{
+			const float4 c = w.connection[2 * path];
+			acc = acc + clampRay(mk(c.x, c.y, c.z));
+		}
+		if ((flags & PF_CONN_ENV) && w.visible[2 * path + 1])
+		{
+			const float4 c = w.connection[2 * path + 1];
+			acc = acc + clampRay(mk(c.x, c.y, c.z));
+		}
+		return acc;
+	}
+
+	// The cleaned colour of sample (path) `g` of a pass.
+	__device__ __forceinline__ void	pathColor(const WaveBuffers& w, const float* __restrict__ colors, size_t g, float (&out)[3])
+	{
+		const float* c = colors + 3 * g;
+		out[0] = c[0];
+		out[1] = c[1];
+		out[2] = c[2];
+		if (__float_as_uint(out[0]) == kPendingColor)
+		{
+			const std::uint32_t path = static_cast<std::uint32_t>(g);
+			const float4 r4 = w.radiance[path];
+			const f3 v = cleanColor(addConnections(w, path, __float_as_uint(r4.w), mk(r4.x, r4.y, r4.z)));
+			out[0] = v.x;
+			out[1] = v.y;
+			out[2] = v.z;
+		}
+	}
 
 	// Image pixel of entry i of a pass's pixel range.
 	__device__ __forceinline__ std::uint32_t	passPixel(const PassJob& J, std::uint32_t i)
@@ -157,7 +213,7 @@ namespace luzgpu
 	__device__ __forceinline__ std::uint32_t	laneId() { return threadIdx.x & 63u; }
 
 	// The pass's total path count: written into counts[0] (queue 0 holds every path).
-	__global__ void	wf_zero_counts(std::uint32_t* counts, std::uint32_t n, const PassJob* jobs, std::uint32_t jobCount)
+	static __global__ void	wf_zero_counts(std::uint32_t* counts, std::uint32_t n, const PassJob* jobs, std::uint32_t jobCount)
 	{
 		const std::uint32_t i = threadIdx.x;
 		if (i < n)
@@ -182,7 +238,7 @@ namespace luzgpu
 
 	// Camera rays of every job of the pass in one launch (queue 0 holds the pass's paths in
 	// job order, counts[0] of them).
-	__global__ __launch_bounds__(kWaveBlock) void	wf_raygen(const PassJob* jobs, std::uint32_t jobCount, WaveBuffers w)
+	static __global__ __launch_bounds__(kWaveBlock) void	wf_raygen(const PassJob* jobs, std::uint32_t jobCount, WaveBuffers w)
 	{
 		const std::uint32_t total = w.counts[0];
 		for (std::uint32_t g = blockIdx.x * kWaveBlock + threadIdx.x; g < total; g += gridDim.x * kWaveBlock)
@@ -203,7 +259,8 @@ namespace luzgpu
 			// (coherent first traversals). The path keeps its row-major id, which the later
 			// stages and the accumulation decode.
 			const std::uint32_t id = g - J.pathBase;
-			const std::uint32_t slot = id / pixels, order = id % pixels;
+			std::uint32_t order;
+			const std::uint32_t slot = divide(id, pixels, J.pixelsInverse, order);
 			std::uint32_t pixel;
 			if (J.pixelList)
 			{
@@ -211,13 +268,17 @@ namespace luzgpu
 			}
 			else
 			{
-				const std::uint32_t band = order / (8u * p.width);
+				std::uint32_t inRow;
+				const std::uint32_t row = divide(order, p.width, J.widthInverse, inRow);
+				const std::uint32_t band = row / 8u;
 				const std::uint32_t bandRows = min(8u, p.height - band * 8u);
 				const std::uint32_t within = order - band * 8u * p.width;
-				pixel = (band * 8u + within % bandRows) * p.width + within / bandRows;
+				const std::uint32_t column = bandRows == 8u ? within / 8u : within / bandRows;
+				pixel = (band * 8u + within - column * bandRows) * p.width + column;
 			}
 			const std::uint32_t path = J.pathBase + slot * pixels + (J.pixelList ? order : pixel);
-			const std::uint32_t x = pixel % p.width, y = pixel / p.width;
+			std::uint32_t x;
+			const std::uint32_t y = divide(pixel, p.width, J.widthInverse, x);
 			PixelSampler ps;
 			ps.begin(p.renderSeed, x, y, p.sampleBegin + slot, sampleStream(p, p.sampleBegin + slot));
 			const Ray r = cameraRay(p, x, y, ps);
@@ -461,18 +522,27 @@ namespace luzgpu
 	// The traversal kernels are asked for at least 4 waves per SIMD (at most 128 VGPRs): the
 	// analytic-primitive specialisation otherwise takes 136 and runs 3 (terrain extend 41.4 ->
 	// 36.8 ms); the triangle-only one needs 88 and is unaffected.
-	__global__ __launch_bounds__(kWaveBlock, 4) void	wf_extend(SceneView s, const PassJob* jobs, WaveBuffers w, int b,
+	static __global__ __launch_bounds__(kWaveBlock, 4) void	wf_extend(SceneView s, const PassJob* jobs, WaveBuffers w, int b,
 		unsigned long long* counters, int refillAt, std::uint32_t chunk)
 	{
 		ExtendQueue src{w, b, w.spill};
 		traceQueue<false, Count, Feat, LdsDepth>(s, jobs, src, w.counts + 2 * kMaxBounceSlots + b, refillAt, chunk, counters, 0);
 	}
 
-	// The plain specialisation is asked for 4 waves per SIMD (128 VGPRs, a few spills): its
-	// loads of per-path state are latency-bound, and 2 waves left them exposed.
+	// Waves per SIMD asked of the shade kernels, whose chains of dependent loads (queue, hit,
+	// primitive, material, light tables) are latency-bound: what their registers allow with
+	// next to no spills. 1080p spheres: shade 12.1 -> 8.8 ms (180 -> 16 bytes spilled at 4 waves);
+	// 720p hazy terrain 35.8 -> 21.4 (1 -> 3 waves); 641 x 479 principled scene 2.7 -> 1.8.
 	template <int Feat>
-	__global__ __launch_bounds__(kWaveBlock, (Feat == 0 ? 4 : 1)) void	wf_shade(SceneView s, const PassJob* jobs, WaveBuffers w, int b,
-		std::uint32_t volumes)
+	constexpr int	kShadeWaves = Feat == 0 ? 4 : (Feat & kFeatRich) ? 2 : 3;
+
+	// Batch: the pass holds several scenes. What a path appends to the queues is staged in LDS
+	// until the block's ranges are known, and its connections' contributions are stored at
+	// once: held in registers they would live across the whole body (in a batch across the
+	// bodies of the wave's other scenes too) and spill.
+	template <int Feat, bool Batch>
+	static __global__ __launch_bounds__(kWaveBlock, kShadeWaves<Feat>) void	wf_shade(SceneView s, const PassJob* jobs, WaveBuffers w, int b,
+		std::uint32_t volumes, float* __restrict__ sampleColors)
 	{
 		const std::uint32_t n = w.counts[b];
 		const int q = b & 1;
@@ -484,6 +554,19 @@ namespace luzgpu
 		// are shared by every XCD, so per-wave atomics on them queue up behind each other.
 		constexpr int kWaves = kWaveBlock / 64;
 		__shared__ std::uint32_t waveNext[kWaves], waveShadow[kWaves], blockNext, blockShadow;
+		// staged per lane: the vertex, the next direction, its origin's identity, the light
+		// connection's direction and distance, the environment's direction, the volume samples
+		// of the next ray and of the shadow rays
+		constexpr int kStageFrom = 6, kStageLight = 8, kStageEnv = 12, kStageLogU = 15, kStageFields = 17;
+		__shared__ float stageMem[kStageFields * kWaveBlock];
+		float* const stage = stageMem + threadIdx.x;
+		auto put = [&](int field, float v) { stage[field * kWaveBlock] = v; };
+		auto put3 = [&](int field, f3 v) {
+			put(field, v.x);
+			put(field + 1, v.y);
+			put(field + 2, v.z);
+		};
+		auto get = [&](int field) { return stage[field * kWaveBlock]; };
 		const int wave = static_cast<int>(threadIdx.x >> 6);
 		// grid-stride loop with a block-uniform trip count so every lane reaches the ballots
 		// and every wave the barriers
@@ -493,46 +576,32 @@ namespace luzgpu
 			const std::uint32_t i = blockBase + threadIdx.x;
 			const bool valid = i < n;
 			bool cont = false, wantLight = false, wantEnv = false;
-			Ray next{};
-			Connection cl{}, ce{};
-			f3 shadePoint = mk(0, 0, 0);
-			RayOrigin from = kNoOrigin;
 			const std::uint32_t qp = valid ? w.qPath[q][i] : 0u;
-			const std::uint32_t job = w.sceneOfPath(qp);
-			const std::uint32_t path = w.pathOf(qp);
-			float nextLogU = 0.0f, shadowLogU = 0.0f;
-			// one scene per iteration, so the scene's parameters are wave-uniform (scalar loads)
-			unsigned long long pending = __ballot(valid);
-			while (pending)
-			{
-				const int leader = __ffsll(static_cast<long long>(pending)) - 1;
-				const std::uint32_t cur = __builtin_amdgcn_readfirstlane(__shfl(job, leader));
-				const bool mine = valid && job == cur;
-				if (mine)
-				{
-				const PassJob& J = jobs[cur];
+			const std::uint32_t job = Batch ? w.sceneOfPath(qp) : 0u;
+			const std::uint32_t path = Batch ? w.pathOf(qp) : qp;
+			auto shadePath = [&](const PassJob& J) {
 				const GpuParams& p = J.params;
-				const bool sampledInfinite = hasEnvLight(p) || hasConstantBackgroundLight(p);
-				const std::uint32_t local = path - J.pathBase;
-				const std::uint32_t pixel = passPixel(J, local % J.pixels), slot = local / J.pixels;
-				const std::uint32_t px = pixel % p.width, py = pixel / p.width;
+				std::uint32_t entry, px;
+				const std::uint32_t slot = divide(path - J.pathBase, J.pixels, J.pixelsInverse, entry);
+				const std::uint32_t py = divide(passPixel(J, entry), p.width, J.widthInverse, px);
 				PixelSampler ps;
 				ps.begin(p.renderSeed, px, py, p.sampleBegin + slot, sampleStream(p, p.sampleBegin + slot));
 				ps.bounce = static_cast<std::uint32_t>(b);
 				const float4 hv = w.qHit[i];
 				const float4 o = w.qOrigin[q][i], d = w.qDir[q][i];
 				const Ray ray = makeRay(mk(o.x, o.y, o.z), mk(d.x, d.y, d.z));
-				shadowLogU = o.w;
 				// a camera path starts with throughput 1, no radiance, and counts as leaving a
 				// specular vertex (the camera): those are not stored by ray generation
-				float4 t4 = b == 0 ? make_float4(1.0f, 1.0f, 1.0f, 0.0f) : w.throughput[path];
-				float4 r4 = b == 0 ? make_float4(0.0f, 0.0f, 0.0f, __uint_as_float(PF_PREV_SPECULAR)) : w.radiance[path];
+				const float4 t4 = b == 0 ? make_float4(1.0f, 1.0f, 1.0f, 0.0f) : w.throughput[path];
+				const float4 r4 = b == 0 ? make_float4(0.0f, 0.0f, 0.0f, __uint_as_float(PF_PREV_SPECULAR)) : w.radiance[path];
 				f3 thr = mk(t4.x, t4.y, t4.z), acc = mk(r4.x, r4.y, r4.z);
-				std::uint32_t flags = __float_as_uint(r4.w) & (PF_PREV_SPECULAR | PF_PREV_INFINITE);
-				const bool prevSpecular = flags & PF_PREV_SPECULAR;
-				const bool prevInfinite = flags & PF_PREV_INFINITE;
+				const std::uint32_t before = __float_as_uint(r4.w);
+				acc = addConnections(w, path, before, acc);
+				const bool prevSpecular = before & PF_PREV_SPECULAR;
+				const bool prevInfinite = before & PF_PREV_INFINITE;
 				const float prevPdf = t4.w;
-				bool done = true;
+				std::uint32_t flags = 0u;	// of this vertex
+				float nextPdf = 0.0f;
 				if (hv.x < 0.0f)
 				{
 					float wgt = 1.0f;
@@ -558,8 +627,7 @@ namespace luzgpu
 					h.hittable = __float_as_uint(hv.w);
 					h.tri = w.qTri[i];
 					Surface sf = surfaceAt<Feat>(s, ray, h);
-					shadePoint = sf.position;
-					from = originOf(s, h);
+					RayOrigin from = originOf(s, h);
 					const GpuMaterial& m = s.materials[sf.material];
 					if (b == 0 && J.features)
 					{
@@ -600,9 +668,8 @@ namespace luzgpu
 								LocalStack probeStack;
 								probeStack.reset();
 								std::uint32_t probes = 0;
-								relocateSubsurface<Feat>(s, p, m, h, sf, sc, ps, probeStack, shadowLogU, probes);
+								relocateSubsurface<Feat>(s, p, m, h, sf, sc, ps, probeStack, o.w, probes);
 								from = originOf(s, h);
-								shadePoint = sf.position;
 							}
 						}
 						f3 att = sc.attenuation;
@@ -614,6 +681,10 @@ namespace luzgpu
 								att = att * mk(expf(-m.absorption[0] * dm), expf(-m.absorption[1] * dm), expf(-m.absorption[2] * dm));
 							}
 						}
+						put3(0, sf.position);
+						put(kStageFrom, __uint_as_float(from.hittable));
+						put(kStageFrom + 1, __int_as_float(from.tri));
+						put(kStageLogU + 1, o.w);
 						if (sc.specular)
 						{
 							if (leavesOpaque(sf, m, sc.direction))
@@ -621,10 +692,9 @@ namespace luzgpu
 								thr = clampRay(thr * att);
 								if (!terminated(thr) && russianRoulette(thr, b, ps))
 								{
-									next = makeRay(sf.position, sc.direction);
+									put3(3, sc.direction);
 									flags = PF_PREV_SPECULAR;
-									t4.w = 0.0f;
-									done = false;
+									cont = b < p.maxBounces;
 								}
 							}
 						}
@@ -633,24 +703,33 @@ namespace luzgpu
 							acc = acc + thr * emitted;
 							if (!terminated(thr * att))
 							{
+								// a connection's clampRay is applied when it is added
+								auto connect = [&](std::uint32_t slotOf, const Connection& c, bool test) {
+									const f3 v = thr * c.contribution;
+									w.connection[2 * path + slotOf] = make_float4(v.x, v.y, v.z, 0.0f);
+									w.visible[2 * path + slotOf] = test ? 0 : 1;
+								};
 								if (p.lightCount > 0)
 								{
-									cl = connectLight<Feat>(s, p, sf, m, sc, b, ps);
-									if (cl.active)
+									const Connection c = connectLight<Feat>(s, p, sf, m, sc, b, ps);
+									if (c.active)
 									{
-										cl.contribution = thr * cl.contribution;	// clampRay applied at resolve
-										wantLight = cl.tMax > 0.0f;
-										flags |= PF_CONN_LIGHT | (wantLight ? 0u : PF_CONN_FREE_LIGHT);
+										wantLight = c.tMax > 0.0f;
+										flags |= PF_CONN_LIGHT;
+										connect(0u, c, wantLight);
+										put3(kStageLight, c.direction);
+										put(kStageLight + 3, c.tMax);
 									}
 								}
-								if (sampledInfinite)
+								if (hasEnvLight(p) || hasConstantBackgroundLight(p))
 								{
-									ce = connectInfinite<Feat>(s, p, sf, m, sc, b, ps);
-									if (ce.active)
+									const Connection c = connectInfinite<Feat>(s, p, sf, m, sc, b, ps);
+									if (c.active)
 									{
-										ce.contribution = thr * ce.contribution;
 										wantEnv = true;
 										flags |= PF_CONN_ENV;
+										connect(1u, c, true);
+										put3(kStageEnv, c.direction);
 									}
 								}
 								const f3 dir = scatterDirection<Feat>(sf, sc, ps);
@@ -662,16 +741,15 @@ namespace luzgpu
 										thr = clampRay(thr * att);
 										if (!terminated(thr) && russianRoulette(thr, b, ps))
 										{
-											next = makeRay(sf.position, dir);
-											flags = (flags & (PF_CONN_LIGHT | PF_CONN_ENV | PF_CONN_FREE_LIGHT))
-												| (samplesVisibleInfinite(p, sc) ? PF_PREV_INFINITE : 0u);
-											t4.w = pdf;
+											put3(3, dir);
+											flags |= samplesVisibleInfinite(p, sc) ? PF_PREV_INFINITE : 0u;
+											nextPdf = pdf;
+											cont = b < p.maxBounces;
 											// read back only for an emitter's MIS weight
-											if (p.lightCount > 0)
+											if (cont && p.lightCount > 0)
 											{
 												w.prevOrigin[path] = make_float4(sf.position.x, sf.position.y, sf.position.z, 0.0f);
 											}
-											done = false;
 										}
 									}
 								}
@@ -679,30 +757,38 @@ namespace luzgpu
 						}
 					}
 				}
-				if (done || b >= p.maxBounces)
+				if (cont)
 				{
-					flags |= PF_DONE;
-					done = true;
+					w.throughput[path] = make_float4(thr.x, thr.y, thr.z, nextPdf);
+					if (p.hasVolumes) put(kStageLogU, pathVolumeLogU(p, px, py, p.sampleBegin + slot, b + 1));
 				}
-				cont = !done;
-				w.throughput[path] = make_float4(thr.x, thr.y, thr.z, t4.w);
-				w.radiance[path] = make_float4(acc.x, acc.y, acc.z, __uint_as_float(flags));
-				if (flags & PF_CONN_LIGHT)
+				const bool pending = (flags & (PF_CONN_LIGHT | PF_CONN_ENV)) != 0u;
+				if (cont || pending) w.radiance[path] = make_float4(acc.x, acc.y, acc.z, __uint_as_float(flags));
+				if (!cont)
 				{
-					w.connection[2 * path] = make_float4(cl.contribution.x, cl.contribution.y, cl.contribution.z, 0.0f);
-					w.visible[2 * path] = wantLight ? 0 : 1;
+					const f3 c = cleanColor(acc);
+					float* out = sampleColors + static_cast<size_t>(path) * 3;
+					out[0] = pending ? __uint_as_float(kPendingColor) : c.x;
+					out[1] = c.y;
+					out[2] = c.z;
 				}
-				if (flags & PF_CONN_ENV)
+			};
+			if constexpr (Batch)
+			{
+				// one scene per iteration, so the scene's parameters are wave-uniform (scalar loads)
+				unsigned long long left = __ballot(valid);
+				while (left)
 				{
-					w.connection[2 * path + 1] = make_float4(ce.contribution.x, ce.contribution.y, ce.contribution.z, 0.0f);
-					w.visible[2 * path + 1] = 0;
+					const int leader = __ffsll(static_cast<long long>(left)) - 1;
+					const std::uint32_t cur = __builtin_amdgcn_readfirstlane(__shfl(job, leader));
+					const bool mine = valid && job == cur;
+					if (mine) shadePath(jobs[cur]);
+					left &= ~__ballot(mine);
 				}
-				if (cont && p.hasVolumes)
-				{
-					nextLogU = pathVolumeLogU(p, px, py, p.sampleBegin + slot, b + 1);
-				}
-				}
-				pending &= ~__ballot(mine);
+			}
+			else if (valid)
+			{
+				shadePath(jobs[0]);
 			}
 			const unsigned long long mNext = __ballot(cont), mLight = __ballot(wantLight), mEnv = __ballot(wantEnv);
 			const std::uint32_t nLight = static_cast<std::uint32_t>(__popcll(mLight));
@@ -731,31 +817,34 @@ namespace luzgpu
 				shadowBase += waveShadow[k];
 			}
 			const unsigned long long below = (1ull << laneId()) - 1ull;
-			const std::uint32_t pos = nextBase + static_cast<std::uint32_t>(__popcll(mNext & below));
-			if (cont)
+			if (cont || wantLight || wantEnv)
 			{
-				const int nq = (b + 1) & 1;
-				w.qOrigin[nq][pos] = make_float4(next.o.x, next.o.y, next.o.z, nextLogU);
-				w.qDir[nq][pos] = make_float4(next.d.x, next.d.y, next.d.z, __uint_as_float(from.hittable));
-				w.qFrom[nq][pos] = from.tri;
-				w.qPath[nq][pos] = qp;
-			}
-			const std::uint32_t tagScene = job;
-			const std::uint32_t sl = shadowBase + static_cast<std::uint32_t>(__popcll(mLight & below));
-			if (wantLight)
-			{
-				w.sOrigin[sl] = make_float4(shadePoint.x, shadePoint.y, shadePoint.z, cl.tMax);
-				w.sDir[sl] = make_float4(cl.direction.x, cl.direction.y, cl.direction.z, __uint_as_float(w.shadowTag(tagScene, 2u * path)));
-				w.sFrom[sl] = make_int2(static_cast<int>(from.hittable), from.tri);
-				if (volumes) w.sLogU[sl] = shadowLogU;
-			}
-			const std::uint32_t se = shadowBase + nLight + static_cast<std::uint32_t>(__popcll(mEnv & below));
-			if (wantEnv)
-			{
-				w.sOrigin[se] = make_float4(shadePoint.x, shadePoint.y, shadePoint.z, INFINITY);
-				w.sDir[se] = make_float4(ce.direction.x, ce.direction.y, ce.direction.z, __uint_as_float(w.shadowTag(tagScene, 2u * path + 1u)));
-				w.sFrom[se] = make_int2(static_cast<int>(from.hittable), from.tri);
-				if (volumes) w.sLogU[se] = shadowLogU;
+				const float x = get(0), y = get(1), z = get(2);
+				const float fromHittable = get(kStageFrom);
+				const std::int32_t fromTri = __float_as_int(get(kStageFrom + 1));
+				if (cont)
+				{
+					const std::uint32_t pos = nextBase + static_cast<std::uint32_t>(__popcll(mNext & below));
+					const int nq = (b + 1) & 1;
+					w.qOrigin[nq][pos] = make_float4(x, y, z, volumes ? get(kStageLogU) : 0.0f);
+					w.qDir[nq][pos] = make_float4(get(3), get(4), get(5), fromHittable);
+					w.qFrom[nq][pos] = fromTri;
+					w.qPath[nq][pos] = qp;
+				}
+				auto appendShadow = [&](std::uint32_t at, int field, float tMax, std::uint32_t slotOf) {
+					w.sOrigin[at] = make_float4(x, y, z, tMax);
+					w.sDir[at] = make_float4(get(field), get(field + 1), get(field + 2), __uint_as_float(w.shadowTag(job, 2u * path + slotOf)));
+					w.sFrom[at] = make_int2(__float_as_int(fromHittable), fromTri);
+					if (volumes) w.sLogU[at] = get(kStageLogU + 1);
+				};
+				if (wantLight)
+				{
+					appendShadow(shadowBase + static_cast<std::uint32_t>(__popcll(mLight & below)), kStageLight, get(kStageLight + 3), 0u);
+				}
+				if (wantEnv)
+				{
+					appendShadow(shadowBase + nLight + static_cast<std::uint32_t>(__popcll(mEnv & below)), kStageEnv, INFINITY, 1u);
+				}
 			}
 			// the next iteration rewrites the per-wave counts
 			__syncthreads();
@@ -764,60 +853,17 @@ namespace luzgpu
 
 	// any-hit test of the shadow rays appended in bounce b
 	template <bool Count, int Feat, int LdsDepth>
-	__global__ __launch_bounds__(kWaveBlock, 4) void	wf_shadow(SceneView s, const PassJob* jobs, WaveBuffers w, int b,
+	static __global__ __launch_bounds__(kWaveBlock, 4) void	wf_shadow(SceneView s, const PassJob* jobs, WaveBuffers w, int b,
 		unsigned long long* counters, int refillAt, std::uint32_t chunk, std::uint32_t volumes)
 	{
 		ShadowQueue src{w, b, w.spill, volumes, 0u};
 		traceQueue<true, Count, Feat, LdsDepth>(s, jobs, src, w.counts + 3 * kMaxBounceSlots + b, refillAt, chunk, counters, 1);
 	}
 
-	// sampleColors is indexed by global path id
-	__global__ __launch_bounds__(kWaveBlock) void	wf_resolve(WaveBuffers w, int b, float* __restrict__ sampleColors)
-	{
-		const std::uint32_t n = w.counts[b];
-		const int q = b & 1;
-		for (std::uint32_t i = blockIdx.x * kWaveBlock + threadIdx.x; i < n; i += gridDim.x * kWaveBlock)
-		{
-			const std::uint32_t path = w.pathOf(w.qPath[q][i]);
-			float4 r4 = w.radiance[path];
-			std::uint32_t flags = __float_as_uint(r4.w);
-			f3 acc = mk(r4.x, r4.y, r4.z);
-			if (flags & PF_CONN_LIGHT)
-			{
-				if (w.visible[2 * path])
-				{
-					const float4 c = w.connection[2 * path];
-					acc = acc + clampRay(mk(c.x, c.y, c.z));
-				}
-			}
-			if (flags & PF_CONN_ENV)
-			{
-				if (w.visible[2 * path + 1])
-				{
-					const float4 c = w.connection[2 * path + 1];
-					acc = acc + clampRay(mk(c.x, c.y, c.z));
-				}
-			}
-			if (flags & PF_DONE)
-			{
-				const f3 c = cleanColor(acc);
-				float* out = sampleColors + static_cast<size_t>(path) * 3;
-				out[0] = c.x;
-				out[1] = c.y;
-				out[2] = c.z;
-			}
-			else
-			{
-				flags &= (PF_PREV_SPECULAR | PF_PREV_INFINITE);
-				w.radiance[path] = make_float4(acc.x, acc.y, acc.z, __uint_as_float(flags));
-			}
-		}
-	}
-
 	// Adds a pass's sample colours of one scene into its FP64 pixel sums, in sample order
 	// (the per-pixel sum of _threadRender, Threads.cpp:551-583), and in adaptive rounds into
 	// the pixel's AdaptiveAccumulator (Threads.cpp:571-576).
-	__global__ void	wf_accumulate(const float* __restrict__ colors, const PassJob* jobs, std::uint32_t job)
+	static __global__ void	wf_accumulate(WaveBuffers w, const float* __restrict__ colors, const PassJob* jobs, std::uint32_t job)
 	{
 		const PassJob& J = jobs[job];
 		const std::uint32_t count = J.params.sampleCount;
@@ -837,8 +883,10 @@ namespace luzgpu
 				for (std::uint32_t k = 0; k < count; k++)
 				{
 					const size_t g = static_cast<size_t>(J.pathBase) + static_cast<size_t>(k) * J.pixels + i;
-					denoiseAddSample(a, colors + 3 * g, J.features + kNforFeatures * g, ((J.params.sampleBegin + k) & 1u) != 0u);
-					if (J.moments) adaptiveAdd(m, colors[3 * g], colors[3 * g + 1], colors[3 * g + 2]);
+					float c[3];
+					pathColor(w, colors, g, c);
+					denoiseAddSample(a, c, J.features + kNforFeatures * g, ((J.params.sampleBegin + k) & 1u) != 0u);
+					if (J.moments) adaptiveAdd(m, c[0], c[1], c[2]);
 				}
 				for (int j = 0; j < kDenoiseStats; j++) J.denoise[kDenoiseStats * px + j] = a[j];
 				if (J.moments)
@@ -859,7 +907,8 @@ namespace luzgpu
 			}
 			for (std::uint32_t k = 0; k < count; k++)
 			{
-				const float* c = colors + (static_cast<size_t>(J.pathBase) + static_cast<size_t>(k) * J.pixels + i) * 3;
+				float c[3];
+				pathColor(w, colors, static_cast<size_t>(J.pathBase) + static_cast<size_t>(k) * J.pixels + i, c);
 				const double cr = c[0], cg = c[1], cb = c[2];
 				r += cr;
 				g += cg;
@@ -1078,9 +1127,24 @@ namespace luzgpu
 		if (e != hipSuccess) throw std::runtime_error(std::string(what) + ": " + hipGetErrorString(e));
 	}
 
+	// Calls f with the scene's feature class as a compile-time constant.
+	template <typename F>
+	inline void	withFeatures(int features, F&& f)
+	{
+		switch (featureClass(features))
+		{
+			case 0: f.template operator()<0>(); break;
+			case kFeatAnalytic: f.template operator()<kFeatAnalytic>(); break;
+			case kFeatMedia: f.template operator()<kFeatMedia>(); break;
+			case kFeatRich: f.template operator()<kFeatRich>(); break;
+			case kFeatAll: f.template operator()<kFeatAll>(); break;
+			default: f.template operator()<kFeatEvery>(); break;
+		}
+	}
+
 	// Enqueues the launches of one pass (the table is already in st.jobs).
 	template <int Feat>
-	inline void	enqueuePassF(WavefrontState& st, const SceneView& s, std::uint32_t jobCount, int maxBounces, bool volumes,
+	void	enqueuePassF(WavefrontState& st, const SceneView& s, std::uint32_t jobCount, int maxBounces, bool volumes,
 		unsigned long long* counters, hipStream_t stream, bool count, WaveTuning tune, std::vector<hipEvent_t>* marks)
 	{
 		const WaveBuffers& w = st.buf;
@@ -1104,32 +1168,37 @@ namespace luzgpu
 			else if (tune.ldsStack == 24) wf_extend<false, T, 24><<<tune.grid, kWaveBlock, 0, stream>>>(s, st.jobs, w, b, counters, tune.extendRefill, ch);
 			else wf_extend<false, T, 16><<<tune.grid, kWaveBlock, 0, stream>>>(s, st.jobs, w, b, counters, tune.extendRefill, ch);
 			mark();
-			wf_shade<Feat><<<kWaveGrid, kWaveBlock, 0, stream>>>(s, st.jobs, w, b, vol);
+			if (jobCount > 1u) wf_shade<Feat, true><<<kWaveGrid, kWaveBlock, 0, stream>>>(s, st.jobs, w, b, vol, st.colors);
+			else wf_shade<Feat, false><<<kWaveGrid, kWaveBlock, 0, stream>>>(s, st.jobs, w, b, vol, st.colors);
 			mark();
 			if (count) wf_shadow<true, T, kWaveLdsStack><<<tune.grid, kWaveBlock, 0, stream>>>(s, st.jobs, w, b, counters, tune.shadowRefill, ch, vol);
 			else if (tune.ldsStack == 8) wf_shadow<false, T, 8><<<tune.grid, kWaveBlock, 0, stream>>>(s, st.jobs, w, b, counters, tune.shadowRefill, ch, vol);
 			else if (tune.ldsStack == 24) wf_shadow<false, T, 24><<<tune.grid, kWaveBlock, 0, stream>>>(s, st.jobs, w, b, counters, tune.shadowRefill, ch, vol);
 			else wf_shadow<false, T, 16><<<tune.grid, kWaveBlock, 0, stream>>>(s, st.jobs, w, b, counters, tune.shadowRefill, ch, vol);
 			mark();
-			wf_resolve<<<kWaveGrid, kWaveBlock, 0, stream>>>(w, b, st.colors);
 		}
 		for (std::uint32_t j = 0; j < jobCount; j++)
 		{
-			wf_accumulate<<<1024, 256, 0, stream>>>(st.colors, st.jobs, j);
+			wf_accumulate<<<1024, 256, 0, stream>>>(w, st.colors, st.jobs, j);
 		}
 	}
+
+#ifndef LUZ_FEATURES
+	// enqueuePassF is instantiated per scene feature class in features.hip
+	#define LUZ_PASS(F) extern template void enqueuePassF<F>(WavefrontState&, const SceneView&, std::uint32_t, int, bool, \
+		unsigned long long*, hipStream_t, bool, WaveTuning, std::vector<hipEvent_t>*);
+	LUZ_PASS(0)
+	LUZ_PASS(kFeatAnalytic)
+	LUZ_PASS(kFeatMedia)
+	LUZ_PASS(kFeatRich)
+	LUZ_PASS(kFeatAll)
+	LUZ_PASS(kFeatEvery)
+	#undef LUZ_PASS
 
 	inline void	enqueuePass(int features, WavefrontState& st, const SceneView& s, std::uint32_t jobCount, int maxBounces, bool volumes,
 		unsigned long long* counters, hipStream_t stream, bool count, WaveTuning tune, std::vector<hipEvent_t>* marks)
 	{
-		switch (features & kFeatEvery)
-		{
-			case kFeatEvery: enqueuePassF<kFeatEvery>(st, s, jobCount, maxBounces, volumes, counters, stream, count, tune, marks); break;
-			case 0: enqueuePassF<0>(st, s, jobCount, maxBounces, volumes, counters, stream, count, tune, marks); break;
-			case kFeatAnalytic: enqueuePassF<kFeatAnalytic>(st, s, jobCount, maxBounces, volumes, counters, stream, count, tune, marks); break;
-			case kFeatRich: enqueuePassF<kFeatRich>(st, s, jobCount, maxBounces, volumes, counters, stream, count, tune, marks); break;
-			default: enqueuePassF<kFeatAll>(st, s, jobCount, maxBounces, volumes, counters, stream, count, tune, marks); break;
-		}
+		withFeatures(features, [&]<int F>() { enqueuePassF<F>(st, s, jobCount, maxBounces, volumes, counters, stream, count, tune, marks); });
 	}
 
 	// Renders every job's sample range into its sums: passes of at most kMaxPassPaths paths
@@ -1186,6 +1255,8 @@ namespace luzgpu
 				pj.params.sampleCount = c;
 				pj.pathBase = base;
 				pj.pixels = pixels;
+				pj.pixelsInverse = inverseOf(pixels);
+				pj.widthInverse = inverseOf(p.width);
 				pj.sums = jobs[j].sums;
 				pj.pixelList = jobs[j].pixelList;
 				pj.moments = jobs[j].moments;
@@ -1280,4 +1351,5 @@ namespace luzgpu
 			}
 		}
 	}
+#endif
 }

@@ -1615,17 +1615,24 @@ namespace luzgpu
 		p.features = 0;
 		for (const Hittable& h : scene.hittables)
 		{
-			if (h.kind == HIT_SPHERE || h.kind == HIT_CUBE || h.kind == HIT_VOLUME || h.kind == HIT_PLANE || h.kind == HIT_DIRECTIONAL
-				|| (h.kind == HIT_INSTANCE && scene.materials[h.material].kind == MAT_EMISSIVE))
+			if (h.kind == HIT_SPHERE || h.kind == HIT_CUBE || h.kind == HIT_VOLUME || h.kind == HIT_PLANE || h.kind == HIT_DIRECTIONAL)
 			{
 				p.features |= kFeatAnalytic;	// the class of rarer primitives and lights
+			}
+			if (h.kind == HIT_INSTANCE && scene.materials[h.material].kind == MAT_EMISSIVE)
+			{
+				p.features |= kFeatAll;	// a light pdf that traverses its mesh lives in the rich kernels
 			}
 		}
 		for (const Material& m : scene.materials)
 		{
-			if (m.kind == MAT_GLOSSY || m.kind == MAT_DIFFUSE_GLOSSY || m.kind == MAT_PRINCIPLED || m.kind == MAT_ISOTROPIC || m.kind == MAT_HG)
+			if (m.kind == MAT_GLOSSY || m.kind == MAT_DIFFUSE_GLOSSY || m.kind == MAT_PRINCIPLED)
 			{
 				p.features |= kFeatRich;
+			}
+			if (m.kind == MAT_ISOTROPIC || m.kind == MAT_HG)
+			{
+				p.features |= kFeatPhase;
 			}
 			if (m.kind == MAT_PRINCIPLED && m.subsurface > 0.0 && !m.subsurfaceThin)
 			{

@@ -11,8 +11,8 @@
 
 #include "../../include/luzgpu.h"
 #include "common/layout.h"
-#include "device/adjoint.hpp"
 #include "device/integrator.hpp"
+#include "device/mega.hpp"
 #include "device/nfor.hpp"
 #include "device/post.hpp"
 #include "device/wavefront.hpp"
@@ -137,10 +137,8 @@ namespace luzgpu
 		unsigned long long	shadowRays;
 	};
 
-	constexpr int	kMegaBlock = 128;
 	constexpr std::uint32_t	kMaxImageSide = 65536;
 	constexpr std::uint64_t	kMaxImagePixels = 1ull << 28;
-	constexpr int	kStackDepth = 48;
 
 	// Device memory of luzgpu_render_noalloc, which allocates nothing: one fixed array per
 	// device, held until the process ends. Layout: 8 ray / visit counters, the FP64 pixel
@@ -157,138 +155,28 @@ namespace luzgpu
 
 	static __device__ __align__(256) unsigned char	scratch[kNoAllocScratchBytes];
 
-	// counters: [0] closest-hit rays, [1] shadow rays, [2] nodes visited, [3] primitives tested.
-	// Renders samples [sampleBegin, sampleBegin + sampleCount) of `pixels` pixels: entries of
-	// `list` (adaptive rounds), or the whole image when `list` is nullptr.
-	template <bool Count, int Feat>
-	__global__ __launch_bounds__(kMegaBlock) void	render_mega(SceneView s, GpuParams p, const std::uint32_t* __restrict__ list,
-		std::uint32_t pixels, float* __restrict__ sampleColors, unsigned long long* __restrict__ counters)
-	{
-		__shared__ std::uint32_t stackMem[kStackDepth * kMegaBlock];
-		const std::uint64_t gid = static_cast<std::uint64_t>(blockIdx.x) * kMegaBlock + threadIdx.x;
-		std::uint32_t closest = 0, shadow = 0;
-		VisitCounter visits{0u, 0u};
-		if (gid < static_cast<std::uint64_t>(pixels) * p.sampleCount)
-		{
-			const std::uint32_t slot = static_cast<std::uint32_t>(gid / pixels);
-			const std::uint32_t entry = static_cast<std::uint32_t>(gid % pixels);
-			const std::uint32_t pixel = list ? list[entry] : entry;
-			LdsStack<kStackDepth, kMegaBlock> stack{stackMem + threadIdx.x, 0};
-			const f3 c = cleanColor(tracePath<Count, Feat>(s, p, pixel % p.width, pixel / p.width, p.sampleBegin + slot, stack, closest, shadow, visits));
-			float* out = sampleColors + (static_cast<size_t>(slot) * pixels + entry) * 3;
-			out[0] = c.x;
-			out[1] = c.y;
-			out[2] = c.z;
-		}
-		// one atomic per wave for the ray counters
-		for (int off = 32; off > 0; off >>= 1)
-		{
-			closest += __shfl_down(closest, off);
-			shadow += __shfl_down(shadow, off);
-			if (Count)
-			{
-				visits.nodes += __shfl_down(visits.nodes, off);
-				visits.prims += __shfl_down(visits.prims, off);
-			}
-		}
-		if ((threadIdx.x & 63) == 0)
-		{
-			atomicAdd(counters + 0, static_cast<unsigned long long>(closest));
-			atomicAdd(counters + 1, static_cast<unsigned long long>(shadow));
-			if (Count)
-			{
-				atomicAdd(counters + 2, static_cast<unsigned long long>(visits.nodes));
-				atomicAdd(counters + 3, static_cast<unsigned long long>(visits.prims));
-			}
-		}
-	}
-
-	template <bool Count>
-	void	launchMegaC(int features, size_t grid, hipStream_t st, const SceneView& s, const GpuParams& p, const std::uint32_t* list,
-		std::uint32_t pixels, float* colors, unsigned long long* counters)
-	{
-		switch (features & kFeatEvery)
-		{
-			case kFeatEvery: render_mega<Count, kFeatEvery><<<grid, kMegaBlock, 0, st>>>(s, p, list, pixels, colors, counters); break;
-			case 0: render_mega<Count, 0><<<grid, kMegaBlock, 0, st>>>(s, p, list, pixels, colors, counters); break;
-			case kFeatAnalytic: render_mega<Count, kFeatAnalytic><<<grid, kMegaBlock, 0, st>>>(s, p, list, pixels, colors, counters); break;
-			case kFeatRich: render_mega<Count, kFeatRich><<<grid, kMegaBlock, 0, st>>>(s, p, list, pixels, colors, counters); break;
-			default: render_mega<Count, kFeatAll><<<grid, kMegaBlock, 0, st>>>(s, p, list, pixels, colors, counters); break;
-		}
-	}
+	// instantiated per scene feature class in features.hip
+	#define LUZ_MEGA(F) \
+		extern template void launchMegaF<F>(bool, size_t, hipStream_t, const SceneView&, const GpuParams&, const std::uint32_t*, std::uint32_t, \
+			float*, unsigned long long*); \
+		extern template void launchMegaBatchF<F>(bool, size_t, hipStream_t, const SceneView&, const MegaJob*, std::uint32_t, float*, \
+			unsigned long long*); \
+		extern template void launchMegaDenoiseF<F>(size_t, hipStream_t, const SceneView&, const GpuParams&, const std::uint32_t*, std::uint32_t, \
+			float*, float*, unsigned long long*); \
+		extern template void launchAdjointF<F>(size_t, size_t, hipStream_t, const SceneView&, const GpuParams&, const float*, double*, \
+			std::uint32_t);
+	LUZ_MEGA(0)
+	LUZ_MEGA(kFeatAnalytic)
+	LUZ_MEGA(kFeatMedia)
+	LUZ_MEGA(kFeatRich)
+	LUZ_MEGA(kFeatAll)
+	LUZ_MEGA(kFeatEvery)
+	#undef LUZ_MEGA
 
 	void	launchMega(bool count, int features, size_t grid, hipStream_t st, const SceneView& s, const GpuParams& p,
 		const std::uint32_t* list, std::uint32_t pixels, float* colors, unsigned long long* counters)
 	{
-		if (count) launchMegaC<true>(features, grid, st, s, p, list, pixels, colors, counters);
-		else launchMegaC<false>(features, grid, st, s, p, list, pixels, colors, counters);
-	}
-
-	// One scene of a batched plain-kernel launch. Its (pixel, sample) threads start on a wave
-	// boundary, so every wave renders one scene and reads that scene's parameters with
-	// scalar loads.
-	struct	MegaJob
-	{
-		GpuParams	params;			// sampleBegin / sampleCount: this launch's slice
-		std::uint32_t	firstWave;	// first wave of the slice in the launch
-		std::uint32_t	pixels;
-		std::uint32_t	count;		// pixels * sampleCount
-		std::uint32_t	pixelBase;	// first pixel of the scene in the launch's pixel numbering
-		std::uint64_t	colorBase;	// first sample colour of the slice
-		double*	sums;			// the scene's FP64 pixel sums
-	};
-
-	// Several scenes in one launch (render_batch on the plain kernel): small scenes that
-	// cannot fill the GPU alone run side by side, each path still in one thread.
-	template <bool Count, int Feat>
-	__global__ __launch_bounds__(kMegaBlock) void	render_mega_batch(SceneView s, const MegaJob* __restrict__ jobs, std::uint32_t jobCount,
-		float* __restrict__ sampleColors, unsigned long long* __restrict__ counters)
-	{
-		__shared__ std::uint32_t stackMem[kStackDepth * kMegaBlock];
-		const std::uint32_t wave = __builtin_amdgcn_readfirstlane((blockIdx.x * kMegaBlock + threadIdx.x) >> 6);
-		std::uint32_t lo = 0, hi = jobCount;
-		while (hi - lo > 1u)
-		{
-			const std::uint32_t mid = (lo + hi) >> 1;
-			if (jobs[mid].firstWave <= wave) lo = mid;
-			else hi = mid;
-		}
-		const MegaJob& J = jobs[__builtin_amdgcn_readfirstlane(lo)];
-		const std::uint32_t local = (wave - J.firstWave) * 64u + (threadIdx.x & 63u);
-		std::uint32_t closest = 0, shadow = 0;
-		VisitCounter visits{0u, 0u};
-		if (wave >= J.firstWave && local < J.count)
-		{
-			const GpuParams& p = J.params;
-			const std::uint32_t slot = local / J.pixels, pixel = local % J.pixels;
-			LdsStack<kStackDepth, kMegaBlock> stack{stackMem + threadIdx.x, 0};
-			const f3 c = cleanColor(tracePath<Count, Feat>(s, p, pixel % p.width, pixel / p.width, p.sampleBegin + slot, stack, closest,
-				shadow, visits));
-			float* out = sampleColors + (J.colorBase + local) * 3;
-			out[0] = c.x;
-			out[1] = c.y;
-			out[2] = c.z;
-		}
-		for (int off = 32; off > 0; off >>= 1)
-		{
-			closest += __shfl_down(closest, off);
-			shadow += __shfl_down(shadow, off);
-			if (Count)
-			{
-				visits.nodes += __shfl_down(visits.nodes, off);
-				visits.prims += __shfl_down(visits.prims, off);
-			}
-		}
-		if ((threadIdx.x & 63) == 0)
-		{
-			atomicAdd(counters + 0, static_cast<unsigned long long>(closest));
-			atomicAdd(counters + 1, static_cast<unsigned long long>(shadow));
-			if (Count)
-			{
-				atomicAdd(counters + 2, static_cast<unsigned long long>(visits.nodes));
-				atomicAdd(counters + 3, static_cast<unsigned long long>(visits.prims));
-			}
-		}
+		withFeatures(features, [&]<int F>() { launchMegaF<F>(count, grid, st, s, p, list, pixels, colors, counters); });
 	}
 
 	// Adds a batched launch's sample colours into every scene's FP64 pixel sums, in sample
@@ -320,68 +208,22 @@ namespace luzgpu
 		J.sums[3 * static_cast<size_t>(px) + 2] = b;
 	}
 
-	template <bool Count>
-	void	launchMegaBatchC(int features, size_t grid, hipStream_t st, const SceneView& s, const MegaJob* jobs, std::uint32_t n,
+	void	launchMegaBatch(bool count, int features, size_t grid, hipStream_t st, const SceneView& s, const MegaJob* jobs, std::uint32_t n,
 		float* colors, unsigned long long* counters)
 	{
-		switch (features & kFeatEvery)
-		{
-			case kFeatEvery: render_mega_batch<Count, kFeatEvery><<<grid, kMegaBlock, 0, st>>>(s, jobs, n, colors, counters); break;
-			case 0: render_mega_batch<Count, 0><<<grid, kMegaBlock, 0, st>>>(s, jobs, n, colors, counters); break;
-			case kFeatAnalytic: render_mega_batch<Count, kFeatAnalytic><<<grid, kMegaBlock, 0, st>>>(s, jobs, n, colors, counters); break;
-			case kFeatRich: render_mega_batch<Count, kFeatRich><<<grid, kMegaBlock, 0, st>>>(s, jobs, n, colors, counters); break;
-			default: render_mega_batch<Count, kFeatAll><<<grid, kMegaBlock, 0, st>>>(s, jobs, n, colors, counters); break;
-		}
-	}
-
-	// The plain kernel with denoising on: each (pixel, sample) also writes its primary
-	// features (kNforFeatures floats, RenderSample of _calculatePixelSample, ColorHelper.cpp:1119-1126).
-	template <int Feat>
-	__global__ __launch_bounds__(kMegaBlock) void	render_mega_denoise(SceneView s, GpuParams p, const std::uint32_t* __restrict__ list,
-		std::uint32_t pixels, float* __restrict__ sampleColors, float* __restrict__ sampleFeatures, unsigned long long* __restrict__ counters)
-	{
-		__shared__ std::uint32_t stackMem[kStackDepth * kMegaBlock];
-		const std::uint64_t gid = static_cast<std::uint64_t>(blockIdx.x) * kMegaBlock + threadIdx.x;
-		std::uint32_t closest = 0, shadow = 0;
-		VisitCounter visits{0u, 0u};
-		if (gid < static_cast<std::uint64_t>(pixels) * p.sampleCount)
-		{
-			const std::uint32_t slot = static_cast<std::uint32_t>(gid / pixels);
-			const std::uint32_t entry = static_cast<std::uint32_t>(gid % pixels);
-			const std::uint32_t pixel = list ? list[entry] : entry;
-			LdsStack<kStackDepth, kMegaBlock> stack{stackMem + threadIdx.x, 0};
-			float f[kNforFeatures];
-			const f3 c = cleanColor(tracePath<false, Feat>(s, p, pixel % p.width, pixel / p.width, p.sampleBegin + slot, stack, closest,
-				shadow, visits, static_cast<NoAdjoint*>(nullptr), f));
-			const size_t k = static_cast<size_t>(slot) * pixels + entry;
-			sampleColors[3 * k] = c.x;
-			sampleColors[3 * k + 1] = c.y;
-			sampleColors[3 * k + 2] = c.z;
-			for (int j = 0; j < kNforFeatures; j++) sampleFeatures[kNforFeatures * k + j] = f[j];
-		}
-		for (int off = 32; off > 0; off >>= 1)
-		{
-			closest += __shfl_down(closest, off);
-			shadow += __shfl_down(shadow, off);
-		}
-		if ((threadIdx.x & 63) == 0)
-		{
-			if (closest) atomicAdd(counters + 0, static_cast<unsigned long long>(closest));
-			if (shadow) atomicAdd(counters + 1, static_cast<unsigned long long>(shadow));
-		}
+		withFeatures(features, [&]<int F>() { launchMegaBatchF<F>(count, grid, st, s, jobs, n, colors, counters); });
 	}
 
 	void	launchMegaDenoise(int features, size_t grid, hipStream_t st, const SceneView& s, const GpuParams& p, const std::uint32_t* list,
 		std::uint32_t pixels, float* colors, float* feats, unsigned long long* counters)
 	{
-		switch (features & kFeatEvery)
-		{
-			case kFeatEvery: render_mega_denoise<kFeatEvery><<<grid, kMegaBlock, 0, st>>>(s, p, list, pixels, colors, feats, counters); break;
-			case 0: render_mega_denoise<0><<<grid, kMegaBlock, 0, st>>>(s, p, list, pixels, colors, feats, counters); break;
-			case kFeatAnalytic: render_mega_denoise<kFeatAnalytic><<<grid, kMegaBlock, 0, st>>>(s, p, list, pixels, colors, feats, counters); break;
-			case kFeatRich: render_mega_denoise<kFeatRich><<<grid, kMegaBlock, 0, st>>>(s, p, list, pixels, colors, feats, counters); break;
-			default: render_mega_denoise<kFeatAll><<<grid, kMegaBlock, 0, st>>>(s, p, list, pixels, colors, feats, counters); break;
-		}
+		withFeatures(features, [&]<int F>() { launchMegaDenoiseF<F>(grid, st, s, p, list, pixels, colors, feats, counters); });
+	}
+
+	void	launchAdjoint(int features, size_t grid, size_t shmem, hipStream_t st, const SceneView& s, const GpuParams& p,
+		const float* dLdI, double* grads, std::uint32_t materialCount)
+	{
+		withFeatures(features & ~kFeatSubsurface, [&]<int F>() { launchAdjointF<F>(grid, shmem, st, s, p, dLdI, grads, materialCount); });
 	}
 
 	// `list` / `pixels`: as render_mega_denoise; `moments` (adaptive rounds, or nullptr):
@@ -455,57 +297,6 @@ namespace luzgpu
 			featA[kNforFeatures * i + j] = nA == 0u ? fallback : a[12 + j] / static_cast<double>(nA);
 			featB[kNforFeatures * i + j] = nB == 0u ? fallback : a[12 + kNforFeatures + j] / static_cast<double>(nB);
 			featVariance[kNforFeatures * i + j] = sampleMeanVariance(a[12 + 2 * kNforFeatures + j], a[12 + 3 * kNforFeatures + j], n);
-		}
-	}
-
-	// Path-replay adjoint, one thread per (pixel, sample): dLdI is dLoss/dImage (W*H*3),
-	// grads receives kGradPerMaterial FP64 sums per material.
-	template <int Feat>
-	__global__ __launch_bounds__(kMegaBlock) void	adjoint_mega(SceneView s, GpuParams p, const float* __restrict__ dLdI,
-		double* __restrict__ grads, std::uint32_t materialCount)
-	{
-		__shared__ std::uint32_t stackMem[kStackDepth * kMegaBlock];
-		extern __shared__ float ldsGrads[];
-		const std::uint32_t n = materialCount * kGradPerMaterial;
-		for (std::uint32_t i = threadIdx.x; i < n; i += kMegaBlock) ldsGrads[i] = 0.0f;
-		__syncthreads();
-		const std::uint32_t pixels = p.width * p.height;
-		const size_t id = static_cast<size_t>(blockIdx.x) * kMegaBlock + threadIdx.x;
-		if (id < static_cast<size_t>(pixels) * p.sampleCount)
-		{
-			const std::uint32_t pixel = static_cast<std::uint32_t>(id % pixels), slot = static_cast<std::uint32_t>(id / pixels);
-			LdsStack<kStackDepth, kMegaBlock> stack{stackMem + threadIdx.x, 0};
-			AdjointRecorder rec;
-			rec.grads = ldsGrads;
-			rec.count = 0;
-			rec.pendingMaterial = -1;
-			rec.pendingScale = 0.0f;
-			rec.materials = s.materials;
-			const float inv = 1.0f / static_cast<float>(p.sampleCount);
-			rec.weight = mk(dLdI[3 * static_cast<size_t>(pixel)] * inv, dLdI[3 * static_cast<size_t>(pixel) + 1] * inv,
-				dLdI[3 * static_cast<size_t>(pixel) + 2] * inv);
-			std::uint32_t closest = 0, shadow = 0;
-			VisitCounter visits{0u, 0u};
-			const f3 L = tracePath<false, Feat>(s, p, pixel % p.width, pixel / p.width, p.sampleBegin + slot, stack, closest, shadow,
-				visits, &rec);
-			rec.finish(L);
-		}
-		__syncthreads();
-		for (std::uint32_t i = threadIdx.x; i < n; i += kMegaBlock)
-		{
-			if (ldsGrads[i] != 0.0f) atomicAdd(grads + i, static_cast<double>(ldsGrads[i]));
-		}
-	}
-
-	void	launchAdjoint(int features, size_t grid, size_t shmem, hipStream_t st, const SceneView& s, const GpuParams& p,
-		const float* dLdI, double* grads, std::uint32_t materialCount)
-	{
-		switch (features & kFeatAll)
-		{
-			case 0: adjoint_mega<0><<<grid, kMegaBlock, shmem, st>>>(s, p, dLdI, grads, materialCount); break;
-			case kFeatAnalytic: adjoint_mega<kFeatAnalytic><<<grid, kMegaBlock, shmem, st>>>(s, p, dLdI, grads, materialCount); break;
-			case kFeatRich: adjoint_mega<kFeatRich><<<grid, kMegaBlock, shmem, st>>>(s, p, dLdI, grads, materialCount); break;
-			default: adjoint_mega<kFeatAll><<<grid, kMegaBlock, shmem, st>>>(s, p, dLdI, grads, materialCount); break;
 		}
 	}
 
@@ -2213,16 +2004,8 @@ int	luzgpu_render_batch(luzgpu_ctx* ctx, uint32_t n, luzgpu_scene* const* scenes
 				check(hipMemcpyAsync(ctx->megaJobs.ptr, table.data(), table.size() * sizeof(MegaJob), hipMemcpyHostToDevice, st),
 					"batch job table");
 				const size_t grid = (static_cast<size_t>(waves) * 64 + kMegaBlock - 1) / kMegaBlock;
-				if (settings[0].count_visits)
-				{
-					launchMegaBatchC<true>(ctx->batch->host.features, grid, st, ctx->batch->view, ctx->megaJobs.as<MegaJob>(), n,
-						ctx->sampleColors.as<float>(), ctx->counters.as<unsigned long long>());
-				}
-				else
-				{
-					launchMegaBatchC<false>(ctx->batch->host.features, grid, st, ctx->batch->view, ctx->megaJobs.as<MegaJob>(), n,
-						ctx->sampleColors.as<float>(), ctx->counters.as<unsigned long long>());
-				}
+				launchMegaBatch(settings[0].count_visits != 0, ctx->batch->host.features, grid, st, ctx->batch->view,
+					ctx->megaJobs.as<MegaJob>(), n, ctx->sampleColors.as<float>(), ctx->counters.as<unsigned long long>());
 				check(hipGetLastError(), "batch render launch");
 				accumulate_batch<<<blocks(totalPixels, 256), 256, 0, st>>>(ctx->sampleColors.as<float>(), ctx->megaJobs.as<MegaJob>(), n,
 					totalPixels);
