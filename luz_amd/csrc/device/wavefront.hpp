@@ -47,6 +47,33 @@ namespace luzgpu
 	constexpr std::uint32_t	PF_CONN_LIGHT = 8u;	// a light connection is pending
 	constexpr std::uint32_t	PF_CONN_ENV = 16u;	// an environment connection is pending
 
+	// A value that all lanes of the wave hold, as a scalar.
+	__device__ __forceinline__ std::uint32_t	uniform(std::uint32_t v) { return __builtin_amdgcn_readfirstlane(v); }
+
+	constexpr int	kMaxBounceSlots = 64;
+	// A queue is eight parts, each with its own counters: the camera rays go to the parts tile by
+	// tile, a path stays in its part, and blocks k, k + 8, ... work on part k. Appends and claims
+	// on one counter queue up behind each other at about 12 ns each however many waves there
+	// are, which bounded every launch of short rays. Eight also follow the eight XCDs that blocks
+	// are dealt to in turn, so a part stays within one XCD's L2. One part -> eight: traversal of
+	// the material test scene at 641x479, 17 samples 2.0 -> 0.8 ms, of the 300x300 box at 50
+	// samples 4.6 -> 2.7 ms, of an uneven 16-scene batch 10.1 -> 7.7 ms (its shade 6.9 -> 6.1 ms).
+	// Tiles are 512 paths: with 64, a shade block's paths lie in four places of the image and
+	// spheres at 1080p shades in 10.1 instead of 8.6 ms; from 512 to 4096 the times are level,
+	// and small passes spread best over the smallest.
+	constexpr std::uint32_t	kQueueParts = 8;
+	constexpr std::uint32_t	kPartTile = 512;	// paths, a multiple of 64
+	constexpr std::uint32_t	kCounterStride = 64;	// words between counters: lines of their own
+	enum : int { COUNT_RAYS = 0, COUNT_SHADOW = 1, CLAIM_EXTEND = 2, CLAIM_SHADOW = 3, kCounterKinds = 4 };
+	constexpr std::uint32_t	kCounterWords = kCounterKinds * kMaxBounceSlots * kQueueParts * kCounterStride;
+
+	// The part of tile t: each row of kQueueParts tiles gives every part one, turned by a hash of
+	// the row so that no part follows a column of the image.
+	__host__ __device__ __forceinline__ std::uint32_t	partOfTile(std::uint32_t t)
+	{
+		return (t + ((t / kQueueParts * 0x9e3779b1u) >> 29)) % kQueueParts;
+	}
+
 	struct	WaveBuffers
 	{
 		// queue-ordered (double-buffered by bounce parity)
@@ -67,9 +94,7 @@ namespace luzgpu
 		float4*	sDir;		// xyz, w = scene << 25 | (2 * path + slot) (bits)
 		float*	sLogU;		// volume free-flight sample of the shadow ray (batches with volumes)
 		int2*	sFrom;		// RayOrigin of the shadow ray (hittable bits, tri)
-		// counters: [b] rays in queue b, [kMaxBounceSlots + b] shadow rays of bounce b,
-		// [2 * kMaxBounceSlots + b] / [3 * ...] extend / shadow work claims
-		std::uint32_t*	counts;
+		std::uint32_t*	counts;		// see counter(); then the pass's path count and the part stride
 		std::uint32_t	capacity;
 		std::uint32_t*	spill;		// traversal stack spill, [entry][grid thread]
 		// Queued extension rays carry their scene above the global path id in qPath
@@ -77,6 +102,15 @@ namespace luzgpu
 		// (scene << (pathBits + 1) | 2 * path + slot). pathBits = 31 - the bits of the largest
 		// scene index of the render: 31 for one scene, 24 for 127.
 		std::uint32_t	pathBits;
+
+		// Counter `kind` of bounce b and queue part `part` (see kQueueParts).
+		__device__ __forceinline__ std::uint32_t*	counter(int kind, int b, std::uint32_t part) const
+		{
+			return counts + ((static_cast<std::uint32_t>(kind) * kMaxBounceSlots + static_cast<std::uint32_t>(b)) * kQueueParts + part) * kCounterStride;
+		}
+		__device__ __forceinline__ std::uint32_t	pathCount() const { return counts[kCounterWords]; }
+		// queue entries of a part: [part * partStride(), + its count); shadow rays at twice that
+		__device__ __forceinline__ std::uint32_t	partStride() const { return counts[kCounterWords + 1]; }
 
 		__device__ __forceinline__ std::uint32_t	sceneOfPath(std::uint32_t qp) const { return qp >> pathBits; }
 		__device__ __forceinline__ std::uint32_t	pathOf(std::uint32_t qp) const { return qp & ((1u << pathBits) - 1u); }
@@ -187,7 +221,6 @@ namespace luzgpu
 	constexpr int	kWaveLdsStack = 16;		// default LDS stack entries per lane (tunable: 8, 16, 24)
 	constexpr int	kWaveLdsStackMin = 8;
 	constexpr int	kWaveStackCapacity = 64;
-	constexpr int	kMaxBounceSlots = 64;
 	constexpr unsigned	kWaveGrid = 2048;	// 256 CUs x 8 waves per SIMD x 4 SIMDs / 4 waves per block
 	// default traversal launch shape: as many persistent waves as the traversal kernels'
 	// registers let every SIMD hold (256 CUs x 4 SIMDs x 5 waves / 4 waves per block; 2 %
@@ -212,18 +245,48 @@ namespace luzgpu
 
 	__device__ __forceinline__ std::uint32_t	laneId() { return threadIdx.x & 63u; }
 
-	// The pass's total path count: written into counts[0] (queue 0 holds every path).
-	static __global__ void	wf_zero_counts(std::uint32_t* counts, std::uint32_t n, const PassJob* jobs, std::uint32_t jobCount)
+	// Clears the pass's counters and sets its path count, the part stride and the parts' shares
+	// of queue 0, which holds every path: tile t of kPartTile paths is in part partOfTile(t).
+	static __global__ void	wf_zero_counts(WaveBuffers w, const PassJob* jobs, std::uint32_t jobCount)
 	{
-		const std::uint32_t i = threadIdx.x;
-		if (i < n)
+		const std::uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+		if (i >= kCounterWords / kCounterStride) return;
+		std::uint32_t first = 0;
+		if (i < kQueueParts)	// the parts of (COUNT_RAYS, bounce 0)
 		{
-			std::uint32_t first = 0;
+			std::uint32_t total = 0;
+			for (std::uint32_t j = 0; j < jobCount; j++) total += jobs[j].pixels * jobs[j].params.sampleCount;
+			const std::uint32_t tiles = (total + kPartTile - 1u) / kPartTile, rows = tiles / kQueueParts;
+			first = kPartTile * rows;
+			for (std::uint32_t t = rows * kQueueParts; t < tiles; t++) first += partOfTile(t) == i ? kPartTile : 0u;
+			if (tiles > 0u && partOfTile(tiles - 1u) == i) first -= kPartTile * tiles - total;
 			if (i == 0)
 			{
-				for (std::uint32_t j = 0; j < jobCount; j++) first += jobs[j].pixels * jobs[j].params.sampleCount;
+				w.counts[kCounterWords] = total;
+				w.counts[kCounterWords + 1] = kPartTile * ((tiles + kQueueParts - 1u) / kQueueParts);
 			}
-			counts[i] = first;
+		}
+		w.counts[i * kCounterStride] = first;
+	}
+
+	// Adds a pass's traced rays (its queues' lengths) to the render's counters.
+	static __global__ void	wf_count_rays(WaveBuffers w, unsigned long long* counters)
+	{
+		unsigned long long rays = 0, shadow = 0;
+		for (std::uint32_t i = threadIdx.x; i < kMaxBounceSlots * kQueueParts; i += 64u)
+		{
+			rays += w.counts[i * kCounterStride];
+			shadow += w.counts[(kMaxBounceSlots * kQueueParts + i) * kCounterStride];
+		}
+		for (int off = 32; off > 0; off >>= 1)
+		{
+			rays += __shfl_down(rays, off);
+			shadow += __shfl_down(shadow, off);
+		}
+		if (threadIdx.x == 0)
+		{
+			counters[0] += rays;
+			counters[1] += shadow;
 		}
 	}
 
@@ -236,11 +299,11 @@ namespace luzgpu
 		return volumeLogU(p, ps);
 	}
 
-	// Camera rays of every job of the pass in one launch (queue 0 holds the pass's paths in
-	// job order, counts[0] of them).
+	// Camera rays of every job of the pass in one launch (the pass's paths in job order, tile by
+	// tile to the parts of queue 0).
 	static __global__ __launch_bounds__(kWaveBlock) void	wf_raygen(const PassJob* jobs, std::uint32_t jobCount, WaveBuffers w)
 	{
-		const std::uint32_t total = w.counts[0];
+		const std::uint32_t total = w.pathCount(), partStride = w.partStride();
 		for (std::uint32_t g = blockIdx.x * kWaveBlock + threadIdx.x; g < total; g += gridDim.x * kWaveBlock)
 		{
 			std::uint32_t lo = 0, hi = jobCount;	// the last job whose slice starts at or before g
@@ -254,7 +317,7 @@ namespace luzgpu
 			const PassJob& J = jobs[job];
 			const GpuParams& p = J.params;
 			const std::uint32_t pixels = J.pixels;
-			// queue entry g holds the job's id-th camera ray; the queue visits the image in
+			// entry g is the job's id-th camera ray; the queue visits the image in
 			// bands of 8 rows, column by column, so a wave's 64 rays cover an 8 x 8 block
 			// (coherent first traversals). The path keeps its row-major id, which the later
 			// stages and the accumulation decode.
@@ -283,10 +346,12 @@ namespace luzgpu
 			ps.begin(p.renderSeed, x, y, p.sampleBegin + slot, sampleStream(p, p.sampleBegin + slot));
 			const Ray r = cameraRay(p, x, y, ps);
 			const float logU = p.hasVolumes ? volumeLogU(p, ps) : 0.0f;
-			w.qOrigin[0][g] = make_float4(r.o.x, r.o.y, r.o.z, logU);
-			w.qDir[0][g] = make_float4(r.d.x, r.d.y, r.d.z, __uint_as_float(kNoOrigin.hittable));
-			w.qFrom[0][g] = kNoOrigin.tri;
-			w.qPath[0][g] = w.queuedPath(job, path);
+			const std::uint32_t tile = g / kPartTile;
+			const std::uint32_t at = partOfTile(tile) * partStride + (tile / kQueueParts) * kPartTile + g % kPartTile;
+			w.qOrigin[0][at] = make_float4(r.o.x, r.o.y, r.o.z, logU);
+			w.qDir[0][at] = make_float4(r.d.x, r.d.y, r.d.z, __uint_as_float(kNoOrigin.hittable));
+			w.qFrom[0][at] = kNoOrigin.tri;
+			w.qPath[0][at] = w.queuedPath(job, path);
 			// the path's throughput and radiance start as constants the first shade stage
 			// supplies itself
 		}
@@ -302,6 +367,9 @@ namespace luzgpu
 		std::uint32_t	next;
 		std::uint32_t	end;
 		bool	drained;
+		std::uint32_t	first;	// the slots before this one were dealt without a claim
+
+		__device__ __forceinline__ bool	any() const { return !drained || next < end; }
 
 		// Gives every lane in `idle` (ballot mask) the next queue slot, in lane order; lanes
 		// left without one (queue exhausted) get 0xffffffff.
@@ -317,12 +385,18 @@ namespace luzgpu
 				next += want;
 				return slot;
 			}
+			if (drained)	// what is left of the last claim
+			{
+				slot = rank < avail ? next + rank : 0xffffffffu;
+				next = end;
+				return slot;
+			}
 			std::uint32_t c = 0;
 			if (laneId() == static_cast<std::uint32_t>(__ffsll(static_cast<long long>(idle)) - 1))
 			{
 				c = atomicAdd(fetch, chunk);
 			}
-			c = __builtin_amdgcn_readfirstlane(__shfl(c, __ffsll(static_cast<long long>(idle)) - 1));
+			c = first + __builtin_amdgcn_readfirstlane(__shfl(c, __ffsll(static_cast<long long>(idle)) - 1));
 			const std::uint32_t cEnd = c >= n ? c : min(c + chunk, n);
 			if (rank < avail) slot = next + rank;
 			else
@@ -344,28 +418,19 @@ namespace luzgpu
 		}
 	};
 
-	// counters: [0] closest rays, [1] shadow rays, [2]/[3] closest nodes/primitives,
-	// [4]/[5] shadow nodes/primitives (the last four only when Count)
-	__device__ __forceinline__ void	flushCounters(unsigned long long* counters, int slot, std::uint32_t rays,
-		VisitCounter visits, bool count)
+	// counters: [0] closest rays, [1] shadow rays (wf_count_rays), [2]/[3] closest
+	// nodes/primitives, [4]/[5] shadow nodes/primitives
+	__device__ __forceinline__ void	flushVisits(unsigned long long* counters, int slot, VisitCounter visits)
 	{
 		for (int off = 32; off > 0; off >>= 1)
 		{
-			rays += __shfl_down(rays, off);
-			if (count)
-			{
-				visits.nodes += __shfl_down(visits.nodes, off);
-				visits.prims += __shfl_down(visits.prims, off);
-			}
+			visits.nodes += __shfl_down(visits.nodes, off);
+			visits.prims += __shfl_down(visits.prims, off);
 		}
-		if (laneId() == 0 && rays)
+		if (laneId() == 0 && visits.nodes + visits.prims)
 		{
-			atomicAdd(counters + slot, static_cast<unsigned long long>(rays));
-			if (count)
-			{
-				atomicAdd(counters + 2 + 2 * slot, static_cast<unsigned long long>(visits.nodes));
-				atomicAdd(counters + 3 + 2 * slot, static_cast<unsigned long long>(visits.prims));
-			}
+			atomicAdd(counters + 2 + 2 * slot, static_cast<unsigned long long>(visits.nodes));
+			atomicAdd(counters + 3 + 2 * slot, static_cast<unsigned long long>(visits.prims));
 		}
 	}
 
@@ -376,31 +441,32 @@ namespace luzgpu
 	// turn has come, then the node code, then the pop they share, each once per wave.
 	// VALU-bound before the node test became a straight line (nodeStep): 1080p spheres extend
 	// 27.7 -> 18.9 ms, shadow 5.8 -> 3.5; 720p hazy terrain 50.9 -> 25.6 and 53.7 -> 26.7.
-	// Source supplies the queue: count(), load(slot, ray, tMax) and store(slot, state).
+	// Source supplies a queue part: load(slot, ray, tMax) and store(slot, state), `n` rays and the
+	// claim counter `fetch`.
 	template <bool AnyHit, bool Count, int Feat, int LdsDepth, typename Source>
-	__device__ __forceinline__ void	traceQueue(const SceneView& s, const PassJob* jobs, Source& src, std::uint32_t* fetch,
-		int refillAt, std::uint32_t maxChunk, unsigned long long* counters, int counterSlot)
+	__device__ __forceinline__ void	traceQueue(const SceneView& s, const PassJob* jobs, Source& src, std::uint32_t n, std::uint32_t* fetch,
+		std::uint32_t wave, std::uint32_t waves, int refillAt, std::uint32_t maxChunk, unsigned long long* counters, int counterSlot,
+		std::uint32_t* stackMem)
 	{
-		__shared__ std::uint32_t stackMem[LdsDepth * kWaveBlock];
 		const std::uint32_t gtid = blockIdx.x * kWaveBlock + threadIdx.x;
 		SpillStack<LdsDepth, kWaveBlock> stack{stackMem + threadIdx.x, src.spill + gtid, gridDim.x * kWaveBlock, 0,
 			kWaveStackCapacity};
-		const std::uint32_t n = src.count();
-		// Rays a wave claims per atomic on the queue's counter (shared by every XCD): about an
-		// eighth of an even share of the queue, a multiple of 64 between 64 and maxChunk, so a
-		// long queue is claimed with few atomics and a short one still spreads over the grid.
-		const std::uint32_t waves = gridDim.x * (kWaveBlock / 64);
+		// Rays a wave claims per atomic on the part's counter: about an eighth of an even share
+		// of the part, a multiple of 64 between 64 and maxChunk, so a long queue is claimed with
+		// few atomics and a short one still spreads over the waves. Its first chunk a wave has
+		// without a claim.
 		const std::uint32_t share = ((n / (8u * waves)) + 63u) & ~63u;
 		const std::uint32_t chunk = min(max(share, 64u), maxChunk);
-		// Waves beyond what the queue can feed leave before touching the claim counter: a
-		// whole grid of claims on one counter costs ~50 us when the queue is short. The waves
-		// that stay claim until the queue is exhausted, so every ray is still traced.
-		if (static_cast<std::uint64_t>(gtid >> 6) * chunk >= n)
+		// Waves beyond what the part can feed leave. The waves that stay claim until it is
+		// exhausted, so every ray is still traced.
+		const std::uint64_t mine = static_cast<std::uint64_t>(wave) * chunk;
+		if (mine >= n)
 		{
 			return;
 		}
-		WaveFeed feed{0u, 0u, false};
-		std::uint32_t rays = 0;
+		const std::uint64_t dealt = static_cast<std::uint64_t>(waves) * chunk;
+		const std::uint32_t begin = static_cast<std::uint32_t>(mine);
+		WaveFeed feed{begin, min(begin + chunk, n), dealt >= n, static_cast<std::uint32_t>(min(dealt, static_cast<std::uint64_t>(n)))};
 		VisitCounter visits{0u, 0u};
 		TraceState st;
 		std::uint32_t slot = 0xffffffffu;
@@ -411,7 +477,7 @@ namespace luzgpu
 		while (true)
 		{
 			const unsigned long long idle = __ballot(!active);
-			if (!feed.drained && (__popcll(idle) >= refillAt || idle == ~0ull))
+			if (feed.any() && (__popcll(idle) >= refillAt || idle == ~0ull))
 			{
 				const std::uint32_t k = feed.hand(idle, n, fetch, chunk);
 				if (!active && k != 0xffffffffu)
@@ -429,14 +495,10 @@ namespace luzgpu
 						lastUnbounded = unboundedOf(jp);
 					}
 					active = traceBegin(st, lastRoot, lastUnbounded, r, tMax, logU, from, stack);
-					if (!active)
-					{
-						src.store(slot, st);
-						rays++;
-					}
+					if (!active) src.store(slot, st);
 				}
 			}
-			if (__ballot(active) == 0ull && feed.drained)
+			if (__ballot(active) == 0ull && !feed.any())
 			{
 				break;
 			}
@@ -461,11 +523,24 @@ namespace luzgpu
 			if (ended)
 			{
 				src.store(slot, st);
-				rays++;
 				active = false;
 			}
 		}
-		flushCounters(counters, counterSlot, rays, visits, Count);
+		if (Count) flushVisits(counters, counterSlot, visits);
+	}
+
+	// Runs `trace(part, wave, waves)` for the queue parts of this block: wave `wave` of the
+	// `waves` that share the part (a grid of fewer than kQueueParts blocks gives a block several).
+	template <typename Trace>
+	__device__ __forceinline__ void	forQueueParts(Trace&& trace)
+	{
+		const std::uint32_t groups = min(gridDim.x, kQueueParts), group = blockIdx.x % groups;
+		const std::uint32_t wave = (blockIdx.x / groups) * (kWaveBlock / 64) + threadIdx.x / 64u;
+		const std::uint32_t waves = ((gridDim.x - group + groups - 1u) / groups) * (kWaveBlock / 64);
+		for (std::uint32_t part = group; part < kQueueParts; part += groups)
+		{
+			trace(part, uniform(wave), waves);
+		}
 	}
 
 	struct	ExtendQueue
@@ -473,10 +548,11 @@ namespace luzgpu
 		const WaveBuffers&	w;
 		int	b;
 		std::uint32_t*	spill;
-		__device__ __forceinline__ std::uint32_t	count() const { return w.counts[b]; }
+		std::uint32_t	base;	// of the queue part
 		// returns the ray's scene job
-		__device__ __forceinline__ std::uint32_t	load(std::uint32_t i, Ray& r, float& tMax, float& logU, RayOrigin& from) const
+		__device__ __forceinline__ std::uint32_t	load(std::uint32_t slot, Ray& r, float& tMax, float& logU, RayOrigin& from) const
 		{
+			const std::uint32_t i = base + slot;
 			const float4 o = w.qOrigin[b & 1][i], d = w.qDir[b & 1][i];
 			r = makeRay(mk(o.x, o.y, o.z), mk(d.x, d.y, d.z));
 			tMax = INFINITY;
@@ -484,8 +560,9 @@ namespace luzgpu
 			from = RayOrigin{__float_as_uint(d.w), w.qFrom[b & 1][i]};
 			return w.sceneOfPath(w.qPath[b & 1][i]);
 		}
-		__device__ __forceinline__ void	store(std::uint32_t i, const TraceState& st) const
+		__device__ __forceinline__ void	store(std::uint32_t slot, const TraceState& st) const
 		{
+			const std::uint32_t i = base + slot;
 			w.qHit[i] = make_float4(st.found ? st.hit.t : -1.0f, st.hit.u, st.hit.v, __uint_as_float(st.hit.hittable));
 			w.qTri[i] = st.hit.tri;
 		}
@@ -497,10 +574,11 @@ namespace luzgpu
 		int	b;
 		std::uint32_t*	spill;
 		std::uint32_t	volumes;	// the batch has volumes: shadow rays carry a sample
+		std::uint32_t	base;	// of the queue part
 		std::uint32_t	target;	// connection slot of the ray being traced
-		__device__ __forceinline__ std::uint32_t	count() const { return w.counts[kMaxBounceSlots + b]; }
-		__device__ __forceinline__ std::uint32_t	load(std::uint32_t i, Ray& r, float& tMax, float& logU, RayOrigin& from)
+		__device__ __forceinline__ std::uint32_t	load(std::uint32_t slot, Ray& r, float& tMax, float& logU, RayOrigin& from)
 		{
+			const std::uint32_t i = base + slot;
 			const float4 o = w.sOrigin[i], d = w.sDir[i];
 			r = makeRay(mk(o.x, o.y, o.z), mk(d.x, d.y, d.z));
 			tMax = o.w;
@@ -525,8 +603,12 @@ namespace luzgpu
 	static __global__ __launch_bounds__(kWaveBlock, 4) void	wf_extend(SceneView s, const PassJob* jobs, WaveBuffers w, int b,
 		unsigned long long* counters, int refillAt, std::uint32_t chunk)
 	{
-		ExtendQueue src{w, b, w.spill};
-		traceQueue<false, Count, Feat, LdsDepth>(s, jobs, src, w.counts + 2 * kMaxBounceSlots + b, refillAt, chunk, counters, 0);
+		__shared__ std::uint32_t stackMem[LdsDepth * kWaveBlock];
+		forQueueParts([&](std::uint32_t part, std::uint32_t wave, std::uint32_t waves) {
+			ExtendQueue src{w, b, w.spill, uniform(part * w.partStride())};
+			traceQueue<false, Count, Feat, LdsDepth>(s, jobs, src, uniform(*w.counter(COUNT_RAYS, b, part)), w.counter(CLAIM_EXTEND, b, part), wave, waves,
+				refillAt, chunk, counters, 0, stackMem);
+		});
 	}
 
 	// Waves per SIMD asked of the shade kernels, whose chains of dependent loads (queue, hit,
@@ -544,14 +626,15 @@ namespace luzgpu
 	static __global__ __launch_bounds__(kWaveBlock, kShadeWaves<Feat>) void	wf_shade(SceneView s, const PassJob* jobs, WaveBuffers w, int b,
 		std::uint32_t volumes, float* __restrict__ sampleColors)
 	{
-		const std::uint32_t n = w.counts[b];
+		// this block's queue part (the grid is a multiple of the parts)
+		const std::uint32_t part = blockIdx.x % kQueueParts;
+		const std::uint32_t n = uniform(*w.counter(COUNT_RAYS, b, part)), partBase = uniform(part * w.partStride());
 		const int q = b & 1;
-		std::uint32_t* nextCount = w.counts + b + 1;
-		std::uint32_t* shadowCount = w.counts + kMaxBounceSlots + b;
+		std::uint32_t* nextCount = w.counter(COUNT_RAYS, b + 1, part);
+		std::uint32_t* shadowCount = w.counter(COUNT_SHADOW, b, part);
 		// Queue appends: each wave counts its continuing paths and its shadow rays (light
 		// connections, then environment ones) in LDS, and one thread claims the block's
-		// ranges of the next queue and the shadow queue with one atomic each. The counters
-		// are shared by every XCD, so per-wave atomics on them queue up behind each other.
+		// ranges of the next queue and the shadow queue with one atomic each.
 		constexpr int kWaves = kWaveBlock / 64;
 		__shared__ std::uint32_t waveNext[kWaves], waveShadow[kWaves], blockNext, blockShadow;
 		// staged per lane: the vertex, the next direction, its origin's identity, the light
@@ -570,11 +653,11 @@ namespace luzgpu
 		const int wave = static_cast<int>(threadIdx.x >> 6);
 		// grid-stride loop with a block-uniform trip count so every lane reaches the ballots
 		// and every wave the barriers
-		const std::uint32_t stride = gridDim.x * kWaveBlock;
-		for (std::uint32_t blockBase = blockIdx.x * kWaveBlock; blockBase < n; blockBase += stride)
+		const std::uint32_t stride = gridDim.x / kQueueParts * kWaveBlock;
+		for (std::uint32_t blockBase = blockIdx.x / kQueueParts * kWaveBlock; blockBase < n; blockBase += stride)
 		{
-			const std::uint32_t i = blockBase + threadIdx.x;
-			const bool valid = i < n;
+			const bool valid = blockBase + threadIdx.x < n;
+			const std::uint32_t i = partBase + blockBase + threadIdx.x;
 			bool cont = false, wantLight = false, wantEnv = false;
 			const std::uint32_t qp = valid ? w.qPath[q][i] : 0u;
 			const std::uint32_t job = Batch ? w.sceneOfPath(qp) : 0u;
@@ -810,7 +893,7 @@ namespace luzgpu
 				blockShadow = tShadow > 0 ? atomicAdd(shadowCount, tShadow) : 0u;
 			}
 			__syncthreads();
-			std::uint32_t nextBase = blockNext, shadowBase = blockShadow;
+			std::uint32_t nextBase = partBase + blockNext, shadowBase = 2u * partBase + blockShadow;
 			for (int k = 0; k < wave; k++)
 			{
 				nextBase += waveNext[k];
@@ -856,8 +939,12 @@ namespace luzgpu
 	static __global__ __launch_bounds__(kWaveBlock, 4) void	wf_shadow(SceneView s, const PassJob* jobs, WaveBuffers w, int b,
 		unsigned long long* counters, int refillAt, std::uint32_t chunk, std::uint32_t volumes)
 	{
-		ShadowQueue src{w, b, w.spill, volumes, 0u};
-		traceQueue<true, Count, Feat, LdsDepth>(s, jobs, src, w.counts + 3 * kMaxBounceSlots + b, refillAt, chunk, counters, 1);
+		__shared__ std::uint32_t stackMem[LdsDepth * kWaveBlock];
+		forQueueParts([&](std::uint32_t part, std::uint32_t wave, std::uint32_t waves) {
+			ShadowQueue src{w, b, w.spill, volumes, uniform(2u * part * w.partStride()), 0u};
+			traceQueue<true, Count, Feat, LdsDepth>(s, jobs, src, uniform(*w.counter(COUNT_SHADOW, b, part)), w.counter(CLAIM_SHADOW, b, part), wave,
+				waves, refillAt, chunk, counters, 1, stackMem);
+		});
 	}
 
 	// Adds a pass's sample colours of one scene into its FP64 pixel sums, in sample order
@@ -1029,6 +1116,7 @@ namespace luzgpu
 		size_t	carve(char* base, std::uint32_t capacity)
 		{
 			const size_t n = capacity;
+			const size_t nq = n + kPartTile * (kQueueParts + 1);	// the parts' strides are whole tiles
 			const size_t spillBytes = static_cast<size_t>(kWaveStackCapacity - kWaveLdsStackMin) * kWaveGrid * kWaveBlock * 4;
 			size_t off = 0;
 			auto take = [&](size_t b) { char* r = base ? base + off : nullptr; off += (b + 255) & ~size_t(255); return r; };
@@ -1036,24 +1124,24 @@ namespace luzgpu
 			std::memset(&nb, 0, sizeof(nb));	// padding too: graph keys compare the raw bytes
 			for (int k = 0; k < 2; k++)
 			{
-				nb.qOrigin[k] = reinterpret_cast<float4*>(take(16 * n));
-				nb.qDir[k] = reinterpret_cast<float4*>(take(16 * n));
-				nb.qFrom[k] = reinterpret_cast<std::int32_t*>(take(4 * n));
-				nb.qPath[k] = reinterpret_cast<std::uint32_t*>(take(4 * n));
+				nb.qOrigin[k] = reinterpret_cast<float4*>(take(16 * nq));
+				nb.qDir[k] = reinterpret_cast<float4*>(take(16 * nq));
+				nb.qFrom[k] = reinterpret_cast<std::int32_t*>(take(4 * nq));
+				nb.qPath[k] = reinterpret_cast<std::uint32_t*>(take(4 * nq));
 			}
-			nb.qHit = reinterpret_cast<float4*>(take(16 * n));
-			nb.qTri = reinterpret_cast<std::int32_t*>(take(4 * n));
+			nb.qHit = reinterpret_cast<float4*>(take(16 * nq));
+			nb.qTri = reinterpret_cast<std::int32_t*>(take(4 * nq));
 			nb.throughput = reinterpret_cast<float4*>(take(16 * n));
 			nb.radiance = reinterpret_cast<float4*>(take(16 * n));
 			nb.prevOrigin = reinterpret_cast<float4*>(take(16 * n));
 			nb.connection = reinterpret_cast<float4*>(take(32 * n));
 			nb.visible = reinterpret_cast<std::uint8_t*>(take(2 * n));
-			nb.sOrigin = reinterpret_cast<float4*>(take(32 * n));
-			nb.sDir = reinterpret_cast<float4*>(take(32 * n));
-			nb.sLogU = reinterpret_cast<float*>(take(8 * n));
-			nb.sFrom = reinterpret_cast<int2*>(take(16 * n));
+			nb.sOrigin = reinterpret_cast<float4*>(take(32 * nq));
+			nb.sDir = reinterpret_cast<float4*>(take(32 * nq));
+			nb.sLogU = reinterpret_cast<float*>(take(8 * nq));
+			nb.sFrom = reinterpret_cast<int2*>(take(16 * nq));
 			float* nc = reinterpret_cast<float*>(take(12 * n));
-			nb.counts = reinterpret_cast<std::uint32_t*>(take(kMaxBounceSlots * 4 * 4));
+			nb.counts = reinterpret_cast<std::uint32_t*>(take((kCounterWords + 2) * 4));
 			PassJob* nj = reinterpret_cast<PassJob*>(take(sizeof(PassJob) * kMaxBatchScenes));
 			nb.spill = reinterpret_cast<std::uint32_t*>(take(spillBytes));
 			nb.capacity = capacity;
@@ -1157,7 +1245,7 @@ namespace luzgpu
 		};
 		const std::uint32_t vol = volumes ? 1u : 0u;
 		constexpr int T = Feat & kFeatAll;	// extend and shadow differ only by primitive / material class
-		wf_zero_counts<<<1, 4 * kMaxBounceSlots, 0, stream>>>(w.counts, 4 * kMaxBounceSlots, st.jobs, jobCount);
+		wf_zero_counts<<<kCounterWords / kCounterStride / 256, 256, 0, stream>>>(w, st.jobs, jobCount);
 		wf_raygen<<<kWaveGrid, kWaveBlock, 0, stream>>>(st.jobs, jobCount, w);
 		for (int b = 0; b <= maxBounces; b++)
 		{
@@ -1177,6 +1265,7 @@ namespace luzgpu
 			else wf_shadow<false, T, 16><<<tune.grid, kWaveBlock, 0, stream>>>(s, st.jobs, w, b, counters, tune.shadowRefill, ch, vol);
 			mark();
 		}
+		wf_count_rays<<<1, 64, 0, stream>>>(w, counters);
 		for (std::uint32_t j = 0; j < jobCount; j++)
 		{
 			wf_accumulate<<<1024, 256, 0, stream>>>(w, st.colors, st.jobs, j);
