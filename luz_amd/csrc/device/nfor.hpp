@@ -18,6 +18,8 @@
 // Gauss-Jordan elimination with partial pivoting.
 #pragma once
 
+#include "median.hpp"
+
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -122,7 +124,7 @@ namespace luzgpu
 	// neighbours in its 5 x 5 window that stands 2.5x and 0.18 above the window's median
 	// luminance takes the luminance-median of its darker neighbours. `average` != 0: the
 	// input is the mean of a and b (averageColorBuffers) instead of a.
-	static __global__ void	nfor_fireflies(const double* __restrict__ a, const double* __restrict__ b, double* __restrict__ out,
+	static __global__ __launch_bounds__(256) void	nfor_fireflies(const double* __restrict__ a, const double* __restrict__ b, double* __restrict__ out,
 		NforParams P, int average)
 	{
 		const std::uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -143,64 +145,42 @@ namespace luzgpu
 		if (P.width < 3 || P.height < 3) return;
 		const std::uint32_t x = i % P.width, y = i / P.width;
 		const double lum = nforLuminance(center);
-		double neighbor[24];
-		std::uint32_t candidate[24];
-		double candidateLum[24];
-		int n = 0, nc = 0;
-		unsigned similar = 0;
-		for (int oy = -2; oy <= 2; oy++)
+		if (lum < 0.30) return;
+		const double none = __builtin_nan("");
+		double key[24];	// neighbours' luminances, row by row
+		std::uint32_t inside = 0, candidates = 0;
+		auto neighbor = [&](int k) {
+			const int at = k + (k >= 12 ? 1 : 0);
+			return (y + static_cast<std::uint32_t>(at / 5) - 2u) * P.width + x + static_cast<std::uint32_t>(at % 5) - 2u;
+		};
+		#pragma unroll
+		for (int k = 0; k < 24; k++)
 		{
-			for (int ox = -2; ox <= 2; ox++)
-			{
-				if (ox == 0 && oy == 0) continue;
-				const long long sx = static_cast<long long>(x) + ox, sy = static_cast<long long>(y) + oy;
-				if (sx < 0 || sy < 0 || sx >= P.width || sy >= P.height) continue;
-				const std::uint32_t k = static_cast<std::uint32_t>(sy) * P.width + static_cast<std::uint32_t>(sx);
-				double c[3];
-				colorAt(k, c);
-				const double l = nforLuminance(c);
-				neighbor[n++] = l;
-				if (l >= lum * 0.65) similar++;
-				else
-				{
-					candidate[nc] = k;
-					candidateLum[nc] = l;
-					nc++;
-				}
-			}
+			const int at = k + (k >= 12 ? 1 : 0);
+			const long long sx = static_cast<long long>(x) + at % 5 - 2, sy = static_cast<long long>(y) + at / 5 - 2;
+			key[k] = none;
+			if (sx < 0 || sy < 0 || sx >= P.width || sy >= P.height) continue;
+			double c[3];
+			colorAt(neighbor(k), c);
+			key[k] = nforLuminance(c);
+			inside |= 1u << k;
+			if (!(key[k] >= lum * 0.65)) candidates |= 1u << k;
 		}
 		// isDenoiseFirefly (NFOR.cpp:115-143)
-		if (nc == 0 || lum < 0.30 || n == 0 || similar >= 2u) return;
-		for (int p = 1; p < n; p++)
-		{
-			const double v = neighbor[p];
-			int q = p - 1;
-			while (q >= 0 && neighbor[q] > v)
-			{
-				neighbor[q + 1] = neighbor[q];
-				q--;
-			}
-			neighbor[q + 1] = v;
-		}
-		const double median = neighbor[n / 2];
+		if (candidates == 0u || __popc(inside & ~candidates) >= 2) return;
+		const int middle = medianIndex(key, inside);
+		double median = 0.0;
+		#pragma unroll
+		for (int k = 0; k < 24; k++) median = k == middle ? key[k] : median;
 		if (!(lum >= median * 2.5 && lum >= median + 0.18)) return;
 		// medianColorByLuminance (NFOR.cpp:105-113)
-		for (int p = 1; p < nc; p++)
+		#pragma unroll
+		for (int k = 0; k < 24; k++)
 		{
-			const double v = candidateLum[p];
-			const std::uint32_t k = candidate[p];
-			int q = p - 1;
-			while (q >= 0 && candidateLum[q] > v)
-			{
-				candidateLum[q + 1] = candidateLum[q];
-				candidate[q + 1] = candidate[q];
-				q--;
-			}
-			candidateLum[q + 1] = v;
-			candidate[q + 1] = k;
+			if ((candidates >> k & 1u) == 0u) key[k] = none;
 		}
 		double c[3];
-		colorAt(candidate[nc / 2], c);
+		colorAt(neighbor(medianIndex(key, candidates)), c);
 		for (int j = 0; j < 3; j++) out[3 * i + j] = c[j];
 	}
 

@@ -8,6 +8,8 @@
 // bright-pass, blur, firefly suppression) read a 5 x 5 or 9-tap neighbourhood from L2.
 #pragma once
 
+#include "median.hpp"
+
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -284,33 +286,9 @@ namespace luzgpu
 		return postMaxChannel(c) >= 0.995 && postMinChannel(c) >= 0.96 && postSceneLuminance(c) >= 0.98;
 	}
 
-	// medianNeighborColor (Image.cpp:141-152): the colour of middle luminance rank. The
-	// candidates are ordered by an insertion sort on luminance, which equals the reference's
-	// ordering whenever luminances differ or tied candidates are the same colour.
-	__device__ inline PostColor	postMedianColor(PostColor* c, int n)
-	{
-		double key[24];
-		for (int k = 0; k < n; k++) key[k] = postSceneLuminance(c[k]);
-		for (int a = 1; a < n; a++)
-		{
-			const double kv = key[a];
-			const PostColor cv = c[a];
-			int b = a - 1;
-			while (b >= 0 && kv < key[b])
-			{
-				key[b + 1] = key[b];
-				c[b + 1] = c[b];
-				b--;
-			}
-			key[b + 1] = kv;
-			c[b + 1] = cv;
-		}
-		return c[n / 2];
-	}
-
 	// suppressIsolatedFireflies (Image.cpp:506-526) with suppressDisplayFirefly
 	// (Image.cpp:154-268), over the display-encoded image.
-	static __global__ void	post_fireflies(const double* __restrict__ src, double* __restrict__ dst, PostParams P)
+	static __global__ __launch_bounds__(256) void	post_fireflies(const double* __restrict__ src, double* __restrict__ dst, PostParams P)
 	{
 		#pragma clang fp contract(off)
 		const size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -331,68 +309,76 @@ namespace luzgpu
 			keep();
 			return;
 		}
+		// Neighbour k of the 5 x 5 window's 24: its luminance, and whether it is a candidate
+		// (no firefly itself).
+		const double none = __builtin_nan("");
+		double key[24];
+		std::uint32_t inside = 0, candidates = 0;
 		unsigned similar = 0, brightN = 0, saturated = 0;
-		double immediate[8];
-		int nImmediate = 0;
-		PostColor candidates[24];
-		int nCandidates = 0;
-		for (int oy = -2; oy <= 2; oy++)
+		auto neighbor = [&](int k) {
+			const int at = k + (k >= 12 ? 1 : 0);
+			return static_cast<size_t>(y + at / 5 - 2) * P.width + static_cast<size_t>(x + at % 5 - 2);
+		};
+		#pragma unroll
+		for (int k = 0; k < 24; k++)
 		{
-			for (int ox = -2; ox <= 2; ox++)
-			{
-				if (ox == 0 && oy == 0) continue;
-				const long long sx = x + ox, sy = y + oy;
-				if (sx < 0 || sy < 0 || sx >= static_cast<long long>(P.width) || sy >= static_cast<long long>(P.height)) continue;
-				const PostColor nb = postLoad(src, static_cast<size_t>(sy) * P.width + static_cast<size_t>(sx));
-				const double nl = postSceneLuminance(nb);
-				if (ox >= -1 && ox <= 1 && oy >= -1 && oy <= 1) immediate[nImmediate++] = nl;
-				if (nl >= luminance * 0.65) similar++;
-				if (nl >= 0.80) brightN++;
-				if (postSaturated(nb)) saturated++;
-				if (!postFireflyCandidate(nb)) candidates[nCandidates++] = nb;
-			}
+			const int at = k + (k >= 12 ? 1 : 0);
+			const long long sx = x + at % 5 - 2, sy = y + at / 5 - 2;
+			key[k] = none;
+			if (sx < 0 || sy < 0 || sx >= static_cast<long long>(P.width) || sy >= static_cast<long long>(P.height)) continue;
+			const PostColor nb = postLoad(src, neighbor(k));
+			const double nl = postSceneLuminance(nb);
+			key[k] = nl;
+			inside |= 1u << k;
+			if (nl >= luminance * 0.65) similar++;
+			if (nl >= 0.80) brightN++;
+			if (postSaturated(nb)) saturated++;
+			if (!postFireflyCandidate(nb)) candidates |= 1u << k;
 		}
+		bool replace;
 		if (!displayCandidate)
 		{
-			if (nImmediate == 0)
+			// the eight neighbours next to the pixel
+			constexpr int kNext[8] = {6, 7, 8, 11, 12, 15, 16, 17};
+			double next[8];
+			std::uint32_t valid = 0;
+			#pragma unroll
+			for (int k = 0; k < 8; k++)
+			{
+				next[k] = key[kNext[k]];
+				valid |= (inside >> kNext[k] & 1u) << k;
+			}
+			if (valid == 0u)
 			{
 				keep();
 				return;
 			}
-			for (int a = 1; a < nImmediate; a++)
-			{
-				const double v = immediate[a];
-				int b = a - 1;
-				while (b >= 0 && v < immediate[b])
-				{
-					immediate[b + 1] = immediate[b];
-					b--;
-				}
-				immediate[b + 1] = v;
-			}
-			const double localMedian = immediate[nImmediate / 2];
+			const int middle = medianIndex(next, valid);
+			double localMedian = 0.0;
+			#pragma unroll
+			for (int k = 0; k < 8; k++) localMedian = k == middle ? next[k] : localMedian;
 			if (luminance < localMedian * 1.65 || luminance < localMedian + 0.08)
 			{
 				keep();
 				return;
 			}
-			if (nCandidates > 0)
-			{
-				postStore(dst, i, postMedianColor(candidates, nCandidates));
-				return;
-			}
+			replace = candidates != 0u;
 		}
-		if (saturatedCandidate && saturated < 3u && nCandidates > 0)
-		{
-			postStore(dst, i, postMedianColor(candidates, nCandidates));
-			return;
-		}
-		if (similar >= 4u || brightN >= 6u || nCandidates == 0)
+		else replace = false;
+		replace = replace || (saturatedCandidate && saturated < 3u && candidates != 0u) || (similar < 4u && brightN < 6u && candidates != 0u);
+		if (!replace)
 		{
 			keep();
 			return;
 		}
-		postStore(dst, i, postMedianColor(candidates, nCandidates));
+		// medianNeighborColor (Image.cpp:141-152): the candidate of middle luminance rank, which
+		// equals the reference's whenever luminances differ or tied candidates are the same colour
+		#pragma unroll
+		for (int k = 0; k < 24; k++)
+		{
+			if ((candidates >> k & 1u) == 0u) key[k] = none;
+		}
+		postStore(dst, i, postLoad(src, neighbor(medianIndex(key, candidates))));
 	}
 
 	static __global__ void	post_to_float(const double* __restrict__ in, float* __restrict__ out, size_t n)
