@@ -17,6 +17,7 @@
 #include "device/post.hpp"
 #include "device/wavefront.hpp"
 #include "host/accel.hpp"
+#include "host/staging.hpp"
 
 #include <atomic>
 #include <unordered_set>
@@ -481,6 +482,7 @@ struct luzgpu_ctx
 	luzgpu::DeviceBuffer	adaptiveMem;
 	// display post-processing: the FP64 mean image and three working images
 	luzgpu::DeviceBuffer	postMem;
+	luzgpu::HostStaging	staging;
 	// batched plain-kernel launches: their job tables
 	luzgpu::DeviceBuffer	megaJobs;
 	// per-pixel sample counts of the last single-scene render: `countsUniform` samples each,
@@ -1475,7 +1477,7 @@ int	luzgpu_render(luzgpu_ctx* ctx, luzgpu_scene* scene, const luzgpu_settings* s
 		check(hipMemcpyAsync(counters, ctx->counters.ptr, sizeof(counters), hipMemcpyDeviceToHost, st), "counter readback");
 		if (dst != rgb_out)
 		{
-			check(hipMemcpyAsync(rgb_out, dst, static_cast<size_t>(pixels) * 3 * sizeof(float), hipMemcpyDeviceToHost, st), "image readback");
+			check(ctx->staging.readback(rgb_out, dst, static_cast<size_t>(pixels) * 3 * sizeof(float), st), "image readback");
 		}
 		check(hipStreamSynchronize(st), "render");
 		const float ms = elapsedMs(e0, e1);
@@ -1722,9 +1724,16 @@ int	luzgpu_render_denoised(luzgpu_ctx* ctx, luzgpu_scene* scene, const luzgpu_se
 		}
 		e2.record(st);
 		const size_t imageBytes = static_cast<size_t>(pixels) * 3 * sizeof(float);
-		const hipMemcpyKind kind = (settings && settings->output_on_device) ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost;
-		check(hipMemcpyAsync(rgb_out, image, imageBytes, kind, st), "image copy");
-		check(hipMemcpyAsync(denoised_out, denoised, imageBytes, kind, st), "denoised copy");
+		if (settings && settings->output_on_device)
+		{
+			check(hipMemcpyAsync(rgb_out, image, imageBytes, hipMemcpyDeviceToDevice, st), "image copy");
+			check(hipMemcpyAsync(denoised_out, denoised, imageBytes, hipMemcpyDeviceToDevice, st), "denoised copy");
+		}
+		else
+		{
+			check(ctx->staging.readback(rgb_out, image, imageBytes, st), "image readback");
+			check(ctx->staging.readback(denoised_out, denoised, imageBytes, st), "denoised readback");
+		}
 		if (buffers_out)
 		{
 			buffers_out->width = p.width;
@@ -1736,8 +1745,7 @@ int	luzgpu_render_denoised(luzgpu_ctx* ctx, luzgpu_scene* scene, const luzgpu_se
 			for (int k = 0; k < 7; k++)
 			{
 				if (!fields[k].first) continue;
-				check(hipMemcpyAsync(fields[k].first, nb + fields[k].second, sizes[k] * pixels * sizeof(double), hipMemcpyDeviceToHost, st),
-					"buffer readback");
+				check(ctx->staging.readback(fields[k].first, nb + fields[k].second, sizes[k] * pixels * sizeof(double), st), "buffer readback");
 			}
 		}
 		unsigned long long counters[2] = {0, 0};
@@ -1783,13 +1791,13 @@ int	luzgpu_nfor(luzgpu_ctx* ctx, const luzgpu_nfor_buffers* in, const luzgpu_nfo
 		const size_t sizes[] = {3, 3, 1, kNforFeatures, kNforFeatures, kNforFeatures};
 		for (int k = 0; k < 6; k++)
 		{
-			check(hipMemcpyAsync(nb + fields[k].second, fields[k].first, sizes[k] * n * sizeof(double), hipMemcpyHostToDevice, st), "buffer upload");
+			check(ctx->staging.upload(nb + fields[k].second, fields[k].first, sizes[k] * n * sizeof(double), st), "buffer upload");
 		}
 		Event e0, e1;
 		e0.record(st);
 		runNfor(ctx, P, nb + L.colorA, nb + L.colorB, nb + L.colorVariance, nb + L.featA, nb + L.featB, nb + L.featVariance, nb + L.total);
 		e1.record(st);
-		check(hipMemcpyAsync(denoised_out, nb + L.total, 3 * n * sizeof(double), hipMemcpyDeviceToHost, st), "denoised readback");
+		check(ctx->staging.readback(denoised_out, nb + L.total, 3 * n * sizeof(double), st), "denoised readback");
 		check(hipStreamSynchronize(st), "NFOR");
 		float ms = 0.0f;
 		check(hipEventElapsedTime(&ms, e0, e1), "hipEventElapsedTime");
@@ -2075,8 +2083,7 @@ int	luzgpu_render_batch(luzgpu_ctx* ctx, uint32_t n, luzgpu_scene* const* scenes
 		{
 			if (settings && settings[i].output_on_device) continue;
 			const size_t bytes = static_cast<size_t>(jobs[i].params.width) * jobs[i].params.height * 3 * sizeof(float);
-			check(hipMemcpyAsync(copies[c].first, static_cast<char*>(ctx->output.ptr) + copies[c].second, bytes, hipMemcpyDeviceToHost, st),
-				"image readback");
+			check(ctx->staging.readback(copies[c].first, static_cast<char*>(ctx->output.ptr) + copies[c].second, bytes, st), "image readback");
 			c++;
 		}
 		check(hipStreamSynchronize(st), "batch render");
@@ -2275,9 +2282,9 @@ int	luzgpu_postprocess(luzgpu_ctx* ctx, const luzgpu_post_settings* post, uint32
 		(void)postParams(*post, width, height);	// validate before any copy
 		ctx->postMem.reserve(4 * bytes);
 		double* buf = ctx->postMem.as<double>();
-		check(hipMemcpyAsync(buf, image_in, bytes, hipMemcpyHostToDevice, st), "image upload");
+		check(ctx->staging.upload(buf, image_in, bytes, st), "image upload");
 		runPost(ctx, *post, width, height, buf, buf);
-		check(hipMemcpyAsync(image_out, buf, bytes, hipMemcpyDeviceToHost, st), "image readback");
+		check(ctx->staging.readback(image_out, buf, bytes, st), "image readback");
 		check(hipStreamSynchronize(st), "post-processing");
 	});
 }

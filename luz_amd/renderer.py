@@ -433,7 +433,7 @@ class Renderer:
         ps = post.post_settings() if isinstance(post, Scene) else _post_settings(post)
         img = np.ascontiguousarray(image, dtype=np.float64)
         h, w = img.shape[:2]
-        out = np.zeros_like(img)
+        out = np.empty_like(img)
         _lib.check(ctx._lib.luzgpu_postprocess(ctx.handle, ctypes.byref(ps), w, h, img.ctypes.data, out.ctypes.data, 0))
         return out
 
