@@ -359,6 +359,34 @@ namespace luzgpu
 		}
 	}
 
+	// The images of a batch's scenes in one launch, block row y for scene y: a launch a scene cost
+	// 32 thumbnails 3.3 us each, a quarter of the call (0.43 -> 0.38 ms). The table travels as the
+	// argument.
+	struct	ResolveBatch
+	{
+		static constexpr std::uint32_t	kScenes = 64;
+
+		struct	Scene
+		{
+			const double*	sums;
+			float*	out;
+			double	count;
+			size_t	values;	// 3 a pixel
+		};
+		Scene	scenes[kScenes];
+	};
+
+	__global__ void	resolve_batch(ResolveBatch B)
+	{
+		const ResolveBatch::Scene& S = B.scenes[blockIdx.y];
+		const size_t stride = static_cast<size_t>(gridDim.x) * blockDim.x;
+		for (size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < S.values; i += stride)
+		{
+			const double v = S.sums[i] / S.count;
+			S.out[i] = isfinite(v) ? static_cast<float>(v) : 0.0f;
+		}
+	}
+
 	// The FP64 mean image (cleanColor'd, Threads.cpp:580-581) for post-processing: each
 	// pixel's sum over `used[i]` samples, or over `count` when used is nullptr.
 	__global__ void	resolve_double(const double* __restrict__ sums, const std::uint32_t* __restrict__ used, double count,
@@ -909,8 +937,10 @@ namespace luzgpu
 		}
 
 		// The integrator a call runs: LUZGPU_INTEGRATOR_AUTO picks the plain kernel for at most
-		// 4M paths. A batch of 32 small scenes measured the crossover between 2.1M paths (the
-		// plain kernel 1.3x faster) and 8.4M (the wavefront 1.2x faster).
+		// 4M paths, as the interface says. A batch of 32 small scenes of 2.1M paths takes 1.2 ms
+		// plain and 2.0 ms on the wavefront; single scenes cross between 0.8M and 2M paths (box of
+		// 34 triangles: 1.28 / 1.27 ms and 2.8 / 2.2 ms; 512 instanced spheres: 1.05 / 1.84 and
+		// 2.24 / 2.29 ms).
 		std::uint32_t	resolveIntegrator(std::uint32_t requested, std::uint64_t paths, const char* who)
 		{
 			if (requested == LUZGPU_INTEGRATOR_AUTO)
@@ -2054,6 +2084,15 @@ int	luzgpu_render_batch(luzgpu_ctx* ctx, uint32_t n, luzgpu_scene* const* scenes
 		if (hostBytes) ctx->output.reserve(hostBytes);
 		size_t staged = 0;
 		std::vector<std::pair<float*, size_t>> copies;
+		ResolveBatch plain;
+		std::uint32_t plainScenes = 0;
+		auto resolvePlain = [&] {
+			if (plainScenes == 0) return;
+			size_t most = 0;
+			for (std::uint32_t k = 0; k < plainScenes; k++) most = std::max(most, plain.scenes[k].values);
+			resolve_batch<<<dim3(std::min(blocks(most, 256), 256u), plainScenes), 256, 0, st>>>(plain);
+			plainScenes = 0;
+		};
 		for (uint32_t i = 0; i < n; i++)
 		{
 			const std::uint32_t pixels = jobs[i].params.width * jobs[i].params.height;
@@ -2074,8 +2113,21 @@ int	luzgpu_render_batch(luzgpu_ctx* ctx, uint32_t n, luzgpu_scene* const* scenes
 				post_to_float<<<blocks(static_cast<size_t>(pixels) * 3, 256), 256, 0, st>>>(mean, dst, static_cast<size_t>(pixels) * 3);
 			}
 			else if (adaptive) resolve_used<<<blocks(pixels, 256), 256, 0, st>>>(jobs[i].sums, A.used + aj[i].offset, dst, pixels);
-			else resolve<<<blocks(pixels, 256), 256, 0, st>>>(jobs[i].sums, dst, pixels, static_cast<double>(jobs[i].params.sampleCount));
+			else
+			{
+				// scenes that share an output keep their order: the last one's image stays
+				const size_t values = static_cast<size_t>(pixels) * 3;
+				bool shared = plainScenes == ResolveBatch::kScenes;
+				for (std::uint32_t k = 0; k < plainScenes; k++)
+				{
+					const ResolveBatch::Scene& other = plain.scenes[k];
+					shared = shared || (dst < other.out + other.values && other.out < dst + values);
+				}
+				if (shared) resolvePlain();
+				plain.scenes[plainScenes++] = ResolveBatch::Scene{jobs[i].sums, dst, static_cast<double>(jobs[i].params.sampleCount), values};
+			}
 		}
+		resolvePlain();
 		check(hipGetLastError(), "resolve launch");
 		unsigned long long counters[6] = {0, 0, 0, 0, 0, 0};
 		check(hipMemcpyAsync(counters, ctx->counters.ptr, sizeof(counters), hipMemcpyDeviceToHost, st), "counter readback");

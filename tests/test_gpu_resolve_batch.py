@@ -1,0 +1,37 @@
+"""The one-launch resolve of a batch (GPU): more scenes than a launch's table holds (64), odd
+sizes from one pixel up, host or device outputs, and scenes that share an output, where
+the last one's image stays. Each image has the bits of the scene's own render."""
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("count", [1, 64, 65, 100])
+def test_batch_images_equal_single_renders(ctx, cornell, count):
+    import torch
+    from luz_amd import Renderer, SceneFile
+    scene = SceneFile.read(ctx, cornell.scene_path)
+    sizes = [(1 + 7 * (i % 9), 1 + 5 * (i % 4)) for i in range(count)]
+    seeds = list(range(1, count + 1))
+    args = dict(samples=[2] * count, resolutions=sizes, integrator="megakernel")
+    images, _ = Renderer.render_batch([scene] * count, seeds, **args)
+    outs = [torch.empty((h, w, 3), device="cuda:0") for w, h in sizes]
+    Renderer.render_batch([scene] * count, seeds, outs=outs, **args)
+    torch.cuda.synchronize()
+    for i in range(count):
+        one, _ = Renderer.render(scene, seed=seeds[i], samples=2, resolution=sizes[i], integrator="megakernel")
+        assert np.array_equal(images[i], one), i
+        assert np.array_equal(outs[i].cpu().numpy(), one), i
+
+
+def test_a_shared_output_holds_the_last_scene(ctx, cornell):
+    import torch
+    from luz_amd import Renderer, SceneFile
+    scene = SceneFile.read(ctx, cornell.scene_path)
+    out = torch.empty((33, 65, 3), device="cuda:0")
+    Renderer.render_batch([scene] * 5, [1, 2, 3, 4, 5], samples=[1] * 5, resolutions=[(65, 33)] * 5, outs=[out] * 5, integrator="megakernel")
+    torch.cuda.synchronize()
+    one, _ = Renderer.render(scene, seed=5, samples=1, resolution=(65, 33), integrator="megakernel")
+    assert np.array_equal(out.cpu().numpy(), one)
