@@ -412,7 +412,7 @@ namespace luzgpu
 	// Bound by VALU issue: the whole node is one straight line (about 130 instructions against
 	// the 330 of a form that branched per child, per push and for axis-parallel rays, and
 	// decoded exponents and leaf counts), so it keeps to four 16-byte loads issued together, a
-	// ready scale and ready stack entries in the node, one five-comparator sort, and stack
+	// ready scale and ready stack entries in the node, one six-comparator sort, and stack
 	// writes that need no branch.
 	template <bool Count, typename Stack>
 	__device__ __forceinline__ bool	nodeStep(const SceneView& s, TraceState& st, Stack& stack, VisitCounter* counter)
@@ -449,20 +449,26 @@ namespace luzgpu
 			const bool in = (far >= near) & (k == 0 || e[k] != kEmptyChild);
 			key[k] = in ? near : INFINITY;
 		}
-		auto exchange = [&](int i, int j) {
-			const bool swap = key[j] < key[i];
+		// Exchanges of neighbours alone keep equal distances in child order: of primitives hit at
+		// the same distance the last one visited is the hit, and boxes entered at the same
+		// distance (primitives of one plane, boxes around the ray's origin) are common. Five
+		// exchanges would sort without keeping it, at most 1 % faster (a 1080p spheres frame
+		// 31.7 against 32.0 ms, 720p hazy terrain 71.5 against 71.9).
+		auto exchange = [&](int i) {
+			const bool swap = key[i + 1] < key[i];
 			const float ki = key[i];
 			const std::uint32_t ei = e[i];
-			key[i] = fminf(key[j], ki);
-			key[j] = fmaxf(key[j], ki);
-			e[i] = swap ? e[j] : ei;
-			e[j] = swap ? ei : e[j];
+			key[i] = fminf(key[i + 1], ki);
+			key[i + 1] = fmaxf(key[i + 1], ki);
+			e[i] = swap ? e[i + 1] : ei;
+			e[i + 1] = swap ? ei : e[i + 1];
 		};
-		exchange(0, 1);
-		exchange(2, 3);
-		exchange(0, 2);
-		exchange(1, 3);
-		exchange(1, 2);
+		exchange(0);
+		exchange(2);
+		exchange(1);
+		exchange(0);
+		exchange(2);
+		exchange(1);
 		stack.push3(e[3], key[3] < INFINITY, e[2], key[2] < INFINITY, e[1], key[1] < INFINITY);
 		st.entry = e[0];
 		return key[0] < INFINITY;
