@@ -1,7 +1,7 @@
 // Two-level BVH traversal (closest hit and any hit) over the 64-byte node layout.
 //
-// One stack serves both levels: entering a mesh instance pushes an exit marker, then
-// the mesh root; popping the marker restores the world-space ray. The instance's ray
+// One stack serves both levels: entering a mesh instance notes the stack's height, and a pop
+// at that height leaves the instance (the world-space ray is restored). The instance's ray
 // keeps the world parameterisation (its direction is the affine image of the world
 // direction, not renormalised), so a hit distance needs no rescaling between levels.
 //
@@ -228,6 +228,12 @@ namespace luzgpu
 	};
 	constexpr RayOrigin	kNoOrigin{0xffffffffu, -1};
 
+	// What a stack holds beyond the bound that a scene is admitted by (its deferred entries,
+	// PackedScene::tlasStackBound + blasStackBound): one entry where a leaf of two kinds was split
+	// into nodes, and the slot above the top entry that push3 writes in vain: with less, the
+	// clamp would put that write on the top entry itself.
+	constexpr int	kStackReserve = 2;
+
 	// Per-thread traversal stack in LDS, laid out [depth][thread] so the 64 lanes of a
 	// wave touch 64 consecutive banks.
 	template <int Depth, int Block>
@@ -236,7 +242,7 @@ namespace luzgpu
 		std::uint32_t*	base;
 		int	sp;
 
-		// The host refuses scenes whose BVH depth could exceed Depth; the clamp only keeps
+		// The host refuses scenes whose bound and kStackReserve exceed Depth; the clamp only keeps
 		// every LDS access inside this thread's column whatever happens.
 		__device__ __forceinline__ void	push(std::uint32_t v) { base[min(sp, Depth - 1) * Block] = v; sp++; }
 		// pushes a if wanted, then b, then c: a slot written in vain is the next push's

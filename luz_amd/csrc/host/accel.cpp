@@ -541,12 +541,23 @@ namespace luzgpu
 			return 1 + d;
 		}
 
+		// Nodes that the device tree has in the place of a leaf.
+		enum : std::uint8_t { kNotSplit = 0, kSplitApart = 1, kSplitChain = 2 };
+
+		bool	overlap(const AABBd& a, const AABBd& b)
+		{
+			bool o = true;
+			for (int i = 0; i < 3; i++) o = o && a.lo[i] <= b.hi[i] && b.lo[i] <= a.hi[i];
+			return o;
+		}
+
 		struct	TlasEmitter
 		{
 			const std::vector<AABBd>&	boxes;
 			const std::vector<GpuHittable>&	hittables;
 			std::vector<BvhNode>&	nodes;
 			std::vector<std::uint32_t>&	prims;
+			std::vector<std::uint8_t>	splits;	// per node (or fewer): kNotSplit, kSplitApart, kSplitChain
 
 			struct	Ref
 			{
@@ -555,23 +566,74 @@ namespace luzgpu
 				AABBd	box;
 			};
 
+			bool	isTriangle(std::uint32_t h) const { return (hittables[h].kindIndex >> kKindShift) == GPU_HIT_TRIANGLE; }
+
+			Ref	leaf(const std::vector<std::uint32_t>& items, const AABBd& box)
+			{
+				const std::int32_t start = static_cast<std::int32_t>(prims.size());
+				prims.insert(prims.end(), items.begin(), items.end());
+				return Ref{start, static_cast<std::int32_t>(items.size()), box};
+			}
+
+			Ref	join(const Ref& l, const Ref& r, const AABBd& box, std::uint8_t split)
+			{
+				const std::size_t idx = nodes.size();
+				nodes.push_back(BvhNode{});
+				setChild(nodes[idx], 0, &l.box, l.child, l.count);
+				setChild(nodes[idx], 1, &r.box, r.child, r.count);
+				splits.resize(nodes.size(), kNotSplit);
+				splits[idx] = split;
+				return Ref{static_cast<std::int32_t>(idx), 0, box};
+			}
+
+			// The reference's leaf tests its list in order, so of primitives at the same distance
+			// the last one is hit. A device leaf holds either triangles (a run of their own array)
+			// or other primitives. A list of both whose triangles meet none of the others' boxes has
+			// no such ties between the two: the triangles go apart from the rest. Otherwise its runs
+			// become leaves that all have the list's box: they are entered at the same distance, and
+			// nodes visit such children in order.
+			Ref	mixedLeaf(const std::vector<std::uint32_t>& items, const AABBd& box)
+			{
+				bool meet = false;
+				for (std::uint32_t a : items)
+				{
+					for (std::uint32_t b : items) meet = meet || (isTriangle(a) && !isTriangle(b) && overlap(boxes[a], boxes[b]));
+				}
+				if (meet) return chain(items, 0, box);
+				std::vector<std::uint32_t> part[2];
+				for (std::uint32_t h : items) part[isTriangle(h) ? 0 : 1].push_back(h);
+				Ref refs[2];
+				for (int k = 0; k < 2; k++)
+				{
+					AABBd own = boxes[part[k][0]];
+					for (std::uint32_t h : part[k]) own = merge(own, boxes[h]);
+					refs[k] = leaf(part[k], own);
+				}
+				return join(refs[0], refs[1], box, kSplitApart);
+			}
+
+			Ref	chain(const std::vector<std::uint32_t>& items, std::size_t from, const AABBd& box)
+			{
+				std::size_t to = from + 1;
+				while (to < items.size() && isTriangle(items[to]) == isTriangle(items[from])) to++;
+				const Ref l = leaf(std::vector<std::uint32_t>(items.begin() + static_cast<std::ptrdiff_t>(from),
+					items.begin() + static_cast<std::ptrdiff_t>(to)), box);
+				return to == items.size() ? l : join(l, chain(items, to, box), box, kSplitChain);
+			}
+
 			Ref	group(std::vector<std::uint32_t> items)
 			{
 				AABBd box = boxes[items[0]];
 				std::size_t instances = 0, triangles = 0;
-				auto isTriangle = [&](std::uint32_t h) { return (hittables[h].kindIndex >> kKindShift) == GPU_HIT_TRIANGLE; };
 				for (std::uint32_t h : items)
 				{
 					box = merge(box, boxes[h]);
 					instances += (hittables[h].kindIndex >> kKindShift) == GPU_HIT_INSTANCE ? 1u : 0u;
 					triangles += isTriangle(h) ? 1u : 0u;
 				}
-				const bool mixed = triangles != 0 && triangles != items.size();
-				if (items.size() == 1 || (instances == 0 && !mixed && items.size() <= kTopLeafMax))
+				if (items.size() == 1 || (instances == 0 && items.size() <= kTopLeafMax))
 				{
-					const std::int32_t start = static_cast<std::int32_t>(prims.size());
-					prims.insert(prims.end(), items.begin(), items.end());
-					return Ref{start, static_cast<std::int32_t>(items.size()), box};
+					return triangles == 0 || triangles == items.size() ? leaf(items, box) : mixedLeaf(items, box);
 				}
 				AABBd cb;
 				for (std::size_t i = 0; i < items.size(); i++)
@@ -581,21 +643,12 @@ namespace luzgpu
 					cb = i == 0 ? cc : merge(cb, cc);
 				}
 				const int axis = largestAxis(cb);
-				std::size_t mid = items.size() / 2;
-				if (instances == 0 && mixed && items.size() <= kTopLeafMax)
-				{
-					// a leaf's triangles are a run of their own array: the other primitives apart
-					std::stable_partition(items.begin(), items.end(), isTriangle);
-					mid = triangles;
-				}
-				else
-				{
-					std::nth_element(items.begin(), items.begin() + static_cast<std::ptrdiff_t>(mid), items.end(),
-						[&](std::uint32_t a, std::uint32_t b) {
-							const double ca = boxes[a].lo[axis] + boxes[a].hi[axis], cbv = boxes[b].lo[axis] + boxes[b].hi[axis];
-							return ca < cbv || (ca == cbv && a < b);
-						});
-				}
+				const std::size_t mid = items.size() / 2;
+				std::nth_element(items.begin(), items.begin() + static_cast<std::ptrdiff_t>(mid), items.end(),
+					[&](std::uint32_t a, std::uint32_t b) {
+						const double ca = boxes[a].lo[axis] + boxes[a].hi[axis], cbv = boxes[b].lo[axis] + boxes[b].hi[axis];
+						return ca < cbv || (ca == cbv && a < b);
+					});
 				const std::size_t idx = nodes.size();
 				nodes.push_back(BvhNode{});
 				const Ref l = group(std::vector<std::uint32_t>(items.begin(), items.begin() + static_cast<std::ptrdiff_t>(mid)));
@@ -696,11 +749,23 @@ namespace luzgpu
 			}
 		}
 
+		// Worst-case traversal stack entries below a node: a node defers every hit child but the
+		// nearest, so they are the largest sum of (children - 1) along a root-to-leaf path.
+		struct	StackBound
+		{
+			int	leaves = 0;	// were every split a leaf: what scenes are admitted by
+			int	splits = 0;	// of the tree as it is: at most one more
+		};
+
 		// Collapses the binary device tree below `node` into 4-wide nodes (largest-area
 		// internal child opened first). Returns the wide index of the new node.
 		template <typename Leaf>
-		std::int32_t	widen(const std::vector<BvhNode>& bin, std::int32_t node, std::vector<Bvh4Node>& out, const Leaf& leaf)
+		std::int32_t	widen(const std::vector<BvhNode>& bin, const std::vector<std::uint8_t>& splits, std::int32_t node,
+			std::vector<Bvh4Node>& out, const Leaf& leaf, StackBound& bound)
 		{
+			auto splitOf = [&](const WideSlot& w) -> int {
+				return w.count == 0 && static_cast<std::size_t>(w.child) < splits.size() ? splits[static_cast<std::size_t>(w.child)] : kNotSplit;
+			};
 			std::vector<WideSlot> slots;
 			auto addChildren = [&](std::int32_t b) {
 				const BvhNode& n = bin[static_cast<std::size_t>(b)];
@@ -723,7 +788,7 @@ namespace luzgpu
 				float bestArea = -1.0f;
 				for (std::size_t k = 0; k < slots.size(); k++)
 				{
-					if (slots[k].count == 0 && slotArea(slots[k]) > bestArea)
+					if (slots[k].count == 0 && splitOf(slots[k]) == kNotSplit && slotArea(slots[k]) > bestArea)
 					{
 						best = static_cast<int>(k);
 						bestArea = slotArea(slots[k]);
@@ -737,29 +802,37 @@ namespace luzgpu
 				slots.erase(slots.begin() + best);
 				addChildren(b);
 			}
+			const int children = static_cast<int>(slots.size());
+			// a lone split that only sets kinds apart: opening it defers one entry more, as below
+			const auto isSplit = [&](const WideSlot& w) { return splitOf(w) != kNotSplit; };
+			const auto lone = std::find_if(slots.begin(), slots.end(), isSplit);
+			if (slots.size() < 4 && lone != slots.end() && splitOf(*lone) == kSplitApart && std::count_if(slots.begin(), slots.end(), isSplit) == 1)
+			{
+				const std::int32_t b = lone->child;
+				slots.erase(lone);
+				addChildren(b);
+			}
 			const std::size_t idx = out.size();
 			out.push_back(Bvh4Node{});
+			StackBound below;
 			for (WideSlot& w : slots)
 			{
-				if (w.count == 0) w.child = widen(bin, w.child, out, leaf);
+				if (w.count != 0) continue;
+				StackBound b;
+				const bool split = isSplit(w);
+				w.child = widen(bin, splits, w.child, out, leaf, b);
+				below.leaves = std::max(below.leaves, split ? 0 : b.leaves);
+				below.splits = std::max(below.splits, b.splits);
+			}
+			bound.leaves = std::max(0, children - 1) + below.leaves;
+			bound.splits = std::max(0, static_cast<int>(slots.size()) - 1) + below.splits;
+			if (static_cast<std::size_t>(node) < splits.size() && splits[static_cast<std::size_t>(node)] != kNotSplit)
+			{
+				// a chain's first child is a leaf that is visited first: one entry at a time
+				bound = StackBound{0, 1};
 			}
 			encodeWide(out[idx], slots, leaf);
 			return static_cast<std::int32_t>(idx);
-		}
-
-		// Worst-case traversal stack entries below `root`: a node defers every hit child but
-		// the nearest, so the bound is the largest sum of (children - 1) along a root-to-leaf path.
-		int	wideStackBound(const std::vector<Bvh4Node>& nodes, std::int32_t root)
-		{
-			const Bvh4Node& n = nodes[static_cast<std::size_t>(root)];
-			int valid = 0, below = 0;
-			for (int k = 0; k < 4; k++)
-			{
-				if (n.child[k] == kEmptyChild) continue;
-				valid++;
-				if (!(n.child[k] & kLeafBit)) below = std::max(below, wideStackBound(nodes, static_cast<std::int32_t>(n.child[k])));
-			}
-			return std::max(0, valid - 1) + below;
 		}
 
 		int	wideDepth(const std::vector<Bvh4Node>& nodes, std::int32_t root)
@@ -1096,15 +1169,16 @@ namespace luzgpu
 				}
 			}
 			const std::int32_t binaryRoot = packBlas(blas, triBase, p.blasNodes);
-			meshRoot[m] = widen(p.blasNodes, binaryRoot, p.blasWide, [](std::int32_t start, std::int32_t count) {
+			StackBound bound;
+			meshRoot[m] = widen(p.blasNodes, {}, binaryRoot, p.blasWide, [](std::int32_t start, std::int32_t count) {
 				if (static_cast<std::uint32_t>(start) > kLeafStartMask || count > 16)
 				{
 					throw std::runtime_error("Unsupported for the device path: mesh triangle slots beyond 27 bits");
 				}
 				return kLeafBit | (static_cast<std::uint32_t>(count - 1) << kLeafCountShift) | static_cast<std::uint32_t>(start);
-			});
+			}, bound);
 			p.blasDeviceDepth = std::max(p.blasDeviceDepth, wideDepth(p.blasWide, meshRoot[m]));
-			p.blasStackBound = std::max(p.blasStackBound, wideStackBound(p.blasWide, meshRoot[m]));
+			p.blasStackBound = std::max(p.blasStackBound, bound.leaves);
 			p.triangleCount += mesh.triangles.size();
 		}
 
@@ -1293,7 +1367,7 @@ namespace luzgpu
 			// n-ary leaf (up to 16 hittables) is refined into a small binary tree so every
 			// mesh instance has its own box test before its mesh BVH is entered, and plain
 			// primitives sit in leaves of at most 4.
-			TlasEmitter em{boxes, p.hittables, p.tlasNodes, p.tlasPrims};
+			TlasEmitter em{boxes, p.hittables, p.tlasNodes, p.tlasPrims, {}};
 			const TlasEmitter::Ref root = em.fromReference(tb, 0);
 			if (root.count > 0)
 			{
@@ -1326,7 +1400,8 @@ namespace luzgpu
 			{
 				if ((h.kindIndex >> kKindShift) == GPU_HIT_TRIANGLE) h.kindIndex = (GPU_HIT_TRIANGLE << kKindShift) | slotOf[h.kindIndex & kIndexMask];
 			}
-			p.params.tlasRoot = widen(p.tlasNodes, p.params.tlasRoot, p.tlasWide, [&](std::int32_t start, std::int32_t count) {
+			StackBound bound;
+			p.params.tlasRoot = widen(p.tlasNodes, em.splits, p.params.tlasRoot, p.tlasWide, [&](std::int32_t start, std::int32_t count) {
 				const std::uint32_t kindIndex = p.hittables[p.tlasPrims[static_cast<std::size_t>(start)]].kindIndex;
 				const std::uint32_t kind = kindIndex >> kKindShift;
 				const std::uint32_t top = kind == GPU_HIT_TRIANGLE ? kTopTriangles : kind == GPU_HIT_INSTANCE ? kTopInstance : kTopItems;
@@ -1336,9 +1411,10 @@ namespace luzgpu
 					throw std::runtime_error("Unsupported for the device path: top-level primitives beyond 27 bits");
 				}
 				return kLeafBit | (top << kTopKindShift) | (static_cast<std::uint32_t>(count - 1) << kLeafCountShift) | first;
-			});
+			}, bound);
 			p.tlasDeviceDepth = wideDepth(p.tlasWide, p.params.tlasRoot);
-			p.tlasStackBound = wideStackBound(p.tlasWide, p.params.tlasRoot);
+			p.tlasStackBound = bound.leaves;
+			if (bound.splits > bound.leaves + 1) throw std::logic_error("top-level stack bound");
 		}
 		// one node array on the device: the mesh BVHs follow the top level
 		if (p.tlasWide.size() + p.blasWide.size() > kMaxNodes)

@@ -86,7 +86,7 @@ namespace luzgpu
 		std::size_t	triangleCount = 0;
 		int	tlasDeviceDepth = 0;	// device-layout (4-wide) node levels
 		int	blasDeviceDepth = 0;
-		int	tlasStackBound = 0;	// worst-case deferred traversal entries
+		int	tlasStackBound = 0;	// worst-case deferred traversal entries (a split leaf counted as one: kStackReserve)
 		int	blasStackBound = 0;
 		Camera	camera;
 		double	metersPerUnit = 1.0;

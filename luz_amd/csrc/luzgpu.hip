@@ -1195,7 +1195,7 @@ namespace
 			for (uint32_t i = 0; i < n; i++) parts[i] = &scenes[i]->gpu.host;
 			auto g = std::make_unique<GpuScene>();
 			g->host = mergeScenes(parts, ctx->batchParams);
-			if (g->host.tlasStackBound + 2 + g->host.blasStackBound > kWaveStackCapacity)
+			if (g->host.tlasStackBound + kStackReserve + g->host.blasStackBound > kWaveStackCapacity)
 			{
 				throw std::runtime_error("Unsupported for the device path: traversal stack bound of the batch");
 			}
@@ -1219,12 +1219,12 @@ namespace
 		sc->serial = ++serials;
 		sc->gpu.host = packScene(scene);
 		const PackedScene& h = sc->gpu.host;
-		// Worst-case stack use: deferred TLAS entries, a leaf-resume entry and the instance
-		// exit marker, then deferred mesh-BVH entries. Scenes that could exceed the smaller
-		// of the two kernels' stacks are refused rather than traversed incompletely.
+		// Worst-case stack use: deferred entries of the top level and of one mesh BVH, and the
+		// reserve. Scenes that could exceed the smaller of the two kernels' stacks are refused
+		// rather than traversed incompletely.
 		const int tlasDepth = h.tlasDeviceDepth;
 		const int blasDepth = h.blasDeviceDepth;
-		const int bound = h.tlasStackBound + 2 + h.blasStackBound;
+		const int bound = h.tlasStackBound + kStackReserve + h.blasStackBound;
 		if (bound > kStackDepth)
 		{
 			throw std::runtime_error("Unsupported for the device path: traversal stack bound " + std::to_string(bound)

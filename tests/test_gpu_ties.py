@@ -85,3 +85,26 @@ def test_equally_near_children_keep_their_order(ctx, workload_dir, last):
         ids, _ = Renderer.primary_hits(SceneFile.read(ctx, path), seed=3)
         # a pixel on a quad's edge may see past it in FP32
         assert (ids[..., 0] != want).sum() <= 2, planes
+
+
+@pytest.mark.parametrize("kinds", ["RT", "TR", "RTR", "TRT", "RRT", "TTR", "RTRT", "TRRT"])
+def test_the_last_of_a_leaf_of_triangles_and_rectangles_is_hit(ctx, workload_dir, kinds):
+    """T a triangle over half of the rectangle R, one on another in one leaf of the top level."""
+    from luz_amd import Renderer, SceneFile
+    directory = os.path.join(workload_dir, "ties")
+    text = {"T": "triangle=(-2,-2,0),(-2,2,0),(2,-2,0),material=a\n", "R": "rectangle=(0,0,0),(0,0,-1),4,4,material=a\n"}
+    shared = _oracle(_write(directory, "triangle", text["T"])) == 0
+    assert shared.sum() > 80
+    path = _write(directory, kinds, "".join(text[k] for k in kinds))
+    want = _oracle(path)
+    assert (want[shared] == len(kinds) - 1).all()
+    scene = SceneFile.read(ctx, path)
+    got = Renderer.primary_hits(scene, seed=3)[0][..., 0]
+    assert (got[~shared] == want[~shared]).all()
+    assert np.isin(got[shared], [kinds.rindex("T"), kinds.rindex("R")]).all()
+    # The FP32 distances of a triangle and a rectangle differ by an ulp in some pixels, either way,
+    # and only there may the earlier one be nearer: were ties given to it, it had most of them
+    assert (got[shared] == len(kinds) - 1).mean() > 0.5
+    one, _ = Renderer.render(scene, seed=3, samples=2, integrator="wavefront")
+    for image in Renderer.render_batch([scene, scene], [3, 3], samples=[2, 2])[0]:
+        assert np.array_equal(image, one)
