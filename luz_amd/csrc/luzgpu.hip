@@ -2093,6 +2093,16 @@ int	luzgpu_render_batch(luzgpu_ctx* ctx, uint32_t n, luzgpu_scene* const* scenes
 			resolve_batch<<<dim3(std::min(blocks(most, 256), 256u), plainScenes), 256, 0, st>>>(plain);
 			plainScenes = 0;
 		};
+		// scenes that share an output keep their order: the last one's image stays
+		auto resolveSharing = [&](const float* dst, size_t values) {
+			bool shared = false;
+			for (std::uint32_t k = 0; k < plainScenes; k++)
+			{
+				const ResolveBatch::Scene& other = plain.scenes[k];
+				shared = shared || (dst < other.out + other.values && other.out < dst + values);
+			}
+			if (shared) resolvePlain();
+		};
 		for (uint32_t i = 0; i < n; i++)
 		{
 			const std::uint32_t pixels = jobs[i].params.width * jobs[i].params.height;
@@ -2103,6 +2113,7 @@ int	luzgpu_render_batch(luzgpu_ctx* ctx, uint32_t n, luzgpu_scene* const* scenes
 				copies.emplace_back(rgb_out[i], staged);
 				staged += static_cast<size_t>(pixels) * 3 * sizeof(float);
 			}
+			resolveSharing(dst, static_cast<size_t>(pixels) * 3);
 			if (settings && settings[i].postprocess)
 			{
 				ctx->postMem.reserve(4 * static_cast<size_t>(pixels) * 3 * sizeof(double));
@@ -2115,16 +2126,9 @@ int	luzgpu_render_batch(luzgpu_ctx* ctx, uint32_t n, luzgpu_scene* const* scenes
 			else if (adaptive) resolve_used<<<blocks(pixels, 256), 256, 0, st>>>(jobs[i].sums, A.used + aj[i].offset, dst, pixels);
 			else
 			{
-				// scenes that share an output keep their order: the last one's image stays
-				const size_t values = static_cast<size_t>(pixels) * 3;
-				bool shared = plainScenes == ResolveBatch::kScenes;
-				for (std::uint32_t k = 0; k < plainScenes; k++)
-				{
-					const ResolveBatch::Scene& other = plain.scenes[k];
-					shared = shared || (dst < other.out + other.values && other.out < dst + values);
-				}
-				if (shared) resolvePlain();
-				plain.scenes[plainScenes++] = ResolveBatch::Scene{jobs[i].sums, dst, static_cast<double>(jobs[i].params.sampleCount), values};
+				if (plainScenes == ResolveBatch::kScenes) resolvePlain();
+				plain.scenes[plainScenes++] = ResolveBatch::Scene{jobs[i].sums, dst, static_cast<double>(jobs[i].params.sampleCount),
+					static_cast<size_t>(pixels) * 3};
 			}
 		}
 		resolvePlain();

@@ -35,3 +35,30 @@ def test_a_shared_output_holds_the_last_scene(ctx, cornell):
     torch.cuda.synchronize()
     one, _ = Renderer.render(scene, seed=5, samples=1, resolution=(65, 33), integrator="megakernel")
     assert np.array_equal(out.cpu().numpy(), one)
+
+
+@pytest.mark.parametrize("post", [[0, 1], [1, 0], [0, 0, 1], [0, 1, 0, 1, 0], [1, 1, 0, 0, 1]])
+@pytest.mark.parametrize("apart", [0, 21])
+def test_a_shared_output_of_plain_and_post_processed_scenes(ctx, cornell, post, apart):
+    """Through the C interface, where each scene has its own ``postprocess``; ``apart`` values lie
+    between the scenes' outputs, so that they overlap (the last one covers its whole range)."""
+    import ctypes
+    import torch
+    from luz_amd import Renderer, SceneFile, _lib, renderer
+    scene = SceneFile.read(ctx, cornell.scene_path)
+    n, values = len(post), 33 * 65 * 3
+    out = torch.empty(values + n * apart, device="cuda:0")
+    arr, ptrs = (_lib.Settings * n)(), (ctypes.c_void_p * n)()
+    for i in range(n):
+        arr[i] = renderer._settings(i + 1, 1, None, 0, None, "megakernel", on_device=True, resolution=(65, 33), postprocess=bool(post[i]))
+        ptrs[i] = out.data_ptr() + 4 * apart * i
+    torch.cuda.synchronize()
+    stats = _lib.Stats()
+    _lib.check(ctx._lib.luzgpu_render_batch(ctx.handle, n, (ctypes.c_void_p * n)(*[scene._h.value] * n), arr, ptrs, ctypes.byref(stats)))
+    torch.cuda.synchronize()
+    want = np.zeros(values + n * apart, dtype=np.float32)
+    for i in range(n):
+        one, _ = Renderer.render(scene, seed=i + 1, samples=1, resolution=(65, 33), integrator="megakernel", postprocess=bool(post[i]))
+        want[apart * i:apart * i + values] = one.ravel()
+    end = values + (n - 1) * apart
+    assert np.array_equal(out.cpu().numpy()[:end], want[:end])
