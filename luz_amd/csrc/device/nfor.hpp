@@ -19,6 +19,7 @@
 #pragma once
 
 #include "median.hpp"
+#include "nfor_weight.hpp"
 
 #include <hip/hip_runtime.h>
 
@@ -273,7 +274,8 @@ namespace luzgpu
 	// Dynamic LDS of nfor_accumulate, in doubles. Staged: the colours (three planes) and
 	// variances of the tile grown by the window and patch radii, and the 11 feature planes of
 	// the tile grown by the window radius, each slot holding the pixel of its clamped
-	// coordinate. Both forms: the patch terms and the weights of two steps each. Strides keep
+	// coordinate. Both forms: the patch terms, the weights and the weights' corrections (a byte
+	// each) of two steps each. Strides keep
 	// the doubles that lanes read together on disjoint banks: an operand reads four planes at
 	// once, up to 7 neighbours of each (planes 8 doubles apart modulo the LDS's 32), and half a
 	// wave reads the patch terms of two rows four apart (rows 4 doubles apart modulo 8).
@@ -281,7 +283,7 @@ namespace luzgpu
 	{
 		int	colorWidth, colorHeight, featureWidth, featureHeight, apronX, apronY, apronStride;
 		std::uint32_t	colorStride, featureStride;	// doubles between planes
-		std::uint32_t	colors, variances, features, pairs, weights, doubles;
+		std::uint32_t	colors, variances, features, pairs, weights, corrections, doubles;
 	};
 
 	__host__ __device__ inline NforLdsLayout	nforLdsLayout(std::uint32_t regressionRadius, std::uint32_t patchRadius, bool staged)
@@ -304,34 +306,9 @@ namespace luzgpu
 		L.features = L.variances + cc;
 		L.pairs = L.features + kNforFeatures * L.featureStride;
 		L.weights = L.pairs + 2 * kNforChunk * static_cast<std::uint32_t>(L.apronStride * L.apronY);
-		L.doubles = L.weights + 2 * kNforChunk * kNforWeightStride;
+		L.corrections = L.weights + 2 * kNforChunk * kNforWeightStride;
+		L.doubles = L.corrections + 2 * kNforChunk * kNforWeightStride / 8;
 		return L;
-	}
-
-	// exp(-x) for x >= 0 (NaN stays NaN): 2^k e^r with k the nearest integer to -x log2 e, r the
-	// rest (ln 2 in two parts), e^r its Taylor sum to r^13 (|r| <= ln 2 / 2: the first term left
-	// out is 4e-18 of it). Within 1 ulp.
-	__device__ __forceinline__ double	nforExpNegative(double x)
-	{
-		x = x > 1000.0 ? 1000.0 : x;	// 2^-1443: zero already
-		const double k = rint(x * -1.4426950408889634);
-		double r = fma(k, -0.69314718055994529, -x);
-		r = fma(k, -2.3190468138462996e-17, r);
-		// two half sums of the even and odd powers: two chains in flight
-		const double r2 = r * r;
-		double even = fma(r2, 2.0876756987868099e-09, 2.7557319223985893e-07);		// 1/12!, 1/10!
-		double odd = fma(r2, 1.6059043836821613e-10, 2.5052108385441720e-08);		// 1/13!, 1/11!
-		even = fma(r2, even, 2.4801587301587302e-05);
-		odd = fma(r2, odd, 2.7557319223985893e-06);
-		even = fma(r2, even, 1.3888888888888889e-03);
-		odd = fma(r2, odd, 1.9841269841269841e-04);
-		even = fma(r2, even, 4.1666666666666664e-02);
-		odd = fma(r2, odd, 8.3333333333333332e-03);
-		even = fma(r2, even, 0.5);
-		odd = fma(r2, odd, 1.6666666666666666e-01);
-		// 1 + (r + r^2 (even + r odd))
-		const double tail = fma(r2, fma(r, odd, even), r);
-		return ldexp(1.0 + tail, static_cast<int>(k));
 	}
 
 	// regressionPass (NFOR.cpp:679-737), accumulation: each pixel's 12 x 12 weighted normal
@@ -352,17 +329,19 @@ namespace luzgpu
 	// evaluated once for every pixel of the tile and its apron into LDS. The stages of a step
 	// of 8 displacements (terms, then weights, then products) run on three consecutive steps
 	// at once, with one barrier a step; the two waves of a SIMD take them in opposite order.
-	// Lanes whose sample would lie off the image take the border sample's own terms. `Two`: bandwidth 1 and half of it; the second weight is the first's fourth
-	// power (the host takes two passes where the variance floor breaks that ratio).
+	// Lanes whose sample would lie off the image take the border sample's own terms. `Two`:
+	// bandwidth 1 and half of it; the second weight is the first's fourth power, from the first
+	// and a correction that keeps it within 0.6 ulp (a byte beside the weight: eight more would
+	// not fit; the host takes two passes where the variance floor breaks that ratio).
 	//
 	// Staged: the block first copies every colour, variance and feature its window reads into
-	// LDS (radius 9, patch radius 1: 152 KiB); the unstaged form reads them from global
+	// LDS (radius 9, patch radius 1: 153 KiB); the unstaged form reads them from global
 	// memory, for windows too wide for LDS.
 	//
 	// Bound by FP64 issue, which matrix and vector instructions share: at 1280 x 720, radius 9,
-	// 5.5 ms for one bandwidth and 7.7 for two, of which the products take 2.4 and 3.8 (1.2 and
-	// 2.4 at the matrix unit's rate), the weights 1.6, the terms 1.5, staging and stores 0.6 and
-	// 0.9. With each lane owning half a pixel's system in vector FMAs, 14 LDS reads a sample and
+	// 5.9 ms for one bandwidth and 8.6 for two, of which the products take 2.4 and 3.8 (1.2 and
+	// 2.4 at the matrix unit's rate), the weights 2.0, their corrections 0.5, the terms 1.5,
+	// staging and stores 0.6 and 0.9 (each stage's time on its own; they overlap in part). With each lane owning half a pixel's system in vector FMAs, 14 LDS reads a sample and
 	// three barriers per 4 displacements, one bandwidth took 8.8 ms. Border lanes that read
 	// their patches from global memory cost 1.8 ms of the weights; 16 waves of half the pixels
 	// each were slower (spills).
@@ -380,6 +359,7 @@ namespace luzgpu
 		double* const feats = lds + L.features;
 		double* const pairs = lds + L.pairs;
 		double* const weights = lds + L.weights;
+		std::int8_t* const corrections = reinterpret_cast<std::int8_t*>(lds + L.corrections);
 		const int cw = L.colorWidth, fw = L.featureWidth, ax = L.apronX, as = L.apronStride;
 		const int cells = cw * L.colorHeight, ff = fw * L.featureHeight, aa = ax * L.apronY, termsSize = as * L.apronY;
 		const int cc = static_cast<int>(L.colorStride), fs = static_cast<int>(L.featureStride);
@@ -533,12 +513,16 @@ namespace luzgpu
 			const double q = distance * inverseScale;
 			return nforExpNegative(fma(fma(-q, scale, distance), inverseScale, q));
 		};
+		auto storeWeight = [&](int at, const NforExp& e, bool sample) {
+			weights[at] = sample ? nforWeight1(e) : 0.0;
+			if (Two) corrections[at] = sample ? nforWeight4Correction(e) : std::int8_t(0);
+		};
 		auto formWeights = [&](int t, const Walk& at0, const Walk& at1) {
 			const double d0 = patchSum(t, kk, at0), d1 = patchSum(t, kk + kNforDepth, at1);
-			const double e0 = weightOf(d0), e1 = weightOf(d1);
-			double* out = weights + ((t & 1) * kNforChunk + kk) * kNforWeightStride + wPixel;
-			out[0] = wActive && at0.s < samples ? e0 : 0.0;
-			out[kNforDepth * kNforWeightStride] = wActive && at1.s < samples ? e1 : 0.0;
+			const NforExp e0 = weightOf(d0), e1 = weightOf(d1);
+			const int at = ((t & 1) * kNforChunk + kk) * kNforWeightStride + wPixel;
+			storeWeight(at, e0, wActive && at0.s < samples);
+			storeWeight(at + kNforDepth * kNforWeightStride, e1, wActive && at1.s < samples);
 		};
 
 		// products of step t
@@ -586,7 +570,7 @@ namespace luzgpu
 			const double* f0 = feats + plane0 * fs + fBase + fOff;
 			const double* f1 = feats + plane1 * fs + fBase + fOff;
 			const double* col = colors + colorPlane * cc + cBase + cOff;
-			const double* w = weights + ((t & 1) * kNforChunk + g * kNforDepth + lk) * kNforWeightStride + wave * kNforTileX + lb;
+			const int wAt = ((t & 1) * kNforChunk + g * kNforDepth + lk) * kNforWeightStride + wave * kNforTileX + lb;
 			#pragma unroll
 			for (int q = 0; q < kNforQuads; q++)
 			{
@@ -609,15 +593,12 @@ namespace luzgpu
 				}
 				const double d0 = v0 - own[q][0], b1 = v1 - own[q][1], b2 = v2 - own[q][2];
 				const double b0 = li == 0 ? 1.0 : d0;
-				double wk = w[4 * q];
+				double wk = weights[wAt + 4 * q];
+				const double w4 = Two ? nforWeight4(wk, corrections[wAt + 4 * q]) : 0.0;
 				#pragma unroll
 				for (int k = 0; k < Bandwidths; k++)
 				{
-					if (k == 1)
-					{
-						wk = wk * wk;
-						wk = wk * wk;
-					}
+					if (k == 1) wk = w4;
 					const double a0 = wk * b0, a1 = wk * b1, a2 = wk * b2;
 					double (&d)[9] = acc[k][q];
 					d[0] = __builtin_amdgcn_mfma_f64_4x4x4f64(a0, b0, d[0], 0, 0, 0);

@@ -869,7 +869,7 @@ namespace luzgpu
 			check(hipGetDevice(&device), "hipGetDevice");
 			check(hipDeviceGetAttribute(&ldsLimit, hipDeviceAttributeMaxSharedMemoryPerBlock, device), "LDS per block");
 			// the LDS-staged accumulation when its window fits the device's LDS per block
-			// (radius 9, patch radius 1: 152 KiB of the MI355X's 160 KiB), else the unstaged form
+			// (radius 9, patch radius 1: 153 KiB of the MI355X's 160 KiB), else the unstaged form
 			const size_t stagedBytes = nforLdsLayout(P.regressionRadius, P.patchRadius, true).doubles * sizeof(double);
 			const size_t plainBytes = nforLdsLayout(P.regressionRadius, P.patchRadius, false).doubles * sizeof(double);
 			// one regression at bandwidth k into dst0, or (Two) one at 1 into dst0 and one at 1/2
