@@ -29,6 +29,15 @@ namespace luzgpu
 		return (a[0] * b[0] + a[1] * b[1]) + a[2] * b[2];
 	}
 
+	// A value that stays in vector registers. The plain kernels hold more scalars than there are
+	// scalar registers, and what the march reads was fetched from spill lanes in its inner loop:
+	// 34 of its 178 instructions (atmosphere scene at 640x480, 16 samples: 5.49 -> 4.74 ms).
+	__device__ __forceinline__ double	inVector(double v)
+	{
+		asm volatile("" : "+v"(v));
+		return v;
+	}
+
 	// planetaryHit (Atmosphere.cpp:311-343): both roots of a sphere of `radius` at the origin
 	__device__ __forceinline__ bool	planetaryHit(double radius, const double* o, const double* d, double& t0, double& t1)
 	{
@@ -106,20 +115,22 @@ namespace luzgpu
 		const double phaseM = mieScale * ((1.0 - g * g) * (1.0 + mu2) / ((2.0 + g * g) * (base * sqrt(base))));
 		const double betaMA = betaM * mieAbsorption;
 
+		const double earthRadius = inVector(A.earthRadius), inverseHR = inVector(A.inverseHR), inverseHM = inVector(A.inverseHM);
+		const double sun[3] = {inVector(A.sunDirection[0]), inVector(A.sunDirection[1]), inVector(A.sunDirection[2])};
 		double sumR[3] = {0.0, 0.0, 0.0}, sumM[3] = {0.0, 0.0, 0.0};
 		double depthR = 0.0, depthM = 0.0;
 		for (std::uint32_t i = 0; i < A.samples; i++)
 		{
 			const double t = tLo + (static_cast<double>(i) + 0.5) * seg;
 			const double pos[3] = {o[0] + t * d[0], o[1] + t * d[1], o[2] + t * d[2]};
-			const double h = sqrt(atmDot(pos, pos)) - A.earthRadius;
-			const double dR = atmDensity(h, A.inverseHR), dM = atmDensity(h, A.inverseHM);
+			const double h = sqrt(atmDot(pos, pos)) - earthRadius;
+			const double dR = atmDensity(h, inverseHR), dM = atmDensity(h, inverseHM);
 			if (dR == 0.0 && dM == 0.0) continue;
 			const double sR = dR * seg, sM = dM * seg;
 			depthR += sR;
 			depthM += sM;
 			double l0, l1;
-			if (!planetaryHit(A.atmosphereRadius, pos, A.sunDirection, l0, l1) || l1 <= 0.0) continue;
+			if (!planetaryHit(A.atmosphereRadius, pos, sun, l0, l1) || l1 <= 0.0) continue;
 			const double segL = l1 / static_cast<double>(A.lightSamples);
 			if (!isfinite(segL) || segL <= 0.0) continue;
 			double lightR = 0.0, lightM = 0.0;
@@ -127,15 +138,15 @@ namespace luzgpu
 			for (std::uint32_t j = 0; j < A.lightSamples; j++)
 			{
 				const double lt = (static_cast<double>(j) + 0.5) * segL;
-				const double q[3] = {pos[0] + lt * A.sunDirection[0], pos[1] + lt * A.sunDirection[1], pos[2] + lt * A.sunDirection[2]};
-				const double hl = sqrt(atmDot(q, q)) - A.earthRadius;
+				const double q[3] = {pos[0] + lt * sun[0], pos[1] + lt * sun[1], pos[2] + lt * sun[2]};
+				const double hl = sqrt(atmDot(q, q)) - earthRadius;
 				if (hl < 0.0)
 				{
 					reaches = false;
 					break;
 				}
-				lightR += atmDensity(hl, A.inverseHR) * segL;
-				lightM += atmDensity(hl, A.inverseHM) * segL;
+				lightR += atmDensity(hl, inverseHR) * segL;
+				lightM += atmDensity(hl, inverseHM) * segL;
 			}
 			if (reaches)
 			{
