@@ -341,9 +341,13 @@ namespace luzgpu
 	// reciprocal is the hardware's (1 ulp); an axis the ray is parallel to takes a huge one, so
 	// its planes lie far behind or ahead, as AABB::hit's test of the origin against the slab
 	// has it (AABB.cpp:37-80). `nearC` / `farC` are -o * inv moved outward by 2^-21 of
-	// itself, which covers the rounding of that product and of the sums, and the far distance
-	// is compared with a relative margin of 2^-19: box tests are conservative (they only decide
-	// which primitives are tested), the primitive tests alone decide the hit.
+	// itself, which covers the rounding of that product, and the far distance is compared with a
+	// relative margin of 2^-19 for the reciprocals' and the last sums'. The sum with
+	// origin * inv rounds by up to 2^-24 of the distance to the node's origin, which neither
+	// covers where that is large against |o| and the plane is near: there a box can be missed by
+	// rays that pass within 2^-24 of that distance of its border (scene units; 6e-5 at 1000),
+	// as vertices that far away are rounded in FP32. Box tests only decide which primitives are
+	// tested; the primitive tests alone decide the hit.
 	struct	TraceState
 	{
 		f3	world_o, world_d;	// world-space ray, restored when an instance is left
