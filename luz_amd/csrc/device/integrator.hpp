@@ -359,7 +359,7 @@ namespace luzgpu
 	// Inlined into every kernel: as a function of its own (the compiler's choice for three
 	// callers) it took the scene and the parameters by address, copied to scratch and read back
 	// through generic loads with 254 VGPRs (163 inlined, no scratch). The 48 waves of a 64x48
-	// preview take one path's latency: the call 0.46 -> 0.39 ms; 32 thumbnails in one launch, the
+	// preview take one path's latency: the call 0.46 -> 0.40 ms; 32 thumbnails in one launch, the
 	// call 0.53 -> 0.44 ms.
 	template <bool Count, int Feat, typename Stack, typename Adj = NoAdjoint>
 	__device__ __forceinline__ f3	tracePath(const SceneView& s, const GpuParams& p, std::uint32_t x, std::uint32_t y, std::uint32_t sample,

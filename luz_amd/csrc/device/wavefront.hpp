@@ -223,13 +223,14 @@ namespace luzgpu
 	constexpr int	kWaveStackCapacity = 64;
 	constexpr unsigned	kWaveGrid = 2048;	// 256 CUs x 8 waves per SIMD x 4 SIMDs / 4 waves per block
 	// default traversal launch shape: as many persistent waves as the traversal kernels'
-	// registers let every SIMD hold (256 CUs x 4 SIMDs x 5 waves / 4 waves per block; 2 %
-	// faster than 1024 blocks on the sphere frame)
+	// registers let every SIMD hold (256 CUs x 4 SIMDs x 5 waves / 4 waves per block). 1080p
+	// spheres: 32.0 ms a frame, against 34.3 with 1024 blocks and 32.2 with 1536 and 2048; 720p
+	// hazy terrain 71.5 to 72.7 with any of them.
 	constexpr unsigned	kDefaultGrid = 1280;
 	// Idle lanes at which a wave takes new rays when the caller names no number: 48 in
-	// triangle-only scenes (1080p spheres: extend + shadow 22.4 ms, against 24.5 at 64 and
-	// 24.1 at 16), 16 in scenes with analytic primitives or volumes, whose rays differ more in
-	// length (720p hazy terrain: 52.3 ms, against 62.2 at 48 and 84.0 at 64).
+	// triangle-only scenes (1080p spheres: 32.0 ms a frame, against 34.3 at 64, 33.0 at 32 and
+	// 33.9 at 16), 16 in scenes with analytic primitives or volumes, whose rays differ more in
+	// length (720p hazy terrain: 71.8 ms, against 72.8 at 8, 76.4 at 32, 83.8 at 48 and 106 at 64).
 	constexpr int	kRefillTriangles = 48;
 	constexpr int	kRefillAnalytic = 16;
 	// Lanes whose next entry is a leaf (primitive tests, an instance entry) wait while other
@@ -237,9 +238,9 @@ namespace luzgpu
 	// lane has a node left; then every live lane takes one step. Each lane's entries are
 	// processed in the same order as without the wait, so results do not depend on it; it
 	// only lets the wave run the node code and the leaf code less often side by side. The
-	// triangle-only kernels wait for 16 lanes (the sphere frame is slower at 8, 12, 24 and 32);
-	// the others for 32 on closest-hit rays and 48 on shadow rays (the hazy terrain: 102.8 ms,
-	// against 103.7 at 32 / 32, 104.5 at 24 / 24 and 107.6 at 16 / 16).
+	// triangle-only kernels wait for 16 lanes (1080p spheres: 31.9 ms a frame, against 32.8 at 8,
+	// 32.4 at 24 and 32.8 at 32); the others for 32 on closest-hit rays and 48 on shadow rays (720p
+	// hazy terrain: 72.3 ms, against 72.6 at 32 / 32, 73.5 at 24 / 24 and 75.6 at 16 / 16).
 	template <int Feat, bool AnyHit>
 	constexpr int	kLeafBatch = Feat == 0 ? 16 : (AnyHit ? 48 : 32);
 
@@ -597,9 +598,10 @@ namespace luzgpu
 
 	// closest hit of every ray of queue b
 	template <bool Count, int Feat, int LdsDepth>
-	// The traversal kernels are asked for at least 4 waves per SIMD (at most 128 VGPRs): the
-	// analytic-primitive specialisation otherwise takes 136 and runs 3 (terrain extend 41.4 ->
-	// 36.8 ms); the triangle-only one needs 88 and is unaffected.
+	// The traversal kernels are asked for at least 4 waves per SIMD (at most 128 VGPRs), which they
+	// keep to by themselves (86 and 82 VGPRs in triangle-only scenes, 109 and 103 with analytic
+	// primitives): the request holds them to it. At 3 waves the terrain's extend took 41.4 ms
+	// instead of 36.8, on a longer node test.
 	static __global__ __launch_bounds__(kWaveBlock, 4) void	wf_extend(SceneView s, const PassJob* jobs, WaveBuffers w, int b,
 		unsigned long long* counters, int refillAt, std::uint32_t chunk)
 	{

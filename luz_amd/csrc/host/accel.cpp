@@ -1697,7 +1697,11 @@ namespace luzgpu
 			}
 			if (h.kind == HIT_INSTANCE && scene.materials[h.material].kind == MAT_EMISSIVE)
 			{
-				p.features |= kFeatAll;	// a light pdf that traverses its mesh lives in the rich kernels
+				// a light pdf that traverses its mesh lives in the rich kernels: in the analytic ones it
+				// would cost every analytic scene on the wavefront 2 % (640 x 480, 16 samples:
+				// primitives 2.82 -> 2.87 ms, volume 4.76 -> 4.88), and give scenes with mesh lights 2 %
+				// there and 7 % at 1280 x 720 (13.8 -> 12.9 ms)
+				p.features |= kFeatAll;
 			}
 		}
 		for (const Material& m : scene.materials)

@@ -938,9 +938,11 @@ namespace luzgpu
 
 		// The integrator a call runs: LUZGPU_INTEGRATOR_AUTO picks the plain kernel for at most
 		// 4M paths, as the interface says. A batch of 32 small scenes of 2.1M paths takes 1.2 ms
-		// plain and 2.0 ms on the wavefront; single scenes cross between 0.8M and 2M paths (box of
-		// 34 triangles: 1.28 / 1.27 ms and 2.8 / 2.2 ms; 512 instanced spheres: 1.05 / 1.84 and
-		// 2.24 / 2.29 ms).
+		// plain and 2.0 ms on the wavefront. Single scenes cross earlier, and between there and 4M
+		// the wavefront would be faster (plain / wavefront): a box of 34 triangles at 0.8M paths
+		// (1.53 / 1.49 ms; at 2M 3.09 / 2.63, at 3.9M 5.8 / 4.1), hazy terrain between 0.8M and 2M
+		// (6.4 / 9.0 and 14.5 / 12.2), 512 instanced spheres at 2M (2.51 / 2.56; at 3.9M 4.6 / 3.4),
+		// glossy materials at 3.9M (2.41 / 2.35).
 		std::uint32_t	resolveIntegrator(std::uint32_t requested, std::uint64_t paths, const char* who)
 		{
 			if (requested == LUZGPU_INTEGRATOR_AUTO)
